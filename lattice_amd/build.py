@@ -43,6 +43,7 @@ HOST_SOURCES = ["pool_core.cpp", "tiering.cpp", "ffi.cpp", "tunables.cpp"]
 HIP_SOURCES = ["kernels/backing.hip", "kernels/attn_decode.hip", "kernels/attn_prefill.hip",
                "kernels/kv_write.hip",
                "kernels/page_copy.hip", "kernels/gemm.hip", "kernels/gemm_tiled.hip",
+               "kernels/gemm_wide.hip",
                "kernels/glue.hip",
                "kernels/tier_copy.hip"]
 

@@ -148,15 +148,38 @@ void host_pinned_free(void* p);
 bool gemm_bf16(uint64_t x, uint64_t w, uint64_t y, uint32_t m, uint32_t n, uint32_t k,
                uint64_t stream, std::string* err, uint64_t residual = 0);
 
-// The same product for many tokens (m > 128) on the LDS-tiled MFMA kernel
-// (kernels/gemm_tiled.hip); n % 64 == 0, k % 64 == 0.
-bool gemm_bf16_tiled(uint64_t x, uint64_t w, uint64_t y, uint32_t m, uint32_t n, uint32_t k,
-                     uint64_t stream, uint64_t residual, std::string* err);
-void gemm_tiled_plan(uint32_t m, uint32_t n, uint32_t k, int* splits, int* tile);
-// The tiled kernel for either weight type: bf16 W (wscale == 0) or fp8-e4m3
-// W [n][k] with an fp32 scale per row (as gemm_fp8w_bf16).
+// The same product for many tokens (m > 128): the LDS-tiled MFMA kernel
+// (kernels/gemm_tiled.hip) for either weight type -- bf16 W (wscale == 0) or
+// fp8-e4m3 W [n][k] with an fp32 scale per row (as gemm_fp8w_bf16) -- or the
+// wide kernel, whichever the plan has; n % 64 == 0, k % 64 == 0.  With part
+// set, a split product is left as its fp32 partials (*part, *splits) for the
+// caller to finish; otherwise *splits is 1 and y is written.
 bool gemm_tiled(uint64_t x, uint64_t w, uint64_t wscale, uint64_t y, uint32_t m, uint32_t n,
-                uint32_t k, uint64_t stream, uint64_t residual, std::string* err);
+                uint32_t k, uint64_t stream, uint64_t residual, std::string* err,
+                float** part = nullptr, int* splits = nullptr);
+// Its K splits and tiling (0..10 of the tiled kernel; 100 + token tile
+// height / 64 on the wide kernel).
+void gemm_tiled_plan(uint32_t m, uint32_t n, uint32_t k, bool fp8_weights, int* splits, int* tile);
+
+// The product for prompt-sized m on 256-row tiles of 8 waves
+// (kernels/gemm_wide.hip), bf16 weights.  swiglu: w = [gate; up] with n rows
+// each, y = act [m][n].
+struct GemmWidePlan {
+    int fb0 = 4, fb1 = 4;   // token tiles of 64 * fb0; the last nw1 weight tiles' of 64 * fb1
+    int nw1 = 0;
+    int splits = 1;         // K splits (fp32 partials [splits][m][n] when > 1)
+    double us = 0.0;        // modelled time (with the split sum)
+};
+struct GemmWideArgs {
+    uint64_t x, w, y, residual;
+    uint32_t m, n, k;
+    float* part;            // plan.splits > 1: where the partials go
+    bool swiglu;
+    GemmWidePlan plan;
+    uint64_t stream;
+};
+GemmWidePlan gemm_wide_plan(uint32_t m, uint32_t n, uint32_t k, bool swiglu);
+bool gemm_wide(const GemmWideArgs& a, std::string* err);
 
 // How a plain product of this shape runs (under the current KCMM_GEMM_*
 // settings): kernel 0 = weight-stream, 1 = LDS-tiled; K splits; tiling (tiled
@@ -220,6 +243,13 @@ bool residual_rmsnorm_from_partials(const float* part, int splits, uint64_t hidd
 bool gemm_bf16_partials(uint64_t x, uint64_t w, uint32_t m, uint32_t n, uint32_t k,
                         uint64_t stream, float** part, int* splits, std::string* err,
                         uint64_t wscale = 0);
+
+// hidden = bf16(hidden + bf16(X W^T)) in place, y = rmsnorm(hidden): the bits
+// of gemm_bf16 with the residual followed by rmsnorm_bf16, the split partials
+// (if the plan has any) summed in the RMSNorm kernel.
+bool gemm_bf16_add_rmsnorm(uint64_t x, uint64_t w, uint64_t hidden, uint64_t norm_w, uint64_t y,
+                           uint32_t m, uint32_t n, uint32_t k, float eps, uint64_t stream,
+                           std::string* err);
 
 // Fused projections (kernels/gemm.hip): the QKV GEMM whose store does what
 // rope_append_bf16 does with its result (a.qkv unused; one token per

@@ -1164,11 +1164,8 @@ int kcmm_gemm_bf16_add_rmsnorm_on_stream(uint64_t x, uint64_t w, uint64_t hidden
         k == 0 || n % 8 != 0 || !(eps >= 0.0f))
         return -1;
     std::string err;
-    float* part = nullptr;
-    int splits = 1;
-    if (!kcmm::dev::gemm_bf16_partials(x, w, m, n, k, stream, &part, &splits, &err) ||
-        !kcmm::dev::residual_rmsnorm_from_partials(part, splits, hidden, norm_w, normed, m, n, eps,
-                                                   stream, &err)) {
+    if (!kcmm::dev::gemm_bf16_add_rmsnorm(x, w, hidden, norm_w, normed, m, n, k, eps, stream,
+                                          &err)) {
         std::fprintf(stderr, "kcmm_gemm_bf16_add_rmsnorm_on_stream: %s\n", err.c_str());
         return -1;
     }
@@ -1457,6 +1454,11 @@ int run_decode_layers(kcmm_pool_t* pool, const char* fn, uint32_t first, uint32_
         // O projection as partials; the residual add is finished by the
         // RMSNorm kernel that reads them
         auto o_step = [&]() {
+            if (!kFp8)
+                return kcmm::dev::gemm_bf16_add_rmsnorm(attn, l.o, hidden, l.mlp_norm, normed, B,
+                                                        hidden_size,
+                                                        static_cast<uint32_t>(attn_k), rms_eps,
+                                                        stream, &err);
             float* part = nullptr;
             int splits = 1;
             return kcmm::dev::gemm_bf16_partials(attn, l.o, B, hidden_size,

@@ -29,6 +29,7 @@
 //    exactly to bf16 in registers; the fp32 row scale multiplies the
 //    accumulator before the store.
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <string>
 #include <type_traits>
@@ -364,23 +365,95 @@ TiledConfig choose(int M, int N, int K) {
     return best;
 }
 
+// Modelled time in us of a plan of this kernel: launch + rounds of workgroups
+// x (chunks x time per 64-element chunk + fixed part), + the split sum's launch
+// and the partials at 3.3 TB/s.  Fitted to timings of 180 products (M 129 ..
+// 2048, N 1024 .. 28672, K 1024 .. 14336): within 4% at the median, 10% for
+// nine in ten.
+double tiled_us(const TiledConfig& c, double M, double N, double K) {
+    const int cls = c.id == 0 ? 0 : c.id == 9 ? 1 : 2;
+    constexpr double kChunk[3] = {0.827, 0.504, 0.554}, kFixed[3] = {7.1, 6.5, 2.7};
+    const double slots = cls == 2 ? 512.0 : 256.0;
+    const double wgs = std::floor(N / c.bn) * std::ceil(M / c.bm) * c.splits;
+    const double rounds = std::ceil(wgs / slots);
+    // two workgroups share a CU at full occupancy only (configuration 10)
+    const double share = cls == 2 ? 0.5 + 0.5 * wgs / (rounds * slots) : 1.0;
+    double us = 0.7 + rounds * (K / 64.0 / c.splits * kChunk[cls] * share + kFixed[cls]);
+    if (c.splits > 1) us += 2.3 + 0.3e-6 * 4.0 * c.splits * M * N;
+    return us;
+}
+
+// Whether the wide kernel takes the product: when its modelled time is at
+// least 8% below this kernel's (both models are off by 4-8%, so closer ones
+// stay here: over the same 180 products every choice but three is within 2%
+// of the faster kernel).  A forced tile (KCMM_GEMM_TILE 0..10) stays here.
+bool use_wide(const TiledConfig& c, uint32_t m, uint32_t n, uint32_t k, dev::GemmWidePlan* plan) {
+    const int forced = dev::tunable_or(dev::Tun::kGemmTile, -1);
+    if (forced >= 0 && forced < kCfgs) return false;
+    *plan = dev::gemm_wide_plan(m, n, k, false);
+    if (plan->splits == 0) return false;
+    if (forced > 100) return true;
+    // (tiles of configurations other than 0, 9, 10 are N % 128 != 0 shapes)
+    return plan->us < 0.92 * tiled_us(c, m, n, k);
+}
+
 }  // namespace
 
 namespace dev {
 
-void gemm_tiled_plan(uint32_t m, uint32_t n, uint32_t k, int* splits, int* tile) {
+void gemm_tiled_plan(uint32_t m, uint32_t n, uint32_t k, bool fp8_weights, int* splits, int* tile) {
     const TiledConfig c = choose(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k));
-    *splits = c.splits;
-    *tile = c.id;
+    GemmWidePlan wp;
+    const bool wide = !fp8_weights && use_wide(c, m, n, k, &wp);
+    *splits = wide ? wp.splits : c.splits;
+    *tile = wide ? 100 + wp.fb0 : c.id;
 }
 
 bool gemm_tiled(uint64_t x, uint64_t w, uint64_t wscale, uint64_t y, uint32_t m, uint32_t n,
-                uint32_t k, uint64_t stream, uint64_t residual, std::string* err) {
+                uint32_t k, uint64_t stream, uint64_t residual, std::string* err, float** part,
+                int* splits) {
     if (m == 0 || n % 64 != 0 || k % 64 != 0) {
         *err = "tiled gemm needs m > 0, n % 64 == 0 and k % 64 == 0";
         return false;
     }
     const TiledConfig c = choose(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k));
+    if (splits != nullptr) *splits = 1;
+    GemmWidePlan wp;
+    const bool wide = wscale == 0 && use_wide(c, m, n, k, &wp);
+    const int ksplits = wide ? wp.splits : c.splits;
+    float* partials = nullptr;
+    if (ksplits > 1) {
+        void* ws = nullptr;
+        if (!stream_workspace(stream, 1, static_cast<size_t>(ksplits) * m * n * sizeof(float), &ws,
+                              false, err))
+            return false;
+        partials = static_cast<float*>(ws);
+    }
+    auto finish = [&]() {
+        if (ksplits == 1) return true;
+        if (part != nullptr) {
+            *part = partials;
+            *splits = ksplits;
+            return true;
+        }
+        return gemm_split_reduce_launch(partials, reinterpret_cast<uint16_t*>(y),
+                                        reinterpret_cast<const uint16_t*>(residual),
+                                        static_cast<int>(m * n), ksplits, stream, err);
+    };
+    if (wide) {
+        GemmWideArgs a{};
+        a.x = x;
+        a.w = w;
+        a.y = y;
+        a.residual = residual;
+        a.m = m;
+        a.n = n;
+        a.k = k;
+        a.part = partials;
+        a.plan = wp;
+        a.stream = stream;
+        return gemm_wide(a, err) && finish();
+    }
     TiledParams p{};
     p.X = reinterpret_cast<const uint8_t*>(x);
     p.W = reinterpret_cast<const uint8_t*>(w);
@@ -395,13 +468,7 @@ bool gemm_tiled(uint64_t x, uint64_t w, uint64_t wscale, uint64_t y, uint32_t m,
     const int tiles = (p.N / c.bn) * p.tiles_m;
     p.xcd_order = tiles % 8 == 0;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (c.splits > 1) {
-        void* ws = nullptr;
-        if (!stream_workspace(stream, 1, static_cast<size_t>(c.splits) * p.M * p.N * sizeof(float),
-                              &ws, false, err))
-            return false;
-        p.part = static_cast<float*>(ws);
-    }
+    p.part = partials;
     by_config(c.id, [&](auto bn, auto bm, auto wn, auto wm, auto ns, auto nt) {
         constexpr int BN = decltype(bn)::value, BM = decltype(bm)::value;
         constexpr int WN = decltype(wn)::value, WM = decltype(wm)::value, NS = decltype(ns)::value;
@@ -414,14 +481,7 @@ bool gemm_tiled(uint64_t x, uint64_t w, uint64_t wscale, uint64_t y, uint32_t m,
                                dim3(64 * WN * WM), 0, s, p);
     });
     KCMM_HIP_CHECK(hipGetLastError(), err);
-    if (c.splits > 1)
-        return gemm_split_reduce_launch(p.part, p.Y, p.R, p.M * p.N, c.splits, stream, err);
-    return true;
-}
-
-bool gemm_bf16_tiled(uint64_t x, uint64_t w, uint64_t y, uint32_t m, uint32_t n, uint32_t k,
-                     uint64_t stream, uint64_t residual, std::string* err) {
-    return gemm_tiled(x, w, 0, y, m, n, k, stream, residual, err);
+    return finish();
 }
 
 }  // namespace dev

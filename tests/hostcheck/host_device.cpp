@@ -242,8 +242,8 @@ bool gemm_bf16_swiglu(uint64_t, uint64_t, uint64_t, uint32_t, uint32_t, uint32_t
                       std::string* err, uint64_t) {
     return no_device(err);
 }
-bool gemm_bf16_tiled(uint64_t, uint64_t, uint64_t, uint32_t, uint32_t, uint32_t, uint64_t, uint64_t,
-                     std::string* err) {
+bool gemm_bf16_add_rmsnorm(uint64_t, uint64_t, uint64_t, uint64_t, uint64_t, uint32_t, uint32_t,
+                           uint32_t, float, uint64_t, std::string* err) {
     return no_device(err);
 }
 bool gemm_fp8w_bf16(uint64_t, uint64_t, uint64_t, uint64_t, uint32_t, uint32_t, uint32_t, uint64_t,
@@ -253,10 +253,6 @@ bool gemm_fp8w_bf16(uint64_t, uint64_t, uint64_t, uint64_t, uint32_t, uint32_t, 
 bool gemm_split_reduce_launch(const float*, uint16_t*, const uint16_t*, int, int, uint64_t,
                               std::string* err) {
     return no_device(err);
-}
-void gemm_tiled_plan(uint32_t, uint32_t, uint32_t, int* splits, int* tile) {
-    *splits = 1;
-    *tile = -1;
 }
 bool gemm_plan(uint32_t, uint32_t, uint32_t, bool, GemmPlan*, std::string* err) {
     return no_device(err);

@@ -387,3 +387,51 @@ def test_gemm_plan(gpu_lib, tunables):
     assert gpu_lib.gemm_plan(256, 6144, 4096)["kernel"] == "stream"
     with pytest.raises(Exception):
         gpu_lib.gemm_plan(64, 100, 4096)          # n not a multiple of 64
+
+
+@pytest.mark.parametrize("tile", [101, 102, 103, 104, 124, 131])
+@pytest.mark.parametrize("m,n,k,splits", [(129, 320, 256, 1), (257, 576, 256, 1), (320, 64, 512, 2),
+                                          (513, 1344, 1024, 4), (700, 192, 512, 1)])
+def test_wide_kernel(gpu_lib, tunables, tile, m, n, k, splits):
+    """Every token-tile height of the wide kernel (KCMM_GEMM_TILE = 100 + fb0
+    [+ 10 fb1 for the second half of the weight tiles]: 64 fb tokens, ragged
+    last tiles of every height), weight tiles past N, the shortest K per
+    split, the residual in place and the SwiGLU store.  Bound: bf16 rounding
+    of the product (8 significant bits, to nearest: half a step of 2^-7, so
+    2^-8 of it; twice with the residual) plus fp32 sums of k terms (2^-23 k
+    sum|x||w|).  SwiGLU: the same bits as the plain product of
+    [gate; up] followed by silu_mul (the same sum order per output)."""
+    import torch
+    tunables.setenv("KCMM_GEMM_TILE", str(tile))
+    tunables.setenv("KCMM_GEMM_SPLITS", str(splits))
+    plan = gpu_lib.gemm_plan(m, n, k)
+    assert plan["tile"] == 100 + tile % 10 and plan["splits"] == splits
+    rng = np.random.default_rng(m + n + k + tile)
+    xb = O.encode(O.BF16, rng.standard_normal((m, k)))
+    wb = O.encode(O.BF16, rng.standard_normal((2 * n, k)) * 0.02)
+    rb = O.encode(O.BF16, rng.standard_normal((m, n)))
+    x = torch.from_numpy(xb.view(np.int16)).view(torch.bfloat16).cuda()
+    w = torch.from_numpy(wb.view(np.int16)).view(torch.bfloat16).cuda()
+    y = torch.from_numpy(rb.view(np.int16)).view(torch.bfloat16).cuda()
+    s = torch.cuda.current_stream().cuda_stream
+    gpu_lib.gemm_bf16_add(x.data_ptr(), w.data_ptr(), y.data_ptr(), y.data_ptr(), m, n, k, s)
+    z = run(gpu_lib, x, w[:n])
+    prod = O.gemm_bf16_f64(xb, wb[:n])
+    terms = k * 2.0 ** -23 * (np.abs(O.decode(O.BF16, xb)).astype(np.float64) @
+                              np.abs(O.decode(O.BF16, wb[:n])).astype(np.float64).T)
+    res = O.decode(O.BF16, rb).astype(np.float64)
+    u = 2.0 ** -8
+    for got, ref, bound in ((z, prod, u * np.abs(prod)),
+                            (y, prod + res, u * (np.abs(prod) + np.abs(prod + res)) * (1 + u))):
+        got = O.decode(O.BF16, got.cpu().view(torch.int16).numpy().view(np.uint16)).astype(np.float64)
+        worst = float((np.abs(got - ref) / (bound + (1 + u) * terms + 1e-30)).max())
+        print(f"wide {tile} {m}x{n}x{k}/{splits} worst {worst:.3f} of the bound", flush=True)
+        assert np.isfinite(got).all() and worst <= 1.0
+    if splits == 1:
+        act = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+        ref = torch.empty_like(act)
+        gu = run(gpu_lib, x, w)
+        gpu_lib.silu_mul_bf16(gu.data_ptr(), ref.data_ptr(), m, n, s)
+        gpu_lib.gemm_bf16_swiglu(x.data_ptr(), w.data_ptr(), act.data_ptr(), m, n, k, s)
+        torch.cuda.synchronize()
+        assert torch.equal(act.view(torch.int16), ref.view(torch.int16))
