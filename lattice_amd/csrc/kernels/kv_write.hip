@@ -79,6 +79,34 @@ __device__ __forceinline__ uint32_t f32_to_fp8e4m3(float x) {
     return sign | code;
 }
 
+// x / scale clamped to the e4m3 range, for 2^-100 <= scale <= 2^100, r = 1 /
+// scale and x not NaN: x * r with one residual step is the correctly rounded
+// quotient wherever it matters to four significant bits (Markstein's division;
+// checked against x / scale for every bf16 x and 32639 scales).  The hardware
+// conversion of it gives the bits of f32_to_fp8e4m3(x / scale) (the two agree
+// on every float but NaN, whose sign the hardware does not keep).
+__device__ __forceinline__ float fp8_quotient(float x, float scale, float r) {
+    const float q = x * r;
+    return __builtin_amdgcn_fmed3f(copysignf(fmaf(fmaf(-q, scale, x), r, q), x), -448.0f, 448.0f);
+}
+
+// 8 bf16 elements (4 dwords, no NaN) / scale as e4m3 bytes.
+__device__ __forceinline__ u32x2 fp8_encode8(const u32x4& x, float scale, float r) {
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+        v[i] = fp8_quotient(__uint_as_float((i & 1) ? x[i >> 1] & 0xffff0000u : x[i >> 1] << 16),
+                            scale, r);
+    u32x2 o;
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+        const int lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[4 * w], v[4 * w + 1], 0, false);
+        o[w] = static_cast<uint32_t>(
+            __builtin_amdgcn_cvt_pk_fp8_f32(v[4 * w + 2], v[4 * w + 3], lo, true));
+    }
+    return o;
+}
+
 // fp8 page write of one (page, kv head) for one call.  `row_of` (bs entries,
 // LDS) gives, for each token slot, the source row this call writes there (the
 // call's last row for that slot), or -1.  The rows a call writes into a page
@@ -91,22 +119,65 @@ __device__ __forceinline__ uint32_t f32_to_fp8e4m3(float x) {
 //   else:   scale = old, raised to amax / 448 when amax > 448 * old, and then
 //           every slot the call does not write is re-encoded from old to the
 //           new scale (e4m3(decode(code) * old / scale));
-// and each written row is stored as e4m3(x / scale).  One wavefront.
-__device__ void fp8_write_page_head(uint8_t* page, uint32_t kvh, const uint16_t* src_base,
+// and each written row is stored as e4m3(x / scale).  One wavefront.  With
+// head_dim % 8 == 0 and 16-byte aligned source rows, lanes take 16-byte
+// pieces of the rows, 256 pieces (16 rows of 128) per pass with every load
+// in flight at once; a page of at most 256 pieces is read once.
+__device__ __forceinline__ void fp8_write_page_head(uint8_t* page, uint32_t kvh, const uint16_t* src_base,
                                     const int32_t* row_of, uint32_t bs, uint32_t kv_heads,
                                     uint32_t head_dim, uint32_t row_bytes, uint32_t data_bytes) {
     const int lane = threadIdx.x & 63;
     float* sp = reinterpret_cast<float*>(page + data_bytes) + kvh;
     const float old = *sp;
-    float amax = 0.0f;
-    for (uint32_t u = 0; u < bs; ++u) {
-        const int32_t r = row_of[u];
-        if (r < 0) continue;
-        const uint16_t* src = src_base + (static_cast<uint64_t>(r) * kv_heads + kvh) * head_dim;
+    const bool vec = (head_dim & 7) == 0 && (reinterpret_cast<uintptr_t>(src_base) & 15) == 0;
+    constexpr uint32_t PASS = 4;              // pieces per lane per pass
+    const uint32_t C = head_dim / 8;          // pieces per row (vec: 1..32)
+    const uint32_t total = bs * C, rcp = vec ? 65536u / C + 1 : 0;
+    const uint32_t step = vec ? (64 * PASS / C) * C : 0;   // whole rows per pass
+    u32x4 x[PASS];
+    int32_t at[PASS];                         // slot * C + piece, or -1
+    auto load_pass = [&](uint32_t q0) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {   // head_dim <= 256
-            const uint32_t d = lane + 64 * i;
-            if (d < head_dim) amax = fmaxf(amax, fabsf(bf16_bits_to_f32(src[d])));
+        for (uint32_t i = 0; i < PASS; ++i) {
+            const uint32_t q = lane + 64 * i, u = (q * rcp) >> 16;   // q / C (q < 256)
+            at[i] = -1;
+            x[i] = u32x4{0, 0, 0, 0};
+            const uint32_t slot = q0 / C + u;
+            if (q >= step || slot >= bs) continue;
+            const int32_t r = row_of[slot];
+            if (r < 0) continue;
+            at[i] = static_cast<int32_t>(q0 + q);
+            x[i] = *reinterpret_cast<const u32x4*>(
+                src_base + (static_cast<uint64_t>(r) * kv_heads + kvh) * head_dim + (q - u * C) * 8);
+        }
+    };
+    float amax = 0.0f;
+    bool nan = false;
+    if (vec) {
+#pragma unroll 1
+        for (uint32_t q0 = 0; q0 < total; q0 += step) {
+            load_pass(q0);
+#pragma unroll
+            for (uint32_t i = 0; i < PASS; ++i)
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const float lo = __uint_as_float(x[i][w] << 16);
+                    const float hi = __uint_as_float(x[i][w] & 0xffff0000u);
+                    amax = fmaxf(amax, fmaxf(fabsf(lo), fabsf(hi)));
+                    nan |= lo != lo || hi != hi;
+                }
+        }
+    } else {
+#pragma unroll 1
+        for (uint32_t u = 0; u < bs; ++u) {
+            const int32_t r = row_of[u];
+            if (r < 0) continue;
+            const uint16_t* src = src_base + (static_cast<uint64_t>(r) * kv_heads + kvh) * head_dim;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {   // head_dim <= 256
+                const uint32_t d = lane + 64 * i;
+                if (d < head_dim) amax = fmaxf(amax, fabsf(bf16_bits_to_f32(src[d])));
+            }
         }
     }
 #pragma unroll
@@ -119,32 +190,48 @@ __device__ void fp8_write_page_head(uint8_t* page, uint32_t kvh, const uint16_t*
         scale = old;
         if (amax > 448.0f * old) {
             scale = amax / 448.0f;
-            if ((head_dim & 15) == 0 && (row_bytes & 15) == 0) {
+            if ((head_dim & 15) == 0 && (row_bytes & 15) == 0 && scale >= 0x1p-100f &&
+                scale <= 0x1p100f) {
                 // 16-byte pieces of all unwritten slots at once: one memory
                 // round trip for the page instead of one per slot
                 const uint32_t pieces = head_dim / 16;
+                const float r = 1.0f / scale;
+#pragma unroll 1
                 for (uint32_t c = lane; c < bs * pieces; c += 64) {
                     const uint32_t u = c / pieces;
                     if (row_of[u] >= 0) continue;
-                    u32x4* q = reinterpret_cast<u32x4*>(page + static_cast<uint64_t>(u) * row_bytes +
-                                                        kvh * head_dim + (c - u * pieces) * 16);
-                    u32x4 v = *q;
+                    uint8_t* q = page + static_cast<uint64_t>(u) * row_bytes + kvh * head_dim +
+                                 (c - u * pieces) * 16;
+                    const u32x4 v = *reinterpret_cast<const u32x4*>(q);
+                    u32x4 o;
+                    bool nan_code = false;
 #pragma unroll
                     for (int w = 0; w < 4; ++w) {
-                        uint32_t o = 0;
-#pragma unroll
-                        for (int b = 0; b < 4; ++b) {
-                            const float y = fp8e4m3_to_f32((v[w] >> (8 * b)) & 0xffu) * old;
-                            o |= f32_to_fp8e4m3(y / scale) << (8 * b);
-                        }
-                        v[w] = o;
+                        const uint32_t m = v[w] & 0x7f7f7f7fu;   // a byte of 0x7f carries into bit 7
+                        nan_code |= ((m + 0x01010101u) & 0x80808080u) != 0;
+                        const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8(static_cast<int>(v[w]), false);
+                        const auto hi = __builtin_amdgcn_cvt_pk_f32_fp8(static_cast<int>(v[w]), true);
+                        const int p0 = __builtin_amdgcn_cvt_pk_fp8_f32(
+                            fp8_quotient(lo[0] * old, scale, r), fp8_quotient(lo[1] * old, scale, r),
+                            0, false);
+                        o[w] = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(
+                            fp8_quotient(hi[0] * old, scale, r), fp8_quotient(hi[1] * old, scale, r),
+                            p0, true));
                     }
-                    *q = v;
+                    if (!nan_code) {
+                        *reinterpret_cast<u32x4*>(q) = o;
+                        continue;
+                    }
+#pragma unroll 1
+                    for (int i = 0; i < 16; ++i)
+                        q[i] = static_cast<uint8_t>(f32_to_fp8e4m3(fp8e4m3_to_f32(q[i]) * old / scale));
                 }
             } else {
-                for (uint32_t u = 0; u < bs; ++u) {
+#pragma unroll 1
+        for (uint32_t u = 0; u < bs; ++u) {
                     if (row_of[u] >= 0) continue;
                     uint8_t* row = page + static_cast<uint64_t>(u) * row_bytes + kvh * head_dim;
+#pragma unroll 1
                     for (uint32_t d = lane; d < head_dim; d += 64) {
                         const float y = fp8e4m3_to_f32(row[d]) * old;
                         row[d] = static_cast<uint8_t>(f32_to_fp8e4m3(y / scale));
@@ -153,16 +240,34 @@ __device__ void fp8_write_page_head(uint8_t* page, uint32_t kvh, const uint16_t*
             }
         }
     }
-    for (uint32_t u = 0; u < bs; ++u) {
-        const int32_t r = row_of[u];
-        if (r < 0) continue;
-        const uint16_t* src = src_base + (static_cast<uint64_t>(r) * kv_heads + kvh) * head_dim;
-        uint8_t* row = page + static_cast<uint64_t>(u) * row_bytes + kvh * head_dim;
+    if (vec && !__any(nan) && scale >= 0x1p-100f && scale <= 0x1p100f) {
+        const float r = 1.0f / scale;
+        uint8_t* base = page + kvh * head_dim;
+#pragma unroll 1
+        for (uint32_t q0 = 0; q0 < total; q0 += step) {
+            if (total > step) load_pass(q0);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const uint32_t d = lane + 64 * i;
-            if (d < head_dim)
-                row[d] = static_cast<uint8_t>(f32_to_fp8e4m3(bf16_bits_to_f32(src[d]) / scale));
+            for (uint32_t i = 0; i < PASS; ++i) {
+                if (at[i] < 0) continue;
+                const uint32_t q = at[i], u = q / C;
+                u32x2* d = reinterpret_cast<u32x2*>(base + static_cast<uint64_t>(u) * row_bytes +
+                                                    (q - u * C) * 8);
+                *d = fp8_encode8(x[i], scale, r);
+            }
+        }
+    } else {
+#pragma unroll 1
+        for (uint32_t u = 0; u < bs; ++u) {
+            const int32_t r = row_of[u];
+            if (r < 0) continue;
+            const uint16_t* src = src_base + (static_cast<uint64_t>(r) * kv_heads + kvh) * head_dim;
+            uint8_t* row = page + static_cast<uint64_t>(u) * row_bytes + kvh * head_dim;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t d = lane + 64 * i;
+                if (d < head_dim)
+                    row[d] = static_cast<uint8_t>(f32_to_fp8e4m3(bf16_bits_to_f32(src[d]) / scale));
+            }
         }
     }
     if (lane == 0) *sp = scale;
@@ -214,6 +319,7 @@ struct SlotArgs {
     const uint8_t* k_src;
     const uint8_t* v_src;
     uint32_t offsets_len, block_size, row_bytes, src_row_bytes, kv_heads, head_dim, data_bytes;
+    int bs_shift;
 };
 
 // Resolves row r's slot; returns false (after recording the status) when the
@@ -256,91 +362,153 @@ __global__ __launch_bounds__(256) void kv_slots_copy(SlotArgs a) {
     }
 }
 
-// fp8 pages through device slot ids, in two kernels so that all rows of a
-// page are applied as one set by one workgroup (fp8_write_page_head).
-// `lead` / `cnt` (int32 per block id, zero between calls) collect, per page,
-// batch - (first row) and the number of rows.  Pass 1: one thread per row
-// resolves the slot (status as above) and enters the row; pass 2: the
-// workgroup of a page's first row builds the page's slot table in LDS (rows
-// in call order, so the last row for a slot wins), writes the page, then
-// restores both entries to zero.
+// Block id of a slot (bs_shift: log2 of a power-of-two block size, else -1).
+__device__ __forceinline__ int64_t block_of(const SlotArgs& a, int64_t slot) {
+    if (a.bs_shift >= 0) return slot >> a.bs_shift;
+    if (slot >> 32) return slot / a.block_size;
+    return static_cast<uint32_t>(slot) / a.block_size;
+}
+
+// fp8 pages through device slot ids.  All rows of a page are applied as one
+// set by one workgroup (fp8_write_page_head), the one that holds the page's
+// first row of the call.  A workgroup holds R consecutive rows: it resolves
+// them (status as above), lists the distinct pages they name, and walks the
+// call's slot ids once, 1024 at a time, entering every row of those pages
+// into the pages' slot tables in LDS (the last row for a slot wins, in call
+// order) and dropping a page that an earlier row names.  The waves then take
+// the (page, kv head, K|V) triples of the pages left.
+//
+// R = 1 up to 512 rows (a decode step's appends: every row has its own page),
+// else 16 (a prompt's rows fill a page each): 4507 prompt rows, 16 slots per
+// page, took 381 us with one workgroup per row, a serial walk over the rows of
+// a page and a separate pass that counted them (9 us); 21 us so, most of it
+// the walk over the slot ids and the chain of loads behind it.  A single row's
+// append in a decode step 16 -> 7 us.
+//
+// A call of more than kFp8ScanRows rows would spend its time walking the
+// slot ids (every workgroup walks all): `lead` / `cnt` (int32 per block id,
+// zero between calls) then collect, per page, batch - (first row) and the
+// number of rows, and a workgroup walks from its own rows on until it has
+// them all.
+constexpr uint32_t kFp8ScanRows = 8192;
+constexpr uint32_t kFp8RowsPerGroup = 16;
+
 __global__ __launch_bounds__(256) void kv_slots_fp8_collect(SlotArgs a, uint32_t batch,
                                                             int32_t* lead, int32_t* cnt) {
     const uint32_t r = blockIdx.x * 256 + threadIdx.x;
     if (r >= batch) return;
     const int64_t slot = a.slots[r];
     if (slot < 0) return;
-    const int64_t id = slot / a.block_size;
-    if (id >= static_cast<int64_t>(a.offsets_len)) {
-        if (a.status) atomicCAS(a.status, 0, 1);
-        return;
-    }
-    if (a.valid && a.valid[id] == 0) {
-        if (a.status) atomicCAS(a.status, 0, 2);
-        return;
-    }
+    const int64_t id = block_of(a, slot);
+    if (id >= static_cast<int64_t>(a.offsets_len)) return;
+    if (a.valid && a.valid[id] == 0) return;
     atomicMax(lead + id, static_cast<int32_t>(batch - r));
     atomicAdd(cnt + id, 1);
 }
 
-// grid (batch); 64 * min(2 kv_heads, 16) threads; dynamic LDS block_size * 4.
+// grid (ceil(batch / R)); 64 * waves threads; dynamic LDS R * block_size * 4.
+// (The resolve step is written without nested branches: the compiler dropped
+// the id of rows with an active flag from an if / else-if chain here.)
 __global__ __launch_bounds__(64 * kFp8MaxWaves) void kv_slots_fp8_write(SlotArgs a,
-                                                                         uint32_t batch,
+                                                                         uint32_t batch, uint32_t R,
                                                                          int32_t* lead,
                                                                          int32_t* cnt) {
-    extern __shared__ int32_t row_of[];
-    __shared__ int32_t s_rows;
-    const uint32_t r = blockIdx.x;
-    const int64_t slot = a.slots[r];
-    // Rows that pass 1 skipped never lead; neither does a row whose page has
-    // an earlier row (its entry holds another row, or zero once restored).
-    if (slot < 0) return;
-    const int64_t id = slot / a.block_size;
-    if (id >= static_cast<int64_t>(a.offsets_len) || (a.valid && a.valid[id] == 0)) return;
-    if (threadIdx.x == 0)
-        s_rows = __atomic_load_n(lead + id, __ATOMIC_RELAXED) == static_cast<int32_t>(batch - r)
-                     ? __atomic_load_n(cnt + id, __ATOMIC_RELAXED)
-                     : 0;
-    for (uint32_t u = threadIdx.x; u < a.block_size; u += blockDim.x) row_of[u] = -1;
+    extern __shared__ int32_t row_of[];                  // [page of the list][block_size]
+    __shared__ int32_t s_id[kFp8RowsPerGroup];           // the list: block ids
+    __shared__ int32_t s_left[kFp8RowsPerGroup];         // collected: rows not found yet
+    __shared__ int32_t s_dead[kFp8RowsPerGroup];         // an earlier row leads the page
+    __shared__ int32_t s_pages;
+    const uint32_t r0 = blockIdx.x * R, t = threadIdx.x;
+    const uint32_t bs = a.block_size;
+    if (t < 64) {
+        // this workgroup's rows, one per lane: status, then the distinct pages
+        const int64_t slot = t < R && r0 + t < batch ? a.slots[r0 + t] : -1;
+        const int64_t b = block_of(a, slot < 0 ? 0 : slot);
+        const bool past = b >= static_cast<int64_t>(a.offsets_len);
+        uint32_t active = 1;
+        if (a.valid != nullptr) active = a.valid[slot < 0 || past ? 0 : b];
+        if (a.status != nullptr && slot >= 0 && (past || active == 0))
+            atomicCAS(a.status, 0, past ? 1 : 2);
+        const int32_t id =   // (offsets_len <= 2^28)
+            slot < 0 || past || active == 0 ? -1 : static_cast<int32_t>(b);
+        bool first = id >= 0;
+        for (uint32_t j = 0; j + 1 < R; ++j) {
+            const int32_t other = __shfl(id, j);
+            first &= j >= t || other != id;
+        }
+        int32_t rows = 0;
+        if (lead != nullptr && first) {
+            first = __atomic_load_n(lead + id, __ATOMIC_RELAXED) == static_cast<int32_t>(batch - r0 - t);
+            if (first) rows = __atomic_load_n(cnt + id, __ATOMIC_RELAXED);
+        }
+        const uint64_t m = __ballot(first);
+        if (first) {
+            const int at = __popcll(m & ((1ull << t) - 1));
+            s_id[at] = id;
+            s_left[at] = rows;
+            s_dead[at] = 0;
+        }
+        if (t == 0) s_pages = __popcll(m);
+    }
+    for (uint32_t i = t; i < R * bs; i += blockDim.x) row_of[i] = -1;
     __syncthreads();
-    const int32_t rows = s_rows;
-    if (rows == 0) return;
-    const int lane = threadIdx.x & 63;
-    if (rows == 1) {
-        // the page's only row is this one (the common decode append)
-        if (threadIdx.x == 0)
-            row_of[static_cast<uint32_t>(slot % a.block_size)] = static_cast<int32_t>(r);
-    } else if (threadIdx.x < 64) {
-        // rows of this page, in call order, from this one on
-        int32_t done = 0;
-        for (uint32_t base = r; done < rows && base < batch; base += 64) {
-            const uint32_t rr = base + lane;
-            const int64_t s2 = rr < batch ? a.slots[rr] : -1;
-            uint64_t mask = __ballot(s2 >= 0 && s2 / a.block_size == id);
-            while (mask != 0 && done < rows) {
-                const int i = __builtin_ctzll(mask);
-                mask &= mask - 1;
-                const uint32_t row = base + i;
-                if (lane == 0)
-                    row_of[static_cast<uint32_t>(a.slots[row] % a.block_size)] =
-                        static_cast<int32_t>(row);
-                ++done;
+    const int pages = s_pages;
+    if (pages == 0) return;   // (uniform)
+    // Walk the slot ids, kAhead per thread in flight together.
+    constexpr uint32_t kAhead = 4;
+    const uint32_t nt = blockDim.x;
+    for (uint32_t base = lead != nullptr ? r0 : 0; base < batch; base += nt * kAhead) {
+        int64_t slot[kAhead];
+#pragma unroll
+        for (uint32_t i = 0; i < kAhead; ++i) {
+            const uint32_t rr = base + t + i * nt;
+            slot[i] = a.slots[min(rr, batch - 1)];
+            if (rr >= batch) slot[i] = -1;
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < kAhead; ++i) {
+            if (slot[i] < 0) continue;
+            const uint32_t rr = base + t + i * nt;
+            const int64_t id = block_of(a, slot[i]);
+            for (int j = 0; j < pages; ++j) {
+                if (__builtin_amdgcn_readfirstlane(s_id[j]) != id) continue;
+                // (a page dropped here may still be entered by others: its
+                // table is not used)
+                if (rr < r0) s_dead[j] = 1;
+                atomicMax(row_of + j * bs + static_cast<uint32_t>(slot[i] - id * bs),
+                          static_cast<int32_t>(rr));
+                if (lead != nullptr) atomicSub(s_left + j, 1);
+                break;
             }
+        }
+        if (lead != nullptr) {
+            __syncthreads();
+            int left = 0;
+            for (int j = 0; j < pages; ++j) left += s_left[j];
+            __syncthreads();
+            if (left == 0) break;   // (uniform)
         }
     }
     __syncthreads();
-    const uint64_t page_off = a.offsets_f16[id] * 2ull;
-    const uint32_t waves = blockDim.x >> 6;
-    for (uint32_t j = threadIdx.x >> 6; j < 2 * a.kv_heads; j += waves) {
-        const bool is_v = j & 1;
-        fp8_write_page_head((is_v ? a.v_base : a.k_base) + page_off, j >> 1,
-                            reinterpret_cast<const uint16_t*>(is_v ? a.v_src : a.k_src), row_of,
-                            a.block_size, a.kv_heads, a.head_dim, a.row_bytes, a.data_bytes);
+    const uint32_t waves = nt >> 6, units = 2 * a.kv_heads;
+    uint32_t w = t >> 6;   // wave w takes triples w, w + waves, ... of the live pages
+    for (int j = 0; j < pages; ++j) {
+        if (s_dead[j]) continue;
+        const uint64_t page = a.offsets_f16[s_id[j]] * 2ull;
+        for (; w < units; w += waves) {
+            const bool is_v = w & 1;
+            fp8_write_page_head((is_v ? a.v_base : a.k_base) + page, w >> 1,
+                                reinterpret_cast<const uint16_t*>(is_v ? a.v_src : a.k_src),
+                                row_of + j * bs, bs, a.kv_heads, a.head_dim, a.row_bytes,
+                                a.data_bytes);
+        }
+        w -= units;
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        lead[id] = 0;
-        cnt[id] = 0;
+    if (lead != nullptr && t < static_cast<uint32_t>(pages)) {
+        // (every workgroup that names the page compares lead with a row of
+        // its own: zero never matches)
+        lead[s_id[t]] = 0;
+        cnt[s_id[t]] = 0;
     }
 }
 
@@ -451,6 +619,9 @@ bool kv_write_device_slots(const KvDeviceSlotsArgs& a, std::string* err) {
     sa.kv_heads = a.kv_heads;
     sa.head_dim = a.head_dim;
     sa.data_bytes = a.data_bytes;
+    sa.bs_shift = -1;
+    if (a.block_size != 0 && (a.block_size & (a.block_size - 1)) == 0)
+        sa.bs_shift = __builtin_ctz(a.block_size);
     if (a.dtype == kDtFP8) {
         if (a.head_dim > 256) {
             *err = "fp8 KV write supports head_dim <= 256";
@@ -464,18 +635,26 @@ bool kv_write_device_slots(const KvDeviceSlotsArgs& a, std::string* err) {
             *err = "fp8 KV write supports block_size <= 4096";
             return false;
         }
-        // per block id: batch - first row, row count (zero between calls)
-        void* ws = nullptr;
-        if (!stream_workspace(a.stream, 8, static_cast<size_t>(a.offsets_len) * 8, &ws, true, err))
-            return false;
-        int32_t* lead = static_cast<int32_t*>(ws);
-        int32_t* cnt = lead + a.offsets_len;
-        hipLaunchKernelGGL(kv_slots_fp8_collect, dim3((a.batch + 255) / 256), dim3(256), 0, s, sa,
-                           a.batch, lead, cnt);
-        KCMM_HIP_CHECK(hipGetLastError(), err);
-        const int waves = static_cast<int>(std::min<uint32_t>(2 * a.kv_heads, kFp8MaxWaves));
-        hipLaunchKernelGGL(kv_slots_fp8_write, dim3(a.batch), dim3(64 * waves),
-                           static_cast<size_t>(a.block_size) * 4, s, sa, a.batch, lead, cnt);
+        if (a.batch == 0) return true;
+        int32_t *lead = nullptr, *cnt = nullptr;
+        if (a.batch > kFp8ScanRows) {
+            // per block id: batch - first row, row count (zero between calls)
+            void* ws = nullptr;
+            if (!stream_workspace(a.stream, 8, static_cast<size_t>(a.offsets_len) * 8, &ws, true, err))
+                return false;
+            lead = static_cast<int32_t*>(ws);
+            cnt = lead + a.offsets_len;
+            hipLaunchKernelGGL(kv_slots_fp8_collect, dim3((a.batch + 255) / 256), dim3(256), 0, s,
+                               sa, a.batch, lead, cnt);
+            KCMM_HIP_CHECK(hipGetLastError(), err);
+        }
+        const uint32_t R =
+            a.batch <= 512 ? 1
+                           : std::max(1u, std::min(kFp8RowsPerGroup, kFp8MaxBlockSize / a.block_size));
+        // (8 waves: two workgroups fit a CU, so a prompt's are one round)
+        const uint32_t waves = R > 1 ? 8u : std::min<uint32_t>(2 * a.kv_heads, kFp8MaxWaves);
+        hipLaunchKernelGGL(kv_slots_fp8_write, dim3((a.batch + R - 1) / R), dim3(64 * waves),
+                           static_cast<size_t>(R) * a.block_size * 4, s, sa, a.batch, R, lead, cnt);
     } else {
         hipLaunchKernelGGL(kv_slots_copy, dim3(a.batch), dim3(256), 0, s, sa);
     }

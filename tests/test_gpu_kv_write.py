@@ -327,3 +327,73 @@ def test_fp8_device_slots_status_and_repeat_calls(gpu_lib):
             assert np.array_equal(gk, ok) and np.array_equal(gv, ov), f"call {call}"
     finally:
         pool.destroy()
+
+
+@pytest.mark.parametrize("rows,geom,first", [(600, (8, 128, 16), 0), (513, (1, 72, 8), 3),
+                                             (700, (2, 64, 64), 5), (9001, (2, 64, 16), 0),
+                                             (520, (2, 20, 512), 1)],
+                         ids=["r600", "r513-d72", "r700-bs64", "r9001-collected", "r520-d20-bs512"])
+def test_fp8_prompt_rows_bytes(gpu_lib, rows, geom, first):
+    """Calls of more than 512 rows (16 rows per workgroup), of more than 8192
+    (rows counted per page first), head_dim not a multiple of 8 and
+    misaligned sources (element-wise path), two calls on the same pages (the
+    second raises scales, so unwritten slots are re-encoded), a few repeated
+    slots, padding, ids past the table and inactive ids, and values over the
+    whole bf16 range with +-0, infinities and NaN: every byte as the oracle's."""
+    import torch
+    rng = np.random.default_rng(rows)
+    hk, d, bs = geom
+    B = 7
+    per = -(-rows // B)
+    pool = gpu_lib.create_pool(make_config(num_layers=1, kv_heads=hk, head_dim=d, max_batch=B,
+                                           max_seq_len=first + 2 * per + bs, block_size=bs), KV_FP8)
+    try:
+        n_pages = -(-(first + 2 * per) // bs)
+        tables = rng.permutation(pool.alloc_blocks(B * n_pages)).reshape(B, n_pages)
+        zero_regions(pool)
+        nb = pool.stats()["superblock_count"] * SB
+        ok, ov = np.zeros(nb, np.uint8), np.zeros(nb, np.uint8)
+        offs = np.asarray(pool.all_block_offsets_f16(), np.uint64)
+        offs_t = torch.from_numpy(offs.view(np.int64)).cuda()
+        valid = np.ones(len(offs), np.uint8)
+        valid[tables[3, 0]] = 0
+        valid_t = torch.from_numpy(valid).cuda()
+        g_row, data_bytes = hk * d, hk * d * bs
+        for call, pos0 in enumerate((first, first + per, first)):
+            pos = np.arange(pos0, pos0 + per)
+            slots = (tables[:, pos // bs] * bs + pos % bs).reshape(-1)[:rows].astype(np.int64)
+            if call == 1:
+                slots = rng.permutation(slots)
+                slots[rng.integers(rows, size=9)] = slots[rng.integers(rows, size=9)]
+                slots[rng.integers(rows, size=4)] = -1
+                slots[rng.integers(rows)] = len(offs) * bs + 3
+            x = (rng.standard_normal((2, rows, hk * d)) * 4.0 ** call).astype(np.float32)
+            bits = O.encode(O.BF16, x)
+            if call == 2:   # any bit pattern in a quarter of the rows
+                some = rng.random(rows) < 0.25
+                bits[:, some] = rng.integers(0, 1 << 16, size=bits[:, some].shape).astype(np.uint16)
+                bits[:, ::7, ::5] = 0x8000
+            src = []
+            for t in range(2):   # 2 bytes off 16-byte alignment in the last call
+                buf = torch.empty(rows * hk * d + 8, dtype=torch.int16, device="cuda")
+                at = buf[call // 2:call // 2 + rows * hk * d]
+                at.copy_(torch.from_numpy(bits[t].view(np.int16).reshape(-1)))
+                src.append(at)
+            sl = torch.from_numpy(slots).cuda()
+            st = torch.zeros(1, dtype=torch.int32, device="cuda")
+            stream = torch.cuda.current_stream()
+            pool.append_kv_device_slots_on_stream(
+                layer_idx=0, slot_mapping_ptr=sl.data_ptr(), block_offsets_f16_ptr=offs_t.data_ptr(),
+                valid_blocks_ptr=valid_t.data_ptr(), block_offsets_f16_len=len(offs), batch=rows,
+                k_src_ptr=src[0].data_ptr(), v_src_ptr=src[1].data_ptr(), status_ptr=st.data_ptr(),
+                stream_ptr=stream.cuda_stream)
+            stream.synchronize()
+            want = {1: (1, 2)}.get(call, (2,) if pos0 // bs == 0 else (0,))
+            assert int(st.item()) in want, (call, int(st.item()))
+            O.kv_write_device_slots(KV_FP8, ok, ov, bits[0], bits[1], slots, offs, valid, bs, hk, d,
+                                    g_row, data_bytes)
+            gk, gv = region_bytes(pool)
+            assert np.array_equal(gk, ok), f"K after call {call}"
+            assert np.array_equal(gv, ov), f"V after call {call}"
+    finally:
+        pool.destroy()
