@@ -15,8 +15,7 @@
 //    workgroup read the same tokens' rows of neighbouring heads together:
 //    with HW = Hkv a workgroup reads whole token rows (all heads, 2 KiB
 //    contiguous at the Llama-3-8B shape) instead of one head's 256-byte
-//    pieces at a 2 KiB stride (used for fp8 pages, HW = 8; 16-bit pages
-//    run HW = 1, one wave per workgroup);
+//    pieces at a 2 KiB stride (HW by the batch's size, see stream_hw);
 //  * one tile read serves all G = Hq/Hkv query heads of its kv head (GQA
 //    reuse: each K/V byte is read from HBM once);
 //  * every load instruction covers eight tokens x 128 contiguous bytes (whole
@@ -140,7 +139,7 @@ struct AttnParams {
     int row_bytes, data_bytes;
     int hw;                 // waves per workgroup = kv heads per head block (divides Hkv)
     int total_waves;        // slices = workgroups of the streaming kernel
-    int min_tiles;          // smallest slice a wave takes
+    int min_tiles;          // smallest slice a wave takes; 0: by length (wave_slice)
     float scale_log2;       // scale * log2(e)
 };
 
@@ -184,10 +183,21 @@ __device__ __forceinline__ f32x4 mfma16x16x32(u32x4 a, u32x4 b, f32x4 c) {
 __device__ __forceinline__ int clamp_len(int L, int cap) { return L < 0 ? 0 : (L > cap ? cap : L); }
 __device__ __forceinline__ int tiles_of(int L) { return (L + 31) >> 5; }
 
-// Slice length of one workgroup for `total` tiles.
+// Slice length of one workgroup for `total` tiles: equal slices for all of
+// them, but not so short that the merge of the many parts costs more than the
+// shorter slices save.  By the mean tiles of a (sequence, head block): up to
+// 32, one tile per slice; up to 160, two; else four.  Call times by slice
+// length, one sequence of 32/8 heads of 128, bf16: 800 tokens 10.0 us (1), 11.0
+// (2), 13.5 (4), 18.8 (8); 3000 tokens 14.3 / 12.5 / 14.0 / 19.9; 10000 tokens
+// 21.0 (3), 18.5 (4), 21.6 (8).
 __device__ __forceinline__ int wave_slice(int total, const AttnParams& p) {
     const int per = (total + p.total_waves - 1) / p.total_waves;
-    return per > p.min_tiles ? per : p.min_tiles;
+    int least = p.min_tiles;
+    if (least == 0) {
+        const int lists = p.batch * (p.kv_heads / p.hw);
+        least = total <= 32 * lists ? 1 : total <= 160 * lists ? 2 : 4;
+    }
+    return per > least ? per : least;
 }
 
 // One 32-token tile: 2 halves of 16 tokens, KC 16-byte fragments per lane
@@ -742,47 +752,54 @@ void attn_decode_stream(AttnParams p, const int32_t* __restrict__ bt,
     }
 }
 
-// Log-sum-exp merge, one wave per (b, kv head g) that spans several slices
-// of the streaming kernel: part k of the np parts from slice wa on sits at
-// the (b, g) unit k for k < kSegPieces and in slot 0 of the wave for g of
-// slice wa+k after that (wave rows (wa + k) * HW + g % HW).  The
-// (max, denominator) pairs of parts 0..kSegPieces-1 (one part per lane) and
-// the accumulators of the first QP parts are loaded together with the
-// segment record, so a (b, g) of at most kSegPieces parts takes one memory
-// step; parts past kSegPieces wait for the record.  The weights reach every
-// lane through v_readlane.  NO = outputs per lane rounded up to a power of
-// two; loads past np read stale units whose values are masked out.
-template <int DT, int D, int NO>
-__global__ __launch_bounds__(64) void attn_decode_merge(AttnParams p,
-                                                        const int2* __restrict__ info) {
-    constexpr int NJ = NO * 64 / D > 0 ? NO * 64 / D : 1;   // heads covered (power of two)
-    constexpr int QP = NO >= 16 ? 2 : 32 / NO > 4 ? 4 : 32 / NO;   // parts per round
-    static_assert(QP <= kSegPieces, "the first round's accumulators are segment-indexed");
-    const int lane = threadIdx.x;
+// Log-sum-exp merge, one 4-wave workgroup per (b, kv head g) that spans several
+// slices of the streaming kernel (and per 1024 outputs): part k of the np
+// parts from slice wa on sits at the (b, g) unit k for k < kSegPieces and in
+// slot 0 of the wave for g of slice wa+k after that (wave rows (wa + k) * HW +
+// g % HW).  Threads split the outputs four at a time and the parts S ways (the
+// sums meet in LDS); waves share the heads' weights, one part per lane.  The
+// (max, denominator) pairs and accumulators of the first kSegPieces parts are
+// loaded together with the segment record, so a (b, g) of few parts takes one
+// memory step; all others follow in one more per 4 S parts (one wave per (b, g)
+// walked them four at a time: 64 parts took 15.8 us, 5.6 so).
+constexpr int kMergeParts = 128;   // parts per pass over the weights
+template <int DT, int D, int S, int NT>
+__global__ __launch_bounds__(NT) void attn_decode_merge(AttnParams p,
+                                                         const int2* __restrict__ info) {
+    constexpr int OG = NT / S;                             // output quads per workgroup
+    constexpr int HB = OG * 4 / D > 0 ? OG * 4 / D : 1;    // heads per workgroup
+    constexpr int NPRE = S >= kSegPieces ? 1 : kSegPieces / S;
+    constexpr int NW = NT / 64;
+    constexpr int HPW = (HB + NW - 1) / NW;                // heads per wave
+    __shared__ float s_w[HB][kMergeParts];
+    __shared__ float s_scale[HB], s_inv[HB];
+    __shared__ f32x4 s_red[S > 1 ? NT : 1];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int G = p.group;
     const int b = blockIdx.x / p.kv_heads;
     const int g = blockIdx.x - b * p.kv_heads;
-    const int n_out = G * D / 64;      // lane holds outputs lane + 64e, e < n_out
+    const int o = tid % OG, sl = tid / OG;
+    const int h0 = blockIdx.y * HB;
+    // threads past the last quad read it again and store nothing
+    const int quads = G * D / 4, quad = min(static_cast<int>(blockIdx.y) * OG + o, quads - 1);
+    const int hl = min(o * 4 / D, HB - 1);
     const size_t seg0 = p.seg_unit0 + static_cast<size_t>(blockIdx.x) * kSegPieces;
+    auto acc_at = [&](size_t unit) {
+        return *reinterpret_cast<const f32x4*>(p.part_acc + unit * G * D + quad * 4);
+    };
 
-    // first round, before the record: (max, denominator) of part min(lane, 3)
-    // and the accumulators of parts 0 .. QP-1
-    float m[NJ], l[NJ], v[QP][NO];
-    {
-        const size_t u0 = seg0 + min(lane, kSegPieces - 1);
+    // before the record: parts 0 .. kSegPieces-1
+    float m[HPW][2], l[HPW][2];   // parts lane, lane + 64 of heads wave, wave + NW, ...
+    f32x4 pre[NPRE];
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            const size_t u = (u0 * G + min(j, G - 1)) * 2;
-            m[j] = p.part_ml[u];
-            l[j] = p.part_ml[u + 1];
-        }
-#pragma unroll
-        for (int q = 0; q < QP; ++q) {
-            const float* pa = p.part_acc + (seg0 + q) * G * D + lane;
-#pragma unroll
-            for (int e = 0; e < NO; ++e) v[q][e] = pa[min(e, n_out - 1) * 64];
-        }
+    for (int i = 0; i < HPW; ++i) {
+        const int h = min(h0 + wave + NW * i, G - 1);
+        const size_t u = ((seg0 + min(lane, kSegPieces - 1)) * G + h) * 2;
+        m[i][0] = p.part_ml[u];
+        l[i][0] = p.part_ml[u + 1];
     }
+#pragma unroll
+    for (int i = 0; i < NPRE; ++i) pre[i] = acc_at(seg0 + min(sl + i * S, kSegPieces - 1));
     const int2 si = info[blockIdx.x];
     const int wa = si.x, np = si.y;
     if (np <= 1) return;
@@ -790,92 +807,114 @@ __global__ __launch_bounds__(64) void attn_decode_merge(AttnParams p,
     auto unit = [&](int k) -> size_t {
         return k < kSegPieces ? seg0 + k : (static_cast<size_t>(wa + k) * p.hw + gofs) * 2;
     };
-    auto load_parts = [&](float (&v)[QP][NO], int k0) {
-#pragma unroll
-        for (int q = 0; q < QP; ++q) {
-            const float* pa = p.part_acc + unit(min(k0 + q, np - 1)) * G * D + lane;
-#pragma unroll
-            for (int e = 0; e < NO; ++e) v[q][e] = pa[min(e, n_out - 1) * 64];
-        }
-    };
 
-    float mx[NJ], ls[NJ], acc[NO];
+    f32x4 acc = f32x4{0, 0, 0, 0};
+    float mx[HPW], ls[HPW];
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-        mx[j] = -INFINITY;
-        ls[j] = 0.0f;
+    for (int i = 0; i < HPW; ++i) {
+        mx[i] = -INFINITY;
+        ls[i] = 0.0f;
     }
+    for (int k0 = 0; k0 < np; k0 += kMergeParts) {
+        // weights of parts k0 .. k0 + 127, one or two per lane
 #pragma unroll
-    for (int e = 0; e < NO; ++e) acc[e] = 0.0f;
-    for (int k0 = 0; k0 < np; k0 += 64) {
-        const bool live = k0 + lane < np;
-        const int k = min(k0 + lane, np - 1);
-        // lanes whose part is not among the ones loaded above
-        if (k0 > 0 || (np > kSegPieces && lane >= kSegPieces)) {
+        for (int i = 0; i < HPW; ++i) {
+            const int h = min(h0 + wave + NW * i, G - 1);
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                const size_t u = (unit(k) * G + min(j, G - 1)) * 2;
-                m[j] = p.part_ml[u];
-                l[j] = p.part_ml[u + 1];
-            }
-        }
-        if (k0 > 0) load_parts(v, k0);   // in flight with the (max, denominator) loads
-        float w[NJ];
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-            float cm = live ? m[j] : -INFINITY;
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) cm = fmaxf(cm, __shfl_xor(cm, o));
-            const float nm = fmaxf(mx[j], cm);
-            const float corr = mx[j] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mx[j] - nm);
-            w[j] = live ? __builtin_amdgcn_exp2f(m[j] - nm) : 0.0f;
-            float wl = w[j] * l[j];
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) wl += __shfl_xor(wl, o);
-            ls[j] = ls[j] * corr + wl;
-            mx[j] = nm;
-#pragma unroll
-            for (int e = 0; e < NO; ++e)
-                if (e * 64 / D == j) acc[e] *= corr;
-        }
-        const int kn = min(64, np - k0);
-        for (int kk0 = 0; kk0 < kn; kk0 += QP) {
-            if (kk0 > 0) load_parts(v, k0 + kk0);
-#pragma unroll
-            for (int q = 0; q < QP; ++q) {
-                const int kk = min(kk0 + q, kn - 1);
-#pragma unroll
-                for (int e = 0; e < NO; ++e) {
-                    const float wt = __int_as_float(
-                        __builtin_amdgcn_readlane(__float_as_int(w[e * 64 / D]), kk));
-                    acc[e] += kk0 + q < kn ? wt * v[q][e] : 0.0f;
+            for (int e = 0; e < 2; ++e) {
+                const int k = k0 + lane + 64 * e;
+                if ((k >= kSegPieces || k0 > 0) && k < np) {
+                    const size_t u = (unit(k) * G + h) * 2;
+                    m[i][e] = p.part_ml[u];
+                    l[i][e] = p.part_ml[u + 1];
                 }
             }
         }
-    }
-    uint16_t* out = reinterpret_cast<uint16_t*>(p.out) +
-                    (static_cast<size_t>(b) * p.num_q_heads + g * G) * D + lane;
 #pragma unroll
-    for (int e = 0; e < NO; ++e)
-        if (e < n_out) out[e * 64] = static_cast<uint16_t>(f32_to_elem<DT>(acc[e] / ls[e * 64 / D]));
+        for (int i = 0; i < HPW; ++i) {
+            const int h = wave + NW * i;
+            const bool live0 = k0 + lane < np, live1 = k0 + lane + 64 < np;
+            float cm = fmaxf(live0 ? m[i][0] : -INFINITY, live1 ? m[i][1] : -INFINITY);
+#pragma unroll
+            for (int x = 32; x > 0; x >>= 1) cm = fmaxf(cm, __shfl_xor(cm, x));
+            const float nm = fmaxf(mx[i], cm);
+            const float corr = mx[i] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mx[i] - nm);
+            const float w0 = live0 ? __builtin_amdgcn_exp2f(m[i][0] - nm) : 0.0f;
+            const float w1 = live1 ? __builtin_amdgcn_exp2f(m[i][1] - nm) : 0.0f;
+            float wl = (live0 ? w0 * l[i][0] : 0.0f) + (live1 ? w1 * l[i][1] : 0.0f);
+#pragma unroll
+            for (int x = 32; x > 0; x >>= 1) wl += __shfl_xor(wl, x);
+            ls[i] = ls[i] * corr + wl;
+            mx[i] = nm;
+            if (h < HB) {
+                s_w[h][lane] = w0;
+                s_w[h][lane + 64] = w1;
+                if (lane == 0) {
+                    s_scale[h] = corr;
+                    s_inv[h] = 1.0f / ls[i];
+                }
+            }
+        }
+        __syncthreads();
+        if (k0 > 0) acc *= s_scale[hl];
+        const int kn = min(kMergeParts, np - k0);
+        int k = sl;
+        if (k0 == 0) {
+#pragma unroll
+            for (int i = 0; i < NPRE; ++i) {
+                if (k < min(kn, kSegPieces)) {
+                    acc += s_w[hl][k] * pre[i];
+                    k += S;
+                }
+            }
+        }
+        for (; k < kn; k += 4 * S) {
+            f32x4 v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = acc_at(unit(min(k0 + k + i * S, np - 1)));
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (k + i * S < kn) acc += s_w[hl][k + i * S] * v[i];
+        }
+        __syncthreads();   // the weights are read
+    }
+    if constexpr (S > 1) {
+        s_red[tid] = acc;
+        __syncthreads();
+        if (sl > 0) return;
+#pragma unroll
+        for (int i = 1; i < S; ++i) acc += s_red[i * OG + o];
+    }
+    if (static_cast<int>(blockIdx.y) * OG + o >= quads) return;
+    acc *= s_inv[hl];
+    u32x2 w;
+    w[0] = f32_to_elem<DT>(acc[0]) | (f32_to_elem<DT>(acc[1]) << 16);
+    w[1] = f32_to_elem<DT>(acc[2]) | (f32_to_elem<DT>(acc[3]) << 16);
+    *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(p.out) +
+                              (static_cast<size_t>(b) * p.num_q_heads + g * G) * D + quad * 4) = w;
 }
 
+template <int DT, int D, int NT>
+void launch_merge_nt(AttnParams& p, hipStream_t s) {
+    const int quads = p.group * D / 4;   // 16 .. 512
+    const dim3 block(NT);
+    const auto grid = [&](int og) { return dim3(p.batch * p.kv_heads, (quads + og - 1) / og); };
+    if (quads <= 32)
+        hipLaunchKernelGGL((attn_decode_merge<DT, D, NT / 32, NT>), grid(32), block, 0, s, p, p.seg_info);
+    else if (quads <= 64)
+        hipLaunchKernelGGL((attn_decode_merge<DT, D, NT / 64, NT>), grid(64), block, 0, s, p, p.seg_info);
+    else if (quads <= 128)
+        hipLaunchKernelGGL((attn_decode_merge<DT, D, NT / 128, NT>), grid(128), block, 0, s, p, p.seg_info);
+    else
+        hipLaunchKernelGGL((attn_decode_merge<DT, D, NT / 256, NT>), grid(256), block, 0, s, p, p.seg_info);
+}
+
+// Few (b, g) pairs have many parts each: 16-wave workgroups while one per CU
+// holds them all, else 4-wave ones.
 template <int DT, int D>
 void launch_merge(AttnParams& p, hipStream_t s) {
-    const int n_out = p.group * D / 64;
-    const dim3 grid(p.batch * p.kv_heads), block(64);
-    if (n_out <= 1)
-        hipLaunchKernelGGL((attn_decode_merge<DT, D, 1>), grid, block, 0, s, p, p.seg_info);
-    else if (n_out <= 2)
-        hipLaunchKernelGGL((attn_decode_merge<DT, D, 2>), grid, block, 0, s, p, p.seg_info);
-    else if (n_out <= 4)
-        hipLaunchKernelGGL((attn_decode_merge<DT, D, 4>), grid, block, 0, s, p, p.seg_info);
-    else if (n_out <= 8)
-        hipLaunchKernelGGL((attn_decode_merge<DT, D, 8>), grid, block, 0, s, p, p.seg_info);
-    else if (n_out <= 16)
-        hipLaunchKernelGGL((attn_decode_merge<DT, D, 16>), grid, block, 0, s, p, p.seg_info);
-    else
-        hipLaunchKernelGGL((attn_decode_merge<DT, D, 32>), grid, block, 0, s, p, p.seg_info);
+    if (p.batch * p.kv_heads <= 256) launch_merge_nt<DT, D, 1024>(p, s);
+    else launch_merge_nt<DT, D, 256>(p, s);
 }
 
 // Any-shape decode attention (head_dim <= 256, any GQA map, any block size;
@@ -1085,16 +1124,29 @@ int env_int(dev::Tun t, int dflt, int lo, int hi) {
 // KCMM_ATTN_WAVES waves of the streaming kernel (default by page type),
 // KCMM_ATTN_HW waves per workgroup (kv heads read together; the largest
 // divisor of Hkv not above it is used), KCMM_ATTN_MIN_TILES the smallest
-// slice a workgroup takes, KCMM_ATTN_DEPTH tiles in flight (2 or 3; 3 keeps
+// slice a workgroup takes (by length when not set), KCMM_ATTN_DEPTH tiles in flight (2 or 3; 3 keeps
 // at most 4 waves per workgroup).
 int stream_waves(int dtype) {
     return env_int(dev::Tun::kAttnWaves, dtype == kDtFP8 ? 2048 : 1024, 1, 1 << 20);
 }
-// Measured in the full decode step (Llama-3-8B shape, three runs each):
-// 16-bit pages are as fast with one-wave workgroups as with head blocks (the
-// layer step is 1% faster with HW = 1), fp8 pages gain 3% at HW = 8.
-int stream_hw(int dtype) { return env_int(dev::Tun::kAttnHw, dtype == kDtFP8 ? 8 : 1, 1, 8); }
-int stream_min_tiles() { return env_int(dev::Tun::kAttnMinTiles, 8, 1, 1 << 16); }
+// Waves per workgroup by the batch's size (head, tile entries of the list at
+// full tables; call times, 32/8 heads of 128 unless said):
+//  * fp8 pages: 8 above 4096 entries (a row of 1 KiB read together), else 1 --
+//    8-wave workgroups are then too few (one sequence of 1456 tokens 11.1 us
+//    with 1, 14.4 with 8; of 10000 19.8 / 20.8; 16 of 1000 .. 4000 28.9 / 27.7);
+//  * 16-bit pages: 4 above 16384 entries at head_dim 128 with whole groups of 8
+//    kv heads, one workgroup per CU (64 sequences of 512 .. 4096 tokens 99.8 us
+//    with 4, 102.4 with 1; two of 41000 and 50000 69.5 / 73.1; 128 of 500 ..
+//    3000 152 / 160, 16 kv heads; the decode step is as fast), else 1 (16 of
+//    1000 .. 4000 40.0 / 38.5; 64 of 300 .. 1000 40.6 / 39.7; head_dim 64: 64
+//    sequences 56.6 / 53.6).
+int stream_hw(int dtype, int head_dim, int kv_heads, long long entries) {
+    int hw = 1;
+    if (dtype == kDtFP8) hw = entries > 4096 ? 8 : 1;
+    else if (head_dim == 128 && kv_heads % 8 == 0 && entries > 16384) hw = 4;
+    return env_int(dev::Tun::kAttnHw, hw, 1, 8);
+}
+int stream_min_tiles() { return env_int(dev::Tun::kAttnMinTiles, 0, 1, 1 << 16); }
 int stream_depth() { return env_int(dev::Tun::kAttnDepth, 2, 2, 3); }
 
 template <int DT, int D, int BS>
@@ -1108,22 +1160,33 @@ bool launch_stream(AttnParams& p, hipStream_t s, bool no_alloc, std::string* err
     }
     if (p.batch == 0) return true;
     const int depth = stream_depth();
-    int hw = std::min(stream_hw(DT), depth == 3 ? 4 : 8);
+    int hw = std::min(stream_hw(DT, D, p.kv_heads, tmax), depth == 3 ? 4 : 8);
     while (p.kv_heads % hw) --hw;
     p.hw = hw;
     p.min_tiles = stream_min_tiles();
     const long long lists = tmax / p.kv_heads * (p.kv_heads / hw);   // entries of the slice list
-    const long long want = (lists + p.min_tiles - 1) / p.min_tiles;
-    p.total_waves = static_cast<int>(
-        std::max(1LL, std::min<long long>(std::max(1, stream_waves(DT) / hw), want)));
+    const long long most = std::max(1, stream_waves(DT) / hw);
+    // slices for slices of at least `tiles` entries
+    auto slices = [&](long long tiles) {
+        return static_cast<int>(std::max(1LL, std::min(most, (lists + tiles - 1) / tiles)));
+    };
+    p.total_waves = slices(std::max(1, p.min_tiles));
     // slice-indexed units, then kSegPieces per (b, g); G rows of each
-    p.seg_unit0 = static_cast<size_t>(p.total_waves) * hw * 2;
-    const size_t units =
-        (p.seg_unit0 + static_cast<size_t>(p.batch) * p.kv_heads * kSegPieces) * p.group;
+    size_t units = 0, part_bytes = 0;
     // idle-load region first: it must cover one tile's lane addresses
     const size_t idle_bytes = (static_cast<size_t>(8) * p.row_bytes + 1023) & ~static_cast<size_t>(255);
-    const size_t part_bytes = idle_bytes + ((units * (D + 2) * sizeof(float) + 255) & ~size_t(255));
     const size_t info_bytes = static_cast<size_t>(p.batch) * p.kv_heads * sizeof(int2);
+    auto size_parts = [&]() {
+        p.seg_unit0 = static_cast<size_t>(p.total_waves) * hw * 2;
+        units = (p.seg_unit0 + static_cast<size_t>(p.batch) * p.kv_heads * kSegPieces) * p.group;
+        part_bytes = idle_bytes + ((units * (D + 2) * sizeof(float) + 255) & ~size_t(255));
+    };
+    size_parts();
+    if (no_alloc && part_bytes + info_bytes > kNoAllocScratchBytes) {
+        // the static scratch holds more sequences with fewer slices
+        p.total_waves = slices(std::max(8, p.min_tiles));
+        size_parts();
+    }
     void* ws = nullptr;
     void* info = nullptr;
     std::unique_lock<std::mutex> noalloc_lock;

@@ -390,3 +390,53 @@ def test_stream_kernel_timing(gpu_lib):
         assert n0 == 0
     finally:
         case.pool.destroy()
+
+
+@pytest.mark.parametrize("hq,hkv,d,dtype,ctx,min_tiles", [
+    (16, 1, 128, KV_BF16, [5001, 0, 4097, 40], 1),      # 157 parts: two passes over the weights,
+                                                        # 2048 outputs: two workgroups per (b, g)
+    (16, 1, 64, KV_F16, [8300, 33], 1),                 # 260 parts, three passes
+    (1, 1, 64, KV_BF16, [4200], 1),                     # 16 output quads on 1024 threads
+    (6, 2, 128, KV_BF16, [700, 129, 1], 1),             # 96 quads: threads past the last
+    (14, 2, 128, KV_BF16, [161, 96], 1),                # 224 quads, 4..6 parts
+    (32, 8, 128, KV_BF16, [150, 290] * 18, 1),          # 288 (b, g) pairs: 4-wave workgroups
+    (32, 8, 128, KV_FP8, [1456], None), (32, 8, 128, KV_FP8, [1000] * 17, None),   # HW 1 / 8
+    (8, 2, 128, KV_BF16, [1024, 1024], None), (8, 2, 128, KV_BF16, [1024, 1056], None),   # slice 1 / 2
+    (8, 2, 64, KV_BF16, [5120], None), (8, 2, 64, KV_BF16, [5121], None),                 # slice 2 / 4
+    (16, 16, 128, KV_F16, [1025] * 32, None)])          # 16896 entries: four waves per workgroup
+def test_merge_and_slice_rules(gpu_lib, tunables, hq, hkv, d, dtype, ctx, min_tiles):
+    """The log-sum-exp merge over many parts, output widths and workgroup
+    sizes, and both sides of each rule that picks slice length and waves per
+    workgroup, against the oracle."""
+    if min_tiles:
+        tunables.setenv("KCMM_ATTN_MIN_TILES", str(min_tiles))
+    case = build_decode_case(gpu_lib, batch=len(ctx), num_q_heads=hq, kv_heads=hkv, head_dim=d,
+                             block_size=16, ctx_lens=ctx, dtype=dtype, seed=len(ctx) + hq)
+    try:
+        check(case)
+    finally:
+        case.pool.destroy()
+
+
+def test_noalloc_takes_fewer_slices_when_its_scratch_is_short(gpu_lib):
+    """150 short sequences with 16 query heads per kv head: one-tile slices
+    would need more than the static scratch, longer ones fit."""
+    import ctypes as C
+    import torch
+    rng = np.random.default_rng(4)
+    ctx = rng.integers(1, 129, size=150)
+    ctx[0] = 128
+    case = build_decode_case(gpu_lib, batch=150, num_q_heads=32, kv_heads=2, head_dim=128,
+                             block_size=16, ctx_lens=ctx, dtype=KV_BF16, seed=5)
+    try:
+        d = case.dev
+        d["out"].fill_(float("nan"))
+        rc = gpu_lib.lib.kcmm_paged_attn_decode_bf16_noalloc_on_stream(
+            case.pool.handle, 0, d["q"].data_ptr(), d["out"].data_ptr(), d["bt"].data_ptr(),
+            d["sl"].data_ptr(), d["offs"].data_ptr(), 150, 32, 2, 128, 16, case.mbps,
+            C.c_float(1 / math.sqrt(128)), 0)
+        assert rc == 0, case.pool.last_error()
+        torch.cuda.synchronize()
+        assert rel_err(gpu_out(case), oracle_out(case)) <= TOL[KV_BF16]
+    finally:
+        case.pool.destroy()
