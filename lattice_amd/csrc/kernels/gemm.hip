@@ -659,6 +659,25 @@ bool shape_ok(uint32_t m, uint32_t n, uint32_t k, std::string* err) {
     return true;
 }
 
+// Decode-sized products over a long weight matrix (an lm_head) run the wide
+// kernel with one token tile: its direct loads keep 40-70 KiB per CU in flight
+// without registers and its weights are read nontemporal.  At the Llama-3-8B
+// lm_head (128256 x 4096; stream kernel / wide): M = 1 173 / 153 us, 16 177 /
+// 160, 64 199 / 169, 100 240 / 173, 128 253 / 172.  Its tiles are 256 rows,
+// one workgroup per CU, so the matrix must fill at least 1.5 rounds up to M =
+// 64 (65536 rows, one round: 90 / 111 at M = 1, 99 / 116 at 64; 100352 rows 160
+// / 151, 181 / 168), 0.75 above (50304 rows 106 / 92 at M = 100; 32000 x 2048
+// 33 / 37), and up to M = 16 the rows must be long (128256 x 1024 41 / 43;
+// 151936 x 2048 106 / 107).
+bool long_weights(uint32_t m, uint32_t n, uint32_t k) {
+    if (dev::tunable_or(dev::Tun::kGemmTiled, 1) == 0 ||
+        dev::tunable_or(dev::Tun::kGemmSplits, 1) > 1)
+        return false;
+    if (m > 64) return m <= 128 && n >= 192 * 256;
+    return n >= 384 * 256 && (m > 16 || k >= 4096);
+}
+int long_weights_fb(uint32_t m) { return m > 64 ? 2 : 1; }
+
 GemmParams base_params(uint64_t x, uint64_t w, uint32_t m, uint32_t n, uint32_t k) {
     GemmParams p{};
     p.X = reinterpret_cast<const uint16_t*>(x);
@@ -684,10 +703,23 @@ bool gemm_split_reduce_launch(const float* part, uint16_t* y, const uint16_t* r,
 bool gemm_bf16(uint64_t x, uint64_t w, uint64_t y, uint32_t m, uint32_t n, uint32_t k,
                uint64_t stream, std::string* err, uint64_t residual) {
     if (!shape_ok(m, n, k, err)) return false;
-    // many tokens: the LDS-tiled MFMA kernel (KCMM_GEMM_TILED=0 keeps the
+    // many tokens: the LDS-tiled MFMA kernels (KCMM_GEMM_TILED=0 keeps the
     // weight-stream kernel)
     if (m > 128 && dev::tunable_or(dev::Tun::kGemmTiled, 1) != 0)
         return gemm_tiled(x, w, 0, y, m, n, k, stream, residual, err);
+    if (long_weights(m, n, k)) {
+        GemmWideArgs a{};
+        a.x = x;
+        a.w = w;
+        a.y = y;
+        a.residual = residual;
+        a.m = m;
+        a.n = n;
+        a.k = k;
+        a.plan.fb0 = a.plan.fb1 = long_weights_fb(m);
+        a.stream = stream;
+        return gemm_wide(a, err);
+    }
     GemmParams p = base_params(x, w, m, n, k);
     p.Y = reinterpret_cast<uint16_t*>(y);
     p.R = reinterpret_cast<const uint16_t*>(residual);
@@ -710,6 +742,10 @@ bool gemm_plan(uint32_t m, uint32_t n, uint32_t k, bool fp8_weights, GemmPlan* p
     if (m > 128 && dev::tunable_or(dev::Tun::kGemmTiled, 1) != 0) {
         plan->kernel = 1;
         gemm_tiled_plan(m, n, k, fp8_weights, &plan->splits, &plan->tile);
+    } else if (!fp8_weights && long_weights(m, n, k)) {
+        plan->kernel = 1;
+        plan->splits = 1;
+        plan->tile = 100 + long_weights_fb(m);
     } else {
         plan->kernel = 0;
         plan->splits = splits_for(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k),

@@ -50,6 +50,11 @@ __device__ __forceinline__ void load_lds16(const uint8_t* g, uint8_t* lds) {
     __builtin_amdgcn_global_load_lds(g, (lds_ptr)lds, 16, 0, 0);
 }
 
+// The same, nontemporal (weights that one token tile reads once).
+__device__ __forceinline__ void load_lds16_nt(const uint8_t* g, uint8_t* lds) {
+    __builtin_amdgcn_global_load_lds(g, (lds_ptr)lds, 16, 0, 2);
+}
+
 // s_waitcnt vmcnt(N) lgkmcnt(0) (gfx9 encoding: vmcnt bits 3:0 and 15:14,
 // expcnt 6:4, lgkmcnt 11:8).
 template <int N>
@@ -95,7 +100,7 @@ constexpr int kWideSwiglu = 1;
 constexpr int kWideLds = 160 * 1024;
 
 // One tile: 256 weight rows of weight tile tn by BM = 64 * FB tokens from m0.
-template <int EPI, int FB>
+template <int EPI, int FB, bool WNT>
 __device__ __forceinline__ void wide_tile(const WideParams& p, uint8_t* lds, int tn, int m0) {
     constexpr int BM = 64 * FB;
     constexpr int BN = EPI == kWideSwiglu ? 128 : 256;   // output columns
@@ -140,7 +145,10 @@ __device__ __forceinline__ void wide_tile(const WideParams& p, uint8_t* lds, int
         uint8_t* dst = lds + (c & 1) * WT + wave * 1024;
         const uint8_t* src = wk + static_cast<size_t>(c) * 128;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) load_lds16(src + wof[i], dst + i * 8192);
+        for (int i = 0; i < 4; ++i) {
+            if constexpr (WNT) load_lds16_nt(src + wof[i], dst + i * 8192);
+            else load_lds16(src + wof[i], dst + i * 8192);
+        }
     };
     auto issue_x = [&](int c, int slot) {
         uint8_t* dst = lds + 2 * WT + slot * XT + wave * 1024;
@@ -309,7 +317,7 @@ __device__ __forceinline__ int xcd_order(int idx, int n) {
     return x * q + min(x, r) + (idx >> 3);
 }
 
-template <int EPI>
+template <int EPI, bool WNT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_wide_kernel(WideParams p) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[kWideLds];
@@ -340,10 +348,10 @@ void gemm_wide_kernel(WideParams p) {
         i -= n;
     }
     switch (fb) {
-        case 1: wide_tile<EPI, 1>(p, lds, tn, m0); break;
-        case 2: wide_tile<EPI, 2>(p, lds, tn, m0); break;
-        case 3: wide_tile<EPI, 3>(p, lds, tn, m0); break;
-        case 4: wide_tile<EPI, 4>(p, lds, tn, m0); break;
+        case 1: wide_tile<EPI, 1, WNT>(p, lds, tn, m0); break;
+        case 2: wide_tile<EPI, 2, WNT>(p, lds, tn, m0); break;
+        case 3: wide_tile<EPI, 3, WNT>(p, lds, tn, m0); break;
+        case 4: wide_tile<EPI, 4, WNT>(p, lds, tn, m0); break;
         default: break;
     }
 }
@@ -484,10 +492,18 @@ bool gemm_wide(const GemmWideArgs& a, std::string* err) {
         grid += p.nw[z] * (p.full[z] + (p.rag[z] > 0));
     }
     hipStream_t s = reinterpret_cast<hipStream_t>(a.stream);
-    if (a.swiglu)
-        hipLaunchKernelGGL((gemm_wide_kernel<kWideSwiglu>), dim3(grid, 1), dim3(512), 0, s, p);
-    else
-        hipLaunchKernelGGL((gemm_wide_kernel<kWidePlain>), dim3(grid, c.splits), dim3(512), 0, s, p);
+    const dim3 g(grid, c.splits);
+    const bool once = p.M <= 64 * c.fb0 && c.nw1 == 0;   // one token tile
+    auto launch = [&](auto epi, auto nt) {
+        hipLaunchKernelGGL((gemm_wide_kernel<decltype(epi)::value, decltype(nt)::value>), g,
+                           dim3(512), 0, s, p);
+    };
+    using P = std::integral_constant<int, kWidePlain>;
+    using S = std::integral_constant<int, kWideSwiglu>;
+    if (a.swiglu && once) launch(S{}, std::true_type{});
+    else if (a.swiglu) launch(S{}, std::false_type{});
+    else if (once) launch(P{}, std::true_type{});
+    else launch(P{}, std::false_type{});
     KCMM_HIP_CHECK(hipGetLastError(), err);
     return true;
 }

@@ -435,3 +435,37 @@ def test_wide_kernel(gpu_lib, tunables, tile, m, n, k, splits):
         gpu_lib.gemm_bf16_swiglu(x.data_ptr(), w.data_ptr(), act.data_ptr(), m, n, k, s)
         torch.cuda.synchronize()
         assert torch.equal(act.view(torch.int16), ref.view(torch.int16))
+
+
+@pytest.mark.parametrize("m,n,k,wide", [(1, 98304, 4096, True), (16, 98304, 256, False),
+                                        (17, 98304, 256, True), (64, 98240, 512, False),
+                                        (64, 98368, 512, True), (65, 49152, 256, True),
+                                        (65, 49088, 256, False), (128, 49216, 768, True)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_long_weights(gpu_lib, tunables, m, n, k, wide, residual):
+    """Both sides of the rule that gives decode-sized products over long
+    weight matrices to the wide kernel: the same bits as the weight-stream
+    kernel (KCMM_GEMM_TILED=0), each output being one sum in the same k
+    order; the plan names the kernel that runs."""
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + n + k)
+    x = torch.randn((m, k), generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn((n, k), generator=g, device="cuda") * 0.02).to(torch.bfloat16)
+    r = torch.randn((m, n), generator=g, device="cuda").to(torch.bfloat16)
+    s = torch.cuda.current_stream().cuda_stream
+    outs = []
+    for tiled in ("0", "1"):
+        tunables.setenv("KCMM_GEMM_TILED", tiled)
+        y = r.clone() if residual else torch.full_like(r, float("nan"))
+        if residual:
+            gpu_lib.gemm_bf16_add(x.data_ptr(), w.data_ptr(), y.data_ptr(), y.data_ptr(), m, n, k, s)
+        else:
+            gpu_lib.gemm_bf16(x.data_ptr(), w.data_ptr(), y.data_ptr(), m, n, k, s)
+        torch.cuda.synchronize()
+        outs.append(y)
+        plan = gpu_lib.gemm_plan(m, n, k)
+        assert plan["kernel"] == ("tiled" if wide and tiled == "1" else "stream"), plan
+        assert plan["splits"] == 1
+    assert bool(torch.isfinite(outs[1].float()).all())
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
