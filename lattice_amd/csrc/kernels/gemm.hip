@@ -536,9 +536,14 @@ int choose_splits(int N, int K, int kch, int mgroups) {
 
 // Tile shape by M: token blocks per pass (the activation chunk, M x KCH
 // bf16, is 32 KiB).
-// fp8 weights need at least 128-element chunks (one 128-byte weight line).
+// fp8 weights need at least 128-element chunks (one 128-byte weight line);
+// up to 16 tokens they take 512-element ones, as many weight bytes in flight
+// as bf16's 256 (M = 1: 28672 x 4096 26.4 -> 23.6 us, 4096 x 14336 15.7 -> 14.2;
+// bf16 at 512: 43 -> 47; fp8 at 64 tokens was slower with them).
 template <typename F>
-bool by_m(int M, F&& f, bool wf8 = false) {
+bool by_m(int M, int K, F&& f, bool wf8 = false) {
+    if (M <= 16 && wf8 && K % 512 == 0)
+        return f(std::integral_constant<int, 1>{}, std::integral_constant<int, 512>{});
     if (M <= 16) return f(std::integral_constant<int, 1>{}, std::integral_constant<int, 256>{});
     if (M <= 32) return f(std::integral_constant<int, 2>{}, std::integral_constant<int, 256>{});
     if (M <= 64) return f(std::integral_constant<int, 4>{}, std::integral_constant<int, 256>{});
@@ -549,7 +554,7 @@ bool by_m(int M, F&& f, bool wf8 = false) {
 
 int splits_for(int M, int N, int K, bool wf8 = false) {
     int s = 1;
-    by_m(M, [&](auto mb, auto kch) {
+    by_m(M, K, [&](auto mb, auto kch) {
         const int mgroups = (M + 16 * mb.value - 1) / (16 * mb.value);
         s = choose_splits(N, K, kch.value, mgroups);
         return true;
@@ -574,9 +579,12 @@ bool launch_stream(GemmParams p, int splits, bool want_partials, float** part, u
     }
     if (part) *part = p.part;
     p.klen = p.K / splits;
-    return by_m(p.M, [&](auto mb, auto kch) {
+    return by_m(p.M, p.K, [&](auto mb, auto kch) {
         constexpr int MB = decltype(mb)::value, KCH = decltype(kch)::value;
-        if constexpr (WF8 && KCH < 128) {
+        if constexpr (!WF8 && KCH > 256) {
+            *err = "512-element chunks are for fp8 weights";
+            return false;
+        } else if constexpr (WF8 && KCH < 128) {
             *err = "fp8 weights need 128-element chunks";
             return false;
         } else {
