@@ -42,7 +42,7 @@ void reload_tunables();
 // Per-(device, stream, slot, host thread) device scratch; grown on demand
 // (slot 0: decode attention partials, 1: GEMM split partials, 2: decode
 // attention segment table, 3: decode layer-step activations, 4: the final
-// norm's output, 5: unused, 6: tiering staging on
+// norm's output, 5: prefill attention key splits, 6: tiering staging on
 // the null stream, 7: fp8 RoPE/append staging, 8: fp8 page-writer row
 // table).  `zero_fill` buffers start zeroed by a fill kernel, and their
 // users leave them zeroed.  Keyed by host thread as well, so a thread that
@@ -51,6 +51,9 @@ void reload_tunables();
 // graph capture: run each shape once before capturing it.
 bool stream_workspace(uint64_t stream, int slot, size_t bytes, void** out, bool zero_fill,
                       std::string* err);
+// Whether stream_workspace can serve `bytes` now: the buffer is large enough
+// already, or the stream is not being captured (growth allocates).
+bool stream_workspace_ready(uint64_t stream, int slot, size_t bytes);
 // Buffers of exited threads are freed by the next workspace allocation;
 // this frees them now (device synchronize first).  Count of those pending.
 bool release_orphaned_workspaces(std::string* err);

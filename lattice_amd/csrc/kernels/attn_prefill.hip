@@ -32,6 +32,7 @@
 #include <algorithm>
 #include <climits>
 #include <cmath>
+#include <type_traits>
 
 #include "../device_api.hpp"
 #include "common.hpp"
@@ -46,7 +47,19 @@ struct PrefillParams {
     int row_bytes, data_bytes, head_dim, bs_shift;
     float scale_log2;
     float scale;
+    // key splits (SPLIT): per (item, kv head) and split, the 256 columns'
+    // unnormalised outputs [column][D] and (max, denominator) pairs
+    float* part_acc;
+    float* part_ml;
+    int splits;
 };
+
+// Tiles per key split of a workgroup with nt tiles: equal parts, but no part
+// shorter than 8 tiles (a part costs its page-table chain, about 4 tiles).
+constexpr int kSplitTiles = 8;
+__device__ __forceinline__ int split_tiles(int nt, int splits) {
+    return max(kSplitTiles, (nt + splits - 1) / splits);
+}
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -124,11 +137,58 @@ struct Shape {
     static constexpr int BUF = KTILE + KT * VROW;   // one K + V tile of KT keys
 };
 
+// Sequence and token block (TWG tokens) of an item; b < 0: a spare one.
+// Items are dealt longest first: rank r = 0 is every sequence's last token
+// block (the most keys under the causal mask), r = 1 the block before it, and
+// so on; within a rank, sequences in order.  For chunks of equal length this is
+// longest-processing-time order, so the workgroups that start last are the
+// short ones and the rounds end together.
+template <int TWG>
+__device__ __forceinline__ void find_item(int item, int batch, const int32_t* __restrict__ qsl,
+                                          int lane, int& b, int& blk) {
+    b = -1;
+    blk = 0;
+    auto blocks_of = [&](int bb) {   // token blocks of sequence bb (0 past the batch)
+        const int n = bb < batch ? qsl[bb + 1] - qsl[bb] : 0;
+        return n > 0 ? (n + TWG - 1) / TWG : 0;
+    };
+    const int v0 = blocks_of(lane);   // the first 64 sequences stay in registers
+    int base = 0;                      // items of the ranks before r
+    for (int r = 0; b < 0; ++r) {
+        int cnt = 0;
+        for (int c = 0; c < batch; c += 64) {
+            const int v = c == 0 ? v0 : blocks_of(c + lane);
+            cnt += __popcll(__ballot(v > r));
+        }
+        if (cnt == 0) break;          // no item of this rank: a spare workgroup
+        if (item < base + cnt) {
+            int j = item - base;       // the j-th sequence (in order) with more than r blocks
+            for (int c = 0; c < batch; c += 64) {
+                const int v = c == 0 ? v0 : blocks_of(c + lane);
+                unsigned long long m = __ballot(v > r);
+                const int n = __popcll(m);
+                if (j < n) {
+                    for (int k = 0; k < j; ++k) m &= m - 1;
+                    const int bit = __ffsll(static_cast<long long>(m)) - 1;
+                    b = c + bit;
+                    blk = __shfl(v, bit) - 1 - r;
+                    break;
+                }
+                j -= n;
+            }
+            break;
+        }
+        base += cnt;
+    }
+}
+
 // Workgroups over (query-token block, kv head), kv head fastest: blockIdx.x
 // = item * Hkv + g, items in longest-first order (see below).  Workgroups are dealt to the 8 XCDs round-robin, so with
 // 8 kv heads every XCD serves one head and its L2 holds that head's pages
 // (shared prefixes included) for all sequences.
-template <int DT, int D, int G, int NW, int NCB, int KT>
+// With SPLIT, blockIdx.y takes one part of the workgroup's keys; a workgroup
+// with more than one part leaves partial results for attn_prefill_merge.
+template <int DT, int D, int G, int NW, int NCB, int KT, bool SPLIT>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void attn_prefill_mfma(PrefillParams p, const uint8_t* __restrict__ kreg,
                        const uint8_t* __restrict__ vreg, const int32_t* __restrict__ bt,
@@ -161,46 +221,8 @@ void attn_prefill_mfma(PrefillParams p, const uint8_t* __restrict__ kreg,
     const int item = static_cast<int>(blockIdx.x) / p.kv_heads;
 
     // ---- sequence and token block of this workgroup ----
-    // Items are dealt longest first: rank r = 0 is every sequence's last
-    // token block (the most keys under the causal mask), r = 1 the block
-    // before it, and so on; within a rank, sequences in order.  For chunks of
-    // equal length this is longest-processing-time order, so the workgroups
-    // that start last are the short ones and the rounds end together.
-    int b = -1, blk = 0;
-    {
-        auto blocks_of = [&](int bb) {   // token blocks of sequence bb (0 past the batch)
-            const int n = bb < p.batch ? qsl[bb + 1] - qsl[bb] : 0;
-            return n > 0 ? (n + TWG - 1) / TWG : 0;
-        };
-        const int v0 = blocks_of(lane);   // the first 64 sequences stay in registers
-        int base = 0;                      // items of the ranks before r
-        for (int r = 0; b < 0; ++r) {
-            int cnt = 0;
-            for (int c = 0; c < p.batch; c += 64) {
-                const int v = c == 0 ? v0 : blocks_of(c + lane);
-                cnt += __popcll(__ballot(v > r));
-            }
-            if (cnt == 0) break;          // no item of this rank: a spare workgroup
-            if (item < base + cnt) {
-                int j = item - base;       // the j-th sequence (in order) with more than r blocks
-                for (int c = 0; c < p.batch; c += 64) {
-                    const int v = c == 0 ? v0 : blocks_of(c + lane);
-                    unsigned long long m = __ballot(v > r);
-                    const int n = __popcll(m);
-                    if (j < n) {
-                        for (int k = 0; k < j; ++k) m &= m - 1;
-                        const int bit = __ffsll(static_cast<long long>(m)) - 1;
-                        b = c + bit;
-                        blk = __shfl(v, bit) - 1 - r;
-                        break;
-                    }
-                    j -= n;
-                }
-                break;
-            }
-            base += cnt;
-        }
-    }
+    int b, blk;
+    find_item<TWG>(item, p.batch, qsl, lane, b, blk);
     b = __builtin_amdgcn_readfirstlane(b);
     if (b < 0) return;                     // whole workgroup: uniform
     blk = __builtin_amdgcn_readfirstlane(blk);
@@ -212,10 +234,21 @@ void attn_prefill_mfma(PrefillParams p, const uint8_t* __restrict__ kreg,
     // queries before position 0 (more queries than cached tokens) see no key;
     // their rows are written as zeros
     const int nt_wg = (max(0, first_pos + min(tok0_wg + TWG, len)) + KT - 1) / KT;
+    // this workgroup's tiles t_beg .. t_end (all of them without SPLIT)
+    int t_beg = 0, t_end = nt_wg;
+    bool partial = false;
+    if constexpr (SPLIT) {
+        const int per = split_tiles(nt_wg, p.splits);
+        t_beg = blockIdx.y * per;
+        if (t_beg > 0 && t_beg >= nt_wg) return;   // uniform
+        t_end = min(nt_wg, t_beg + per);
+        partial = nt_wg > per;
+    }
     const int tok0 = tok0_wg + wave * TPW;  // this wave's first query (chunk index)
     const bool wave_live = tok0 < len;
     const int tok_last = min(tok0 + TPW, len) - 1;
-    const int nt_w = wave_live ? (max(0, first_pos + tok_last + 1) + KT - 1) / KT : 0;
+    const int nt_w =
+        min(t_end, wave_live ? (max(0, first_pos + tok_last + 1) + KT - 1) / KT : 0);
     const int qmin = first_pos + tok0;     // smallest position among the wave's columns
 
     // ---- columns: query token (clamped into the chunk; extra columns are
@@ -478,18 +511,18 @@ void attn_prefill_mfma(PrefillParams p, const uint8_t* __restrict__ kreg,
         uint64_t pg[NPG];
         int ent[NPG];
 #pragma unroll
-        for (int i = 0; i < NPG; ++i) pg[i] = page_offs(page_entry(0, i));
-        gather(0, pg);
+        for (int i = 0; i < NPG; ++i) pg[i] = page_offs(page_entry(t_beg, i));
+        gather(t_beg, pg);
 #pragma unroll
-        for (int i = 0; i < NPG; ++i) pg[i] = page_offs(page_entry(1, i));
+        for (int i = 0; i < NPG; ++i) pg[i] = page_offs(page_entry(t_beg + 1, i));
 #pragma unroll
-        for (int i = 0; i < NPG; ++i) ent[i] = page_entry(2, i);
+        for (int i = 0; i < NPG; ++i) ent[i] = page_entry(t_beg + 2, i);
         store_tile(0);
-        gather(1, pg);
+        gather(t_beg + 1, pg);
 #pragma unroll
-        for (int i = 0; i < NPG; ++i) pg[i] = page_offs(ent[i]);       // tile 2
+        for (int i = 0; i < NPG; ++i) pg[i] = page_offs(ent[i]);       // tile t_beg + 2
 #pragma unroll
-        for (int i = 0; i < NPG; ++i) ent[i] = page_entry(3, i);        // tile 3
+        for (int i = 0; i < NPG; ++i) ent[i] = page_entry(t_beg + 3, i);   // tile t_beg + 3
         __syncthreads();
         // Gathers past the last tile read clamped (valid) rows and are never
         // consumed; issuing them unconditionally keeps every iteration's
@@ -510,7 +543,7 @@ void attn_prefill_mfma(PrefillParams p, const uint8_t* __restrict__ kreg,
 #pragma unroll
             for (int i = 0; i < NPG; ++i) ent[i] = page_entry(kt + 4, i);
         };
-        for (int kt = 0; kt < nt_wg; kt += 2) {
+        for (int kt = t_beg; kt < t_end; kt += 2) {
             step(kt, 0);
             step(kt + 1, 1);
         }
@@ -518,6 +551,23 @@ void attn_prefill_mfma(PrefillParams p, const uint8_t* __restrict__ kreg,
 
     // ---- store the columns that are real queries ----
     if (!wave_live) return;
+    if constexpr (SPLIT) {
+        if (partial) {
+            const size_t unit = static_cast<size_t>(blockIdx.x) * p.splits + blockIdx.y;
+#pragma unroll
+            for (int cb = 0; cb < NCB; ++cb) {
+                const size_t col = unit * (NW * NCB * 16) + (wave * NCB + cb) * 16 + ln;
+                if (lg == 0) {
+                    p.part_ml[2 * col] = m_run[cb];
+                    p.part_ml[2 * col + 1] = lsum[cb][0];
+                }
+                float* o = p.part_acc + col * D + 4 * lg;
+#pragma unroll
+                for (int db = 0; db < DB; ++db) *reinterpret_cast<f32x4*>(o + 16 * db) = acc[cb][db];
+            }
+            return;
+        }
+    }
 #pragma unroll
     for (int cb = 0; cb < NCB; ++cb) {
         const float lt = lsum[cb][0];
@@ -535,6 +585,68 @@ void attn_prefill_mfma(PrefillParams p, const uint8_t* __restrict__ kreg,
                 *reinterpret_cast<u32x2*>(o + 16 * db) = w;
             }
         }
+    }
+}
+
+// Combines the key splits of (item, kv head) workgroup blockIdx.x for the 32
+// columns of its wave blockIdx.y: weights 2^(max - overall max) per column and
+// split in LDS, then every thread sums four dims of a column at a time.
+constexpr int kMaxSplits = 16;
+template <int DT, int D, int G, int NW, int NCB, int KT>
+__global__ __launch_bounds__(256) void attn_prefill_merge(PrefillParams p,
+                                                          const int32_t* __restrict__ sl,
+                                                          const int32_t* __restrict__ qsl) {
+    constexpr int MDT = DT == kDtFP8 ? kDtBF16 : DT;
+    constexpr int TPB = 16 / G, TPW = NCB * TPB, TWG = NW * TPW, COLS = NCB * 16;
+    __shared__ float s_w[kMaxSplits][COLS];
+    const int tid = threadIdx.x;
+    const int g = static_cast<int>(blockIdx.x) % p.kv_heads;
+    int b, blk;
+    find_item<TWG>(static_cast<int>(blockIdx.x) / p.kv_heads, p.batch, qsl, tid & 63, b, blk);
+    if (b < 0) return;
+    const int q0 = qsl[b], len = qsl[b + 1] - q0;
+    const int L = min(sl[b], p.mbps << p.bs_shift);
+    const int nt = (max(0, L - len + min((blk + 1) * TWG, len)) + KT - 1) / KT;
+    const int per = split_tiles(nt, p.splits);
+    const int tok0 = blk * TWG + static_cast<int>(blockIdx.y) * TPW;
+    if (nt <= per || tok0 >= len) return;   // (uniform: one part, or no query)
+    const int parts = (nt + per - 1) / per;
+    const size_t col0 = static_cast<size_t>(blockIdx.x) * p.splits * (NW * COLS) + blockIdx.y * COLS;
+    auto col_at = [&](int s, int c) { return col0 + static_cast<size_t>(s) * (NW * COLS) + c; };
+    if (tid < COLS) {
+        float top = -INFINITY, l = 0.0f;
+        for (int s = 0; s < parts; ++s) top = fmaxf(top, p.part_ml[2 * col_at(s, tid)]);
+        for (int s = 0; s < parts; ++s) {
+            const float m = p.part_ml[2 * col_at(s, tid)];
+            // a part without a visible key (m = -inf) has weight 0
+            const float w = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - top);
+            s_w[s][tid] = w;
+            l += w * p.part_ml[2 * col_at(s, tid) + 1];
+        }
+        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        for (int s = 0; s < parts; ++s) s_w[s][tid] *= inv;
+    }
+    __syncthreads();
+    for (int i = tid; i < COLS * D / 4; i += 256) {
+        const int c = i / (D / 4), d = (i - c * (D / 4)) * 4;
+        const int t = tok0 + c / 16 * TPB + c % 16 / G;
+        if (t >= len) continue;
+        f32x4 o = f32x4{0, 0, 0, 0};
+        for (int s0 = 0; s0 < parts; s0 += 4) {
+            f32x4 v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                v[e] = *reinterpret_cast<const f32x4*>(p.part_acc + col_at(min(s0 + e, parts - 1), c) * D + d);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (s0 + e < parts) o += s_w[s0 + e][c] * v[e];
+        }
+        u32x2 w;
+        w[0] = pack2<MDT>(o[0], o[1]);
+        w[1] = pack2<MDT>(o[2], o[3]);
+        *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(p.out) +
+                                  ((static_cast<size_t>(q0) + t) * p.num_q_heads + g * G + c % G) * D +
+                                  d) = w;
     }
 }
 
@@ -640,13 +752,51 @@ bool launch_mfma(const dev::AttnPrefillArgs& a, PrefillParams& p, hipStream_t s,
         *err = "prefill: too many query tokens";
         return false;
     }
-    hipLaunchKernelGGL((attn_prefill_mfma<DT, D, G, NW, NCB, KT>), dim3(static_cast<unsigned>(blocks)),
-                       dim3(NW * 64), 0, s, p, reinterpret_cast<const uint8_t*>(a.k_base),
-                       reinterpret_cast<const uint8_t*>(a.v_base),
-                       reinterpret_cast<const int32_t*>(a.block_tables),
-                       reinterpret_cast<const int32_t*>(a.seq_lens),
-                       reinterpret_cast<const int32_t*>(a.query_start_loc),
-                       reinterpret_cast<const uint64_t*>(a.offsets_f16));
+    // Too few token blocks for one workgroup per CU: split the keys.  The
+    // host knows the chunk's tokens and the tables' width, not the lengths:
+    // as many parts as fill the CUs once, each at least 8 tiles of a full
+    // table (the parts of a shorter sequence are longer ones, fewer:
+    // split_tiles).  A merge kernel follows, about 2 us where nothing was
+    // split after all (64 tokens without a prefix in a wide table 10.5 ->
+    // 12.3 us).  32/8 heads of 128, bf16, unsplit / split: 64 tokens behind 500
+    // 25 / 22 us, 2000 68 / 26, 8000 237 / 46; 512 behind 2000 84 / 46; 1000
+    // behind 1000 68 / 54; 4 sequences of up to 120 behind 2000 70 / 40.  More
+    // parts than fill the CUs once lose (512 behind 2000: 4 parts 45 us, 8 57).
+    // A capture that may not allocate runs unsplit.
+    const long long busy = std::max<long long>((a.total_query_tokens + TWG - 1) / TWG, a.batch) *
+                           p.kv_heads;
+    const long long cap_tiles = ((static_cast<long long>(p.mbps) << p.bs_shift) + KT - 1) / KT;
+    int splits = static_cast<int>(std::min<long long>(
+        {256 / std::max(1LL, busy), cap_tiles / kSplitTiles, static_cast<long long>(kMaxSplits)}));
+    const size_t cols = static_cast<size_t>(blocks) * std::max(splits, 1) * NW * NCB * 16;
+    const size_t part_bytes = cols * (D + 2) * sizeof(float);
+    if (splits > 1 && !dev::stream_workspace_ready(a.stream, 5, part_bytes)) splits = 1;
+    const dim3 grid(static_cast<unsigned>(blocks), splits > 1 ? splits : 1);
+    auto run = [&](auto split) {
+        hipLaunchKernelGGL((attn_prefill_mfma<DT, D, G, NW, NCB, KT, decltype(split)::value>), grid,
+                           dim3(NW * 64), 0, s, p, reinterpret_cast<const uint8_t*>(a.k_base),
+                           reinterpret_cast<const uint8_t*>(a.v_base),
+                           reinterpret_cast<const int32_t*>(a.block_tables),
+                           reinterpret_cast<const int32_t*>(a.seq_lens),
+                           reinterpret_cast<const int32_t*>(a.query_start_loc),
+                           reinterpret_cast<const uint64_t*>(a.offsets_f16));
+    };
+    if (splits > 1) {
+        void* ws = nullptr;
+        if (!dev::stream_workspace(a.stream, 5, part_bytes, &ws, false, err))
+            return false;
+        p.splits = splits;
+        p.part_ml = static_cast<float*>(ws);
+        p.part_acc = p.part_ml + 2 * cols;
+        run(std::true_type{});
+        KCMM_HIP_CHECK(hipGetLastError(), err);
+        hipLaunchKernelGGL((attn_prefill_merge<DT, D, G, NW, NCB, KT>),
+                           dim3(static_cast<unsigned>(blocks), NW), dim3(256), 0, s, p,
+                           reinterpret_cast<const int32_t*>(a.seq_lens),
+                           reinterpret_cast<const int32_t*>(a.query_start_loc));
+    } else {
+        run(std::false_type{});
+    }
     KCMM_HIP_CHECK(hipGetLastError(), err);
     return true;
 }

@@ -420,6 +420,11 @@ bool gemm_tiled(uint64_t x, uint64_t w, uint64_t wscale, uint64_t y, uint32_t m,
     if (splits != nullptr) *splits = 1;
     GemmWidePlan wp;
     const bool wide = wscale == 0 && use_wide(c, m, n, k, &wp);
+    // a shape that ran unsplit here before the wide kernel may be captured
+    // without a call before it: no new split then
+    if (wide && wp.splits > 1 && c.splits == 1 &&
+        !stream_workspace_ready(stream, 1, static_cast<size_t>(wp.splits) * m * n * sizeof(float)))
+        wp.splits = 1;
     const int ksplits = wide ? wp.splits : c.splits;
     float* partials = nullptr;
     if (ksplits > 1) {

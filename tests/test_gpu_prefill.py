@@ -259,3 +259,74 @@ def test_running_max_grows_on_most_tiles(gpu_lib):
         assert np.isfinite(got).all() and err <= TOL[KV_BF16]
     finally:
         case.pool.destroy()
+
+
+SPLIT_CTX = [1500, 700, 513, 90, 5, 257, 30]
+SPLIT_LENS = [40, 3, 64, 90, 5, 1, 45]   # the last: more queries than cached tokens
+
+
+@pytest.mark.parametrize("dtype,hq,hkv,d,bs,batch", [
+    (KV_BF16, 32, 8, 128, 16, 7), (KV_F16, 32, 8, 64, 16, 7), (KV_FP8, 16, 8, 128, 32, 7),
+    (KV_BF16, 16, 1, 128, 8, 7), (KV_BF16, 8, 8, 128, 16, 3), (KV_F16, 4, 2, 64, 16, 1)])
+def test_key_splits(gpu_lib, dtype, hq, hkv, d, bs, batch):
+    """Chunks of too few token blocks split their keys over workgroups: full,
+    short and single parts in one call (a 5-token sequence beside one of 1500:
+    47 tiles in parts of 8 or more), one-token chunks, rows before position 0
+    (zeros), every page type and head_dim, groups 1, 2, 4 and 16."""
+    case = build_decode_case(gpu_lib, batch=batch, num_q_heads=hq, kv_heads=hkv, head_dim=d,
+                             block_size=bs, ctx_lens=SPLIT_CTX[:batch], dtype=dtype, seed=hq + d)
+    try:
+        got, ref = run_prefill(case, SPLIT_LENS[:batch], hq, seed=bs + hq)
+        err = rel_err(got, ref)
+        print(f"prefill splits dtype={dtype} G={hq // hkv} D={d} B={batch} err={err:.3e}", flush=True)
+        assert np.isfinite(got).all() and err <= TOL[dtype]
+        if batch == 7:
+            assert not got[sum(SPLIT_LENS[:6]):sum(SPLIT_LENS[:6]) + 15].any()
+    finally:
+        case.pool.destroy()
+
+
+def test_key_splits_under_capture(gpu_lib):
+    """A chunk whose keys would be split, captured on a stream without a call
+    before it: the capture may not allocate, so it runs unsplit; replays equal
+    each other and the oracle, with an eager (split) call between them."""
+    import torch
+    case = build_decode_case(gpu_lib, batch=2, num_q_heads=32, kv_heads=8, head_dim=128,
+                             block_size=16, ctx_lens=[1100, 900], dtype=KV_BF16, seed=3)
+    try:
+        lens = [30, 20]
+        got, ref = run_prefill(case, lens, 32, seed=9)          # eager: split
+        q = encode16(KV_BF16, np.random.default_rng(9).standard_normal((50, 32, 128)).astype(np.float32))
+        qt = torch.from_numpy(q.view(np.int16)).view(torch.bfloat16).cuda()
+        out = torch.empty((50, 32, 128), dtype=torch.bfloat16, device="cuda")
+        qsl = torch.tensor([0, 30, 50], dtype=torch.int32, device="cuda")
+        dv = case.dev
+
+        def run(sp):
+            case.pool.paged_attn_prefill(
+                layer_idx=0, query_ptr=qt.data_ptr(), out_ptr=out.data_ptr(),
+                block_tables_ptr=dv["bt"].data_ptr(), seq_lens_ptr=dv["sl"].data_ptr(),
+                query_start_loc_ptr=qsl.data_ptr(), block_offsets_f16_ptr=dv["offs"].data_ptr(),
+                batch=2, total_query_tokens=50, num_q_heads=32, kv_heads=8, head_dim=128,
+                block_size=16, max_blocks_per_seq=case.mbps, scale=1 / math.sqrt(128),
+                stream_ptr=sp)
+
+        st = torch.cuda.Stream()
+        graph = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=st):
+            run(st.cuda_stream)
+        seen = []
+        for _ in range(3):
+            out.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            seen.append(out.clone())
+            run(torch.cuda.current_stream().cuda_stream)
+            torch.cuda.synchronize()
+        assert all(torch.equal(s, seen[0]) for s in seen)
+        for x in (seen[0], out):
+            assert rel_err(x.float().cpu().numpy().astype(np.float64), ref) <= TOL[KV_BF16]
+        assert rel_err(got, ref) <= TOL[KV_BF16]
+    finally:
+        case.pool.destroy()
