@@ -60,6 +60,8 @@ __device__ __forceinline__ void load_lds16_nt(const uint8_t* g, uint8_t* lds) {
 template <int N>
 __device__ __forceinline__ void wait_vm_lgkm0() {
     static_assert(N >= 0 && N < 64, "vmcnt is 6 bits");
+    asm volatile("" ::: "memory");   // the LDS reads before it stay before it
+    __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4));
 }
 
