@@ -221,7 +221,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmParams& p, f32x4 (&acc)[
 // 8 with CW = 4, or 6 for the QKV / RoPE product; unsplit plain and SwiGLU
 // products NW = 12 with CW = 8, or NW = CW = 8 without helpers; the NW - CW
 // helper waves do all of the activation staging) x up to 16*MB tokens x one
-// K split of `klen`, walked in chunks of KCH:
+// K split of `klen` (the last one may be shorter), walked in chunks of KCH:
 //  * each wave's weight chunk (16 rows x KCH) goes HBM -> registers with
 //    whole-line streaming loads (8 rows x 128 B per instruction) and is put
 //    into MFMA A layout by fix_lines, one line at a time; chunk c+1 is in
@@ -283,7 +283,7 @@ void gemm_bf16_stream(GemmParams p) {
     const int K = p.K;
     const int m_base = blockIdx.z * MROWS;
     const int kbeg = blockIdx.y * p.klen;
-    const int nchunks = p.klen / KCH;
+    const int nchunks = min(p.klen, K - kbeg) / KCH;   // the last split may be shorter
     const uint32_t rowb = static_cast<uint32_t>(K) * (WF8 ? 1 : 2);   // weight row bytes
 
     // the first CW waves stream weight rows; the rest (CW < NW) only stage
@@ -517,7 +517,12 @@ __global__ __launch_bounds__(256) void gemm_split_swiglu(const float* __restrict
 // K splits: the smallest divisor of K/kch giving at least `target` workgroups
 // (KCMM_GEMM_WGS, default 256: fewer, longer splits measured faster than
 // 512-1024 at the Llama-3-8B decode shapes) with each split at least two
-// chunks long; at most 16.
+// chunks long; at most 16. Where the divisors leave more than half of the
+// target empty (K / kch prime, or twice a prime), the last split may be
+// shorter than the others: the smallest count that reaches the target with no
+// split empty (bf16, one token, equal -> uneven splits: 4096 x 11008 at 1 -> 4
+// splits 79 -> 19.6 us, 1024 x 2816 at 1 -> 6 22.3 -> 7.6, 3584 x 18944 at
+// 2 -> 5 38.7 -> 35.3; 64 tokens 99 -> 25.3, 27.6 -> 9.0, 58 -> 49).
 int choose_splits(int N, int K, int kch, int mgroups) {
     const int chunks = K / kch;
     const int forced = dev::tunable_or(dev::Tun::kGemmSplits, 0);
@@ -528,6 +533,14 @@ int choose_splits(int N, int K, int kch, int mgroups) {
     for (int s = 1; s <= std::min(chunks, 16); ++s) {
         if (chunks % s) continue;
         if (chunks / s < 2 && s > 1) break;
+        best = s;
+        if (tiles * s >= target) break;
+    }
+    if (2 * tiles * best >= target) return best;
+    for (int s = best + 1; s <= 16; ++s) {
+        const int per = (chunks + s - 1) / s;
+        if (per < 2) break;
+        if ((s - 1) * per >= chunks) continue;
         best = s;
         if (tiles * s >= target) break;
     }
@@ -578,9 +591,9 @@ bool launch_stream(GemmParams p, int splits, bool want_partials, float** part, u
         p.part = static_cast<float*>(ws);
     }
     if (part) *part = p.part;
-    p.klen = p.K / splits;
     return by_m(p.M, p.K, [&](auto mb, auto kch) {
         constexpr int MB = decltype(mb)::value, KCH = decltype(kch)::value;
+        p.klen = (p.K / KCH + splits - 1) / splits * KCH;
         if constexpr (!WF8 && KCH > 256) {
             *err = "512-element chunks are for fp8 weights";
             return false;

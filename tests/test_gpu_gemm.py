@@ -469,3 +469,53 @@ def test_long_weights(gpu_lib, tunables, m, n, k, wide, residual):
         assert plan["splits"] == 1
     assert bool(torch.isfinite(outs[1].float()).all())
     assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
+@pytest.mark.parametrize("m", [1, 17, 64, 128])
+@pytest.mark.parametrize("n,k,fp8", [(128, 1792, False), (64, 2816, True), (320, 11008, False),
+                                     (64, 5632, True), (1024, 4864, False)])
+def test_uneven_splits(gpu_lib, tunables, m, n, k, fp8):
+    """Where the divisors of the chunk count leave the chip empty, the last K
+    split is shorter than the others: plain products, with and without a
+    residual, against float64, within the fp32 rounding of k products summed
+    in any order plus the bf16 roundings."""
+    import torch
+    plan = gpu_lib.gemm_plan(m, n, k, fp8_weights=fp8)
+    chunk = 128 if m > 64 else 512 if fp8 and m <= 16 and k % 512 == 0 else 256
+    per = -(-(k // chunk) // plan["splits"])
+    assert plan["splits"] > 1 and (plan["splits"] - 1) * per < k // chunk
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + n + k)
+    x = torch.randn((m, k), generator=g, device="cuda").to(torch.bfloat16)
+    r = torch.randn((m, n), generator=g, device="cuda").to(torch.bfloat16)
+    if fp8:
+        w = torch.randint(0, 120, (n, k), generator=g, device="cuda", dtype=torch.uint8)
+        scale = torch.rand(n, generator=g, device="cuda") * 0.01
+        wd = w.cpu().view(torch.float8_e4m3fn).double() * scale.cpu().double()[:, None]
+    else:
+        w = (torch.randn((n, k), generator=g, device="cuda") * 0.02).to(torch.bfloat16)
+        wd = w.cpu().double()
+    ref = x.cpu().double() @ wd.t()
+    mag = x.cpu().double().abs() @ wd.abs().t()
+    st = torch.cuda.current_stream().cuda_stream
+    for residual in (0, 1):
+        y = torch.full((m, n), float("nan"), device="cuda", dtype=torch.bfloat16)
+        want = ref
+        if residual and fp8:
+            continue
+        if residual:
+            gpu_lib.gemm_bf16_add(x.data_ptr(), w.data_ptr(), r.data_ptr(), y.data_ptr(), m, n, k, st)
+            want = ref + r.cpu().double()
+        elif fp8:
+            gpu_lib.gemm_fp8w_bf16(x.data_ptr(), w.data_ptr(), scale.data_ptr(), y.data_ptr(), m, n,
+                                   k, st)
+        else:
+            gpu_lib.gemm_bf16(x.data_ptr(), w.data_ptr(), y.data_ptr(), m, n, k, st)
+        # fp32 sums of k products: at most k roundings of 2^-24 of the magnitude
+        # sum; bf16: 2^-8 of each value rounded (the product, and its sum with
+        # the residual)
+        tol = k * 2.0 ** -24 * mag + 2.0 ** -8 * (want.abs() + residual * ref.abs()) * 1.01
+        worst = float(((y.cpu().double() - want).abs() / tol).max())
+        print(f"uneven {m}x{n}x{k} fp8={fp8} residual={residual} splits={plan['splits']} "
+              f"worst {worst:.3f}", flush=True)
+        assert worst <= 1.0
