@@ -301,7 +301,8 @@ uint32_t kcmm_prefix_cached_blocks(kcmm_pool_t *pool);
  *  accumulation on MFMA.  Replaces the cuBLAS call of ref runtime.rs:17-41
  *  (whose column-major arguments equal this product only at m == 1).
  *  m <= 128 runs the weight-stream MFMA kernel (weights streamed into
- *  registers); m > 128 the LDS-tiled MFMA kernel (same product, fp32
+ *  registers; products of lm_head size run the wide kernel); m > 128 the
+ *  wide or the LDS-tiled MFMA kernel, by the shape (same product, fp32
  *  accumulation, not the same bits; KCMM_GEMM_TILED=0 keeps the
  *  weight-stream kernel).  Enqueue only; requires k % 256 == 0 and
  *  n % 64 == 0. */
@@ -312,8 +313,8 @@ int kcmm_gemm_bf16_on_stream(uint64_t x_ptr, uint64_t w_ptr, uint64_t y_ptr,
 /** How kcmm_gemm_bf16_on_stream (fp8_weights = 0) or
  *  kcmm_gemm_fp8w_bf16_on_stream (fp8_weights = 1) runs a product of this
  *  shape under the current KCMM_GEMM_* settings, written to out[4]: kernel
- *  (0 weight-stream, 1 LDS-tiled), K splits, tiling of the tiled kernel (-1
- *  otherwise), bytes of fp32 split partials written and read back by the
+ *  (0 weight-stream, 1 LDS-tiled or wide), K splits, tiling of the tiled
+ *  kernel (100 and above: the wide kernel; -1 for the weight-stream kernel), bytes of fp32 split partials written and read back by the
  *  reduction (0 without a split).  No reference counterpart (the reference's
  *  cuBLAS call, runtime.rs:17-41, exposes no plan); for sizing workspaces and
  *  for counting a product's HBM bytes.  Host-only, no device work.  0 on
