@@ -523,7 +523,7 @@ __global__ __launch_bounds__(256) void gemm_split_swiglu(const float* __restrict
 // split empty (bf16, one token, equal -> uneven splits: 4096 x 11008 at 1 -> 4
 // splits 79 -> 19.6 us, 1024 x 2816 at 1 -> 6 22.3 -> 7.6, 3584 x 18944 at
 // 2 -> 5 38.7 -> 35.3; 64 tokens 99 -> 25.3, 27.6 -> 9.0, 58 -> 49).
-int choose_splits(int N, int K, int kch, int mgroups) {
+int choose_splits(int N, int K, int kch, int mgroups, bool equal) {
     const int chunks = K / kch;
     const int forced = dev::tunable_or(dev::Tun::kGemmSplits, 0);
     if (forced >= 1 && forced <= 16 && chunks % forced == 0) return forced;
@@ -536,7 +536,7 @@ int choose_splits(int N, int K, int kch, int mgroups) {
         best = s;
         if (tiles * s >= target) break;
     }
-    if (2 * tiles * best >= target) return best;
+    if (equal || 2 * tiles * best >= target) return best;
     for (int s = best + 1; s <= 16; ++s) {
         const int per = (chunks + s - 1) / s;
         if (per < 2) break;
@@ -565,13 +565,26 @@ bool by_m(int M, int K, F&& f, bool wf8 = false) {
     return f(std::integral_constant<int, 16>{}, std::integral_constant<int, 64>{});
 }
 
-int splits_for(int M, int N, int K, bool wf8 = false) {
+int splits_for(int M, int N, int K, bool wf8, bool equal = false) {
     int s = 1;
     by_m(M, K, [&](auto mb, auto kch) {
         const int mgroups = (M + 16 * mb.value - 1) / (16 * mb.value);
-        s = choose_splits(N, K, kch.value, mgroups);
+        s = choose_splits(N, K, kch.value, mgroups, equal);
         return true;
     }, wf8);
+    return s;
+}
+
+// splits_for a launch on `stream`.  Under a capture whose stream never ran
+// the shape, the partials of an uneven split cannot be allocated: equal
+// splits then, which for most such shapes need none.
+int splits_on(uint64_t stream, const GemmParams& p) {
+    const bool wf8 = p.wscale != nullptr;
+    const int s = splits_for(p.M, p.N, p.K, wf8);
+    const int e = splits_for(p.M, p.N, p.K, wf8, true);
+    if (s != e && !dev::stream_workspace_ready(
+                      stream, 1, static_cast<size_t>(s) * p.M * p.N * sizeof(float)))
+        return e;
     return s;
 }
 
@@ -744,7 +757,7 @@ bool gemm_bf16(uint64_t x, uint64_t w, uint64_t y, uint32_t m, uint32_t n, uint3
     GemmParams p = base_params(x, w, m, n, k);
     p.Y = reinterpret_cast<uint16_t*>(y);
     p.R = reinterpret_cast<const uint16_t*>(residual);
-    const int splits = splits_for(p.M, p.N, p.K);
+    const int splits = splits_on(stream, p);
     float* part = nullptr;
     if (!launch_stream<kEpiPlain>(p, splits, false, &part, stream, err)) return false;
     if (splits > 1) {
@@ -794,7 +807,7 @@ bool gemm_fp8w_bf16(uint64_t x, uint64_t w8, uint64_t wscale, uint64_t y, uint32
     p.Y = reinterpret_cast<uint16_t*>(y);
     p.R = reinterpret_cast<const uint16_t*>(residual);
     p.wscale = reinterpret_cast<const float*>(wscale);
-    const int splits = splits_for(p.M, p.N, p.K, true);
+    const int splits = splits_on(stream, p);
     float* part = nullptr;
     if (!launch_stream<kEpiPlain, true>(p, splits, false, &part, stream, err)) return false;
     if (splits > 1) return gemm_split_reduce_launch(part, p.Y, p.R, p.M * p.N, splits, stream, err);
@@ -807,7 +820,7 @@ bool gemm_bf16_partials(uint64_t x, uint64_t w, uint32_t m, uint32_t n, uint32_t
     if (!shape_ok(m, n, k, err)) return false;
     GemmParams p = base_params(x, w, m, n, k);
     p.wscale = reinterpret_cast<const float*>(wscale);
-    *splits = splits_for(p.M, p.N, p.K, wscale != 0);
+    *splits = splits_on(stream, p);
     return launch_weights<kEpiPlain>(p, *splits, true, part, stream, err);
 }
 
@@ -856,7 +869,7 @@ bool gemm_bf16_swiglu(uint64_t x, uint64_t w_gate_up, uint64_t act, uint32_t m, 
     GemmParams p = base_params(x, w_gate_up, m, 2 * inter, k);
     p.Y = reinterpret_cast<uint16_t*>(act);
     p.wscale = reinterpret_cast<const float*>(wscale);
-    const int splits = splits_for(p.M, p.N, p.K, wscale != 0);
+    const int splits = splits_on(stream, p);
     float* part = nullptr;
     if (!launch_weights<kEpiSwiglu>(p, splits, false, &part, stream, err)) return false;
     if (splits > 1) {
@@ -904,7 +917,7 @@ bool gemm_bf16_rope_append(uint64_t x, uint64_t w_qkv, uint32_t m, uint32_t k,
     p.mbps = static_cast<int>(a.mbps);
     p.row_bytes = static_cast<int>(a.row_bytes);
     p.wscale = reinterpret_cast<const float*>(wscale);
-    const int splits = splits_for(p.M, p.N, p.K, wscale != 0);
+    const int splits = splits_on(a.stream, p);
     float* part = nullptr;
     if (!launch_weights<kEpiRope>(p, splits, false, &part, a.stream, err)) return false;
     if (splits > 1) return rope_append_from_partials(a, part, splits, err);

@@ -519,3 +519,49 @@ def test_uneven_splits(gpu_lib, tunables, m, n, k, fp8):
         print(f"uneven {m}x{n}x{k} fp8={fp8} residual={residual} splits={plan['splits']} "
               f"worst {worst:.3f}", flush=True)
         assert worst <= 1.0
+
+
+@pytest.mark.parametrize("fp8", [False, True])
+def test_uneven_splits_under_capture(gpu_lib, fp8):
+    """An unevenly split product captured on a stream that never ran it: the
+    capture may not allocate the partials, so it runs unsplit; its replays
+    equal each other and the eager split call up to fp32 rounding."""
+    import torch
+    m, n, k = 5, 320, 11008
+    assert gpu_lib.gemm_plan(m, n, k, fp8_weights=fp8)["splits"] > 1
+    g = torch.Generator(device="cuda")
+    g.manual_seed(7)
+    x = torch.randn((m, k), generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randint(0, 120, (n, k), generator=g, device="cuda", dtype=torch.uint8) if fp8
+         else (torch.randn((n, k), generator=g, device="cuda") * 0.02).to(torch.bfloat16))
+    scale = torch.full((n,), 1e-3, device="cuda")
+    y = torch.empty((m, n), device="cuda", dtype=torch.bfloat16)
+
+    def run(sp):
+        if fp8:
+            gpu_lib.gemm_fp8w_bf16(x.data_ptr(), w.data_ptr(), scale.data_ptr(), y.data_ptr(), m, n,
+                                   k, sp)
+        else:
+            gpu_lib.gemm_bf16(x.data_ptr(), w.data_ptr(), y.data_ptr(), m, n, k, sp)
+
+    run(torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    eager = y.double()
+    graph = torch.cuda.CUDAGraph()
+    st = torch.cuda.Stream()
+    with torch.cuda.graph(graph, stream=st):
+        run(st.cuda_stream)
+    seen = []
+    for _ in range(3):
+        y.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        seen.append(y.clone())
+        run(torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+    assert all(torch.equal(s, seen[0]) for s in seen)
+    # two fp32 sums of the same k products, each rounded to bf16 (2^-8)
+    wd = w.cpu().view(torch.float8_e4m3fn).double() * 1e-3 if fp8 else w.cpu().double()
+    mag = x.cpu().double().abs() @ wd.abs().t()
+    tol = 2 * k * 2.0 ** -24 * mag + 2 * 2.0 ** -8 * eager.cpu().abs() * 1.01
+    assert float(((seen[0].double() - eager).abs().cpu() / tol).max()) <= 1.0
