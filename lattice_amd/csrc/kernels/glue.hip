@@ -17,8 +17,11 @@
 //    rope_type is served;
 //  * silu_mul: act = bf16(bf16(silu(gate)) * up) over the fused [gate | up]
 //    row (F.silu on a bf16 tensor rounds before the multiply).
+#include <algorithm>
+
 #include "../device_api.hpp"
 #include "common.hpp"
+#include "fp8_page.hpp"
 
 namespace kcmm {
 namespace {
@@ -172,6 +175,59 @@ struct RopeAppendParams {
     int64_t* slots;
 };
 
+// Elements e1..e1+3 and e2..e2+3 of sequence b's qkv row (as bf16 values).
+template <bool FROM_PARTIALS>
+__device__ __forceinline__ void rope_load(const RopeAppendParams& p, int b, int batch, int stride,
+                                          int e1, int e2, float (&x1)[4], float (&x2)[4]) {
+    if constexpr (FROM_PARTIALS) {
+        const size_t MN = static_cast<size_t>(batch) * stride;
+        const float* row = p.part + static_cast<size_t>(b) * stride;
+        const f32x4 s1 = sum_partials(row + e1, MN, p.splits);
+        const f32x4 s2 = sum_partials(row + e2, MN, p.splits);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            x1[j] = bf16_round_f32(s1[j]);
+            x2[j] = bf16_round_f32(s2[j]);
+        }
+    } else {
+        const uint16_t* row = p.qkv + static_cast<size_t>(b) * stride;
+        const u32x2 a = *reinterpret_cast<const u32x2*>(row + e1);
+        const u32x2 c = *reinterpret_cast<const u32x2*>(row + e2);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            x1[2 * j] = __uint_as_float(a[j] << 16);
+            x1[2 * j + 1] = __uint_as_float(a[j] & 0xffff0000u);
+            x2[2 * j] = __uint_as_float(c[j] << 16);
+            x2[2 * j + 1] = __uint_as_float(c[j] & 0xffff0000u);
+        }
+    }
+}
+
+// Rotates (HF rotate_half) the pairs by position `pos`.
+__device__ __forceinline__ void rope_rotate(int pos, const float (&fr)[4], const float (&x1)[4],
+                                            const float (&x2)[4], float (&y1)[4], float (&y2)[4]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        float cs, sn;
+        rope_cos_sin(pos, fr[j], &cs, &sn);
+        y1[j] = rope_first(x1[j], x2[j], cs, sn);
+        y2[j] = rope_second(x1[j], x2[j], cs, sn);
+    }
+}
+
+// Stores the pairs as bf16 elements 4iq..+3 and D/2 + 4iq..+3 of a head row.
+__device__ __forceinline__ void rope_store(uint16_t* dst, int iq, int D, const float (&y1)[4],
+                                           const float (&y2)[4]) {
+    u32x2 o1, o2;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        o1[j] = f32_to_bf16_bits(y1[2 * j]) | (f32_to_bf16_bits(y1[2 * j + 1]) << 16);
+        o2[j] = f32_to_bf16_bits(y2[2 * j]) | (f32_to_bf16_bits(y2[2 * j + 1]) << 16);
+    }
+    *reinterpret_cast<u32x2*>(dst + 4 * iq) = o1;
+    *reinterpret_cast<u32x2*>(dst + D / 2 + 4 * iq) = o2;
+}
+
 // Workgroup (b, y) handles heads [y*hs, (y+1)*hs) of sequence b's qkv row,
 // hs = 256 / (D/8): thread t takes quad iq = t % (D/8) of the D/2 rotation
 // pairs (elements 4iq..4iq+3 and D/2 + 4iq..+3) of head y*hs + t / (D/8).
@@ -201,28 +257,7 @@ __global__ __launch_bounds__(256) void rope_append_rows(RopeAppendParams p) {
     for (int j = 0; j < 4; ++j) fr[j] = p.inv_freq[4 * iq + j];
     // elements e..e+3 of the row (as bf16 values)
     float x1[4], x2[4];
-    if constexpr (FROM_PARTIALS) {
-        const size_t MN = static_cast<size_t>(gridDim.x) * stride;
-        const float* row = p.part + static_cast<size_t>(b) * stride;
-        const f32x4 s1 = sum_partials(row + e1, MN, p.splits);
-        const f32x4 s2 = sum_partials(row + e2, MN, p.splits);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            x1[j] = bf16_round_f32(s1[j]);
-            x2[j] = bf16_round_f32(s2[j]);
-        }
-    } else {
-        const uint16_t* row = p.qkv + static_cast<size_t>(b) * stride;
-        const u32x2 a = *reinterpret_cast<const u32x2*>(row + e1);
-        const u32x2 c = *reinterpret_cast<const u32x2*>(row + e2);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            x1[2 * j] = __uint_as_float(a[j] << 16);
-            x1[2 * j + 1] = __uint_as_float(a[j] & 0xffff0000u);
-            x2[2 * j] = __uint_as_float(c[j] << 16);
-            x2[2 * j + 1] = __uint_as_float(c[j] & 0xffff0000u);
-        }
-    }
+    rope_load<FROM_PARTIALS>(p, b, gridDim.x, stride, e1, e2, x1, x2);
     const int L = p.seq_lens[b];
     const int pos = L - 1;
     const bool has_row = pos >= 0 && pos < p.mbps * p.block_size;   // no token / past the table
@@ -235,13 +270,7 @@ __global__ __launch_bounds__(256) void rope_append_rows(RopeAppendParams p) {
     if (!has_row || !live) return;
     float y1[4], y2[4];
     if (h < p.num_q_heads + p.kv_heads) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            float cs, sn;
-            rope_cos_sin(pos, fr[j], &cs, &sn);
-            y1[j] = rope_first(x1[j], x2[j], cs, sn);
-            y2[j] = rope_second(x1[j], x2[j], cs, sn);
-        }
+        rope_rotate(pos, fr, x1, x2, y1, y2);
     } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -265,14 +294,114 @@ __global__ __launch_bounds__(256) void rope_append_rows(RopeAppendParams p) {
         dst = reinterpret_cast<uint16_t*>((is_k ? p.k_base : p.v_base) + page +
                                           static_cast<uint64_t>(kvh) * D * 2);
     }
-    u32x2 o1, o2;
+    rope_store(dst, iq, D, y1, y2);
+}
+
+// rope_append_rows for fp8 pages with the page write in the same launch.
+// Bound by latency: the chain length -> block id -> offset -> scale, and the
+// launch itself.  Rotation and page writer as two dependent kernels / this
+// one, back to back, 32/8 heads of 128: 1 sequence 9.5 / 7.8 us, 16 10.5 /
+// 8.4, 128 11.3 / 9.3, 256 12.2 / 11.7 (512: 20.2 / 21.9, see launch_rope).
+// Rows staged in LDS instead of the staging buffers: 8.2-8.9 us at 1, the
+// flat loads cost more than the round trip through L2.  Workgroup (b, 0)
+// takes the new token's k and v rows: it finds the call's rows for the
+// same page (a decode step's sequences normally have a page each; the rows
+// of a shared page are one set, written by the page's first sequence, the
+// last row for a slot winning, as in kv_slots_fp8_write), rotates them into
+// the bf16 staging rows and writes the page from there, one wave per (kv
+// head, K|V).  Workgroups (b, 1 + y) rotate q heads [y*hs, (y+1)*hs).
+// blockDim.x = 64 * waves; dynamic LDS block_size * 4.
+template <bool FROM_PARTIALS>
+__global__ __launch_bounds__(64 * kFp8MaxWaves) void rope_append_fp8(RopeAppendParams p, uint32_t n_ids,
+                                                                     uint32_t data_bytes) {
+    extern __shared__ int32_t row_of[];   // [block_size]
+    __shared__ int32_t s_first, s_rows;
+    const int b = blockIdx.x, batch = gridDim.x, nt = blockDim.x, t = threadIdx.x;
+    const int D = p.head_dim, quads = D / 8, hs = nt / quads;
+    const int iq = t % quads, hl = t / quads;
+    const int Hq = p.num_q_heads, Hkv = p.kv_heads, stride = (Hq + 2 * Hkv) * D;
+    float fr[4], x1[4], x2[4];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        o1[j] = f32_to_bf16_bits(y1[2 * j]) | (f32_to_bf16_bits(y1[2 * j + 1]) << 16);
-        o2[j] = f32_to_bf16_bits(y2[2 * j]) | (f32_to_bf16_bits(y2[2 * j + 1]) << 16);
+    for (int j = 0; j < 4; ++j) fr[j] = p.inv_freq[4 * iq + j];
+    const int h_begin = blockIdx.y == 0 ? Hq : (blockIdx.y - 1) * hs;
+    const int h_end = blockIdx.y == 0 ? Hq + 2 * Hkv : min(Hq, h_begin + hs);
+    const int h0 = hl < hs && h_begin + hl < h_end ? h_begin + hl : -1;
+    {
+        const int e = max(h0, 0) * D + 4 * iq;
+        rope_load<FROM_PARTIALS>(p, b, batch, stride, e, e + D / 2, x1, x2);
     }
-    *reinterpret_cast<u32x2*>(dst + 4 * iq) = o1;
-    *reinterpret_cast<u32x2*>(dst + D / 2 + 4 * iq) = o2;
+    // position, block id and slot of sequence r's new token; id -1: none
+    auto find = [&](int r, int* id, int* slot) {
+        const int pos = p.seq_lens[r] - 1;
+        const bool has = pos >= 0 && pos < p.mbps * p.block_size;
+        const int lb = has ? pos / p.block_size : 0;
+        int32_t e = -1;
+        if (has) e = p.block_tables[static_cast<size_t>(r) * p.mbps + lb];
+        *id = e >= 0 && static_cast<uint32_t>(e) < n_ids ? e : -1;
+        *slot = has ? pos - lb * p.block_size : 0;
+        return has ? pos : -1;
+    };
+    int id, slot;
+    const int pos = find(b, &id, &slot);
+    float y1[4], y2[4];
+    if (blockIdx.y != 0) {
+        if (pos < 0 || h0 < 0) return;
+        rope_rotate(pos, fr, x1, x2, y1, y2);
+        rope_store(p.q_out + (static_cast<size_t>(b) * Hq + h0) * D, iq, D, y1, y2);
+        return;
+    }
+    if (id < 0) return;   // (uniform)
+    const uint64_t page = p.offsets_f16[id] * 2ull;
+    for (int i = t; i < p.block_size; i += nt) row_of[i] = i == slot ? b : -1;
+    if (t == 0) {
+        s_first = b;
+        s_rows = 1;
+    }
+    __syncthreads();
+    for (int r = t; r < batch; r += nt) {
+        if (r == b) continue;
+        int rid, rslot;
+        find(r, &rid, &rslot);
+        if (rid != id) continue;
+        atomicMin(&s_first, r);
+        atomicAdd(&s_rows, 1);
+        atomicMax(row_of + rslot, r);
+    }
+    __syncthreads();
+    if (s_first != b) return;   // (uniform) an earlier sequence writes this page
+    const int rows = s_rows;
+    // rotates row r's k and v heads into its staging rows
+    auto stage = [&](int r, int at) {
+        for (int h = h0; h >= 0 && h < h_end; h += hs) {
+            const int kvh = h < Hq + Hkv ? h - Hq : h - Hq - Hkv;
+            if (r != b || h != h0) {
+                const int e = h * D + 4 * iq;
+                rope_load<FROM_PARTIALS>(p, r, batch, stride, e, e + D / 2, x1, x2);
+            }
+            uint16_t* dst = (h < Hq + Hkv ? p.k_stage : p.v_stage) +
+                            (static_cast<size_t>(r) * Hkv + kvh) * D;
+            if (h < Hq + Hkv) {
+                rope_rotate(at, fr, x1, x2, y1, y2);
+                rope_store(dst, iq, D, y1, y2);
+            } else {
+                rope_store(dst, iq, D, x1, x2);
+            }
+        }
+    };
+    stage(b, pos);
+    if (rows > 1) {
+        for (int r = b + 1; r < batch; ++r) {
+            int rid, rslot;
+            const int at = find(r, &rid, &rslot);
+            if (rid == id && row_of[rslot] == r) stage(r, at);
+        }
+    }
+    __syncthreads();
+    for (int w = t >> 6; w < 2 * Hkv; w += nt >> 6) {
+        const bool is_v = w & 1;
+        fp8_write_page_head((is_v ? p.v_base : p.k_base) + page, w >> 1, is_v ? p.v_stage : p.k_stage,
+                            row_of, p.block_size, Hkv, D, p.row_bytes, data_bytes);
+    }
 }
 
 // act[m][j] = bf16(bf16(silu(gu[m][j])) * gu[m][I + j]); 8 elements per thread.
@@ -395,6 +524,24 @@ bool launch_rope(const RopeAppendArgs& a, const float* part, int splits, std::st
         p.k_stage = reinterpret_cast<uint16_t*>(stage);
         p.v_stage = reinterpret_cast<uint16_t*>(stage + rows_bytes);
         p.slots = reinterpret_cast<int64_t*>(stage + 2 * rows_bytes);
+    }
+    // up to one sequence per CU in one launch (figures at rope_append_fp8);
+    // more sequences, or what the page writer refuses, as rotation and page
+    // writer
+    if (fp8 && a.batch <= 256 && a.head_dim <= 256 && a.block_size != 0 &&
+        a.block_size <= kFp8MaxBlockSize && a.n_ids <= (1u << 28)) {
+        const uint32_t nt = 64 * std::min<uint32_t>(2 * a.kv_heads, kFp8MaxWaves);
+        const uint32_t heads = nt / (a.head_dim / 8);
+        const dim3 grid(a.batch, 1 + (a.num_q_heads + heads - 1) / heads);
+        const size_t lds = static_cast<size_t>(a.block_size) * 4;
+        if (part != nullptr)
+            hipLaunchKernelGGL(rope_append_fp8<true>, grid, dim3(nt), lds,
+                               reinterpret_cast<hipStream_t>(a.stream), p, a.n_ids, a.data_bytes);
+        else
+            hipLaunchKernelGGL(rope_append_fp8<false>, grid, dim3(nt), lds,
+                               reinterpret_cast<hipStream_t>(a.stream), p, a.n_ids, a.data_bytes);
+        KCMM_HIP_CHECK(hipGetLastError(), err);
+        return true;
     }
     const uint32_t hs = 256 / (a.head_dim / 8);
     const dim3 grid(a.batch, (a.num_q_heads + 2 * a.kv_heads + hs - 1) / hs);

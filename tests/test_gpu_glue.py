@@ -213,6 +213,52 @@ def test_rope_append_fp8_pool(gpu_lib, hq, hkv, d):
     assert np.array_equal(f8["v"], vref)
 
 
+@pytest.mark.parametrize("hq,hkv,d,pages", [(32, 8, 128, 600), (8, 2, 64, 40), (24, 12, 72, 300),
+                                            (2, 1, 256, 500)])
+def test_rope_append_fp8_one_launch(gpu_lib, hq, hkv, d, pages):
+    """Rotation and fp8 page write in one launch (up to 256 sequences) give
+    the bytes of the two-launch path (257 sequences here, the last without a
+    token): sequences that share pages and slots, first and later slots of a
+    page, no token, a token past the table, and table entries that are
+    negative or past the issued ids."""
+    import torch
+    n = 256
+    rng = np.random.default_rng(pages + d)
+    case = build_decode_case(gpu_lib, batch=4, num_q_heads=hq, kv_heads=hkv, head_dim=d,
+                             block_size=16, ctx_lens=[pages * 4] * 4, dtype=KV_FP8, seed=d)
+    try:
+        ids = np.unique(case.block_tables[case.block_tables >= 0])[:pages]
+        table = rng.choice(ids, size=(n + 1, 1)).astype(np.int32)
+        lens = rng.integers(0, 18, n + 1).astype(np.int32)      # 0: none, 17: past the table
+        table[rng.choice(n, 9, replace=False)] = -1
+        table[rng.choice(n, 9, replace=False)] = 1 << 28
+        lens[n] = 0
+        bt, sl = torch.from_numpy(table).cuda(), torch.from_numpy(lens).cuda()
+        x = rng.standard_normal((n + 1, (hq + 2 * hkv) * d)) * np.exp(rng.normal(0, 2, (n + 1, 1)))
+        qkv = bf16_dev(torch, O.encode(O.BF16, x))
+        inv = torch.from_numpy(O.default_inv_freq(500000.0, d).astype(np.float32)).cuda()
+        start = {w: _region(case, w) for w in "kv"}
+        got = []
+        for batch in (n, n + 1, 1):
+            memcpy_htod(case.pool.va_k(0), start["k"])
+            memcpy_htod(case.pool.va_v(0), start["v"])
+            qo = torch.zeros((n + 1, hq, d), dtype=torch.bfloat16, device="cuda")
+            case.pool.rope_append(layer_idx=0, qkv_ptr=qkv.data_ptr(), q_out_ptr=qo.data_ptr(),
+                                  block_tables_ptr=bt.data_ptr(), seq_lens_ptr=sl.data_ptr(),
+                                  block_offsets_f16_ptr=case.dev["offs"].data_ptr(),
+                                  inv_freq_ptr=inv.data_ptr(), batch=batch, num_q_heads=hq,
+                                  max_blocks_per_seq=1,
+                                  stream_ptr=torch.cuda.current_stream().cuda_stream)
+            torch.cuda.synchronize()
+            got.append((bits_of(qo), _region(case, "k"), _region(case, "v")))
+        for a, b in zip(got[0], got[1]):
+            assert np.array_equal(a, b)
+        assert not np.array_equal(got[0][1], start["k"])
+        assert np.array_equal(got[2][0][0], got[0][0][0])
+    finally:
+        case.pool.destroy()
+
+
 def _layer_weights(torch, rng, h, inter, hq, hkv, d):
     enc = lambda shape, std: O.encode(O.BF16, rng.standard_normal(shape) * std)
     w = {"attn_norm": O.encode(O.BF16, 1.0 + 0.1 * rng.standard_normal(h)),
