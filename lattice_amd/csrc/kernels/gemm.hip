@@ -517,32 +517,38 @@ __global__ __launch_bounds__(256) void gemm_split_swiglu(const float* __restrict
 // K splits: the smallest divisor of K/kch giving at least `target` workgroups
 // (KCMM_GEMM_WGS, default 256: fewer, longer splits measured faster than
 // 512-1024 at the Llama-3-8B decode shapes) with each split at least two
-// chunks long; at most 16. Where the divisors leave more than half of the
+// chunks long; at most 16.  A split that gives 7/8 of the target is taken
+// too: one round with a few idle CUs beats a second round (one token, bf16,
+// more -> fewer splits: 5120 x 3072 at 4 -> 3 10.9 -> 9.7 us, 7680 x 2560 at
+// 5 -> 2 13.9 -> 10.6, 5120 x 13824 at 6 -> 3 25.2 -> 25.6; 64 tokens 17.1 ->
+// 13.1, 20.0 -> 14.8, 38.4 -> 34.2).  Not unsplit: 15360 x 5120 40.6 us
+// unsplit, 27.4 at 2.  Where the divisors leave more than a quarter of the
 // target empty (K / kch prime, or twice a prime), the last split may be
-// shorter than the others: the smallest count that reaches the target with no
-// split empty (bf16, one token, equal -> uneven splits: 4096 x 11008 at 1 -> 4
+// shorter than the others: the smallest count that is enough with no split
+// empty (one token, bf16, equal -> uneven splits: 4096 x 11008 at 1 -> 4
 // splits 79 -> 19.6 us, 1024 x 2816 at 1 -> 6 22.3 -> 7.6, 3584 x 18944 at
-// 2 -> 5 38.7 -> 35.3; 64 tokens 99 -> 25.3, 27.6 -> 9.0, 58 -> 49).
+// 2 -> 4 38.7 -> 25.2; 64 tokens 99 -> 25.3, 27.6 -> 9.0, 58 -> 35).
 int choose_splits(int N, int K, int kch, int mgroups, bool equal) {
     const int chunks = K / kch;
     const int forced = dev::tunable_or(dev::Tun::kGemmSplits, 0);
     if (forced >= 1 && forced <= 16 && chunks % forced == 0) return forced;
     const int target = dev::tunable_or(dev::Tun::kGemmWgs, 256);
     const int tiles = (N / 64) * mgroups;
+    auto enough = [&](int s) { return tiles * s >= target || (s > 1 && 8 * tiles * s >= 7 * target); };
     int best = 1;
     for (int s = 1; s <= std::min(chunks, 16); ++s) {
         if (chunks % s) continue;
         if (chunks / s < 2 && s > 1) break;
         best = s;
-        if (tiles * s >= target) break;
+        if (enough(s)) break;
     }
-    if (equal || 2 * tiles * best >= target) return best;
+    if (equal || 4 * tiles * best >= 3 * target) return best;
     for (int s = best + 1; s <= 16; ++s) {
         const int per = (chunks + s - 1) / s;
         if (per < 2) break;
         if ((s - 1) * per >= chunks) continue;
         best = s;
-        if (tiles * s >= target) break;
+        if (enough(s)) break;
     }
     return best;
 }

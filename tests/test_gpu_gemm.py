@@ -473,7 +473,8 @@ def test_long_weights(gpu_lib, tunables, m, n, k, wide, residual):
 
 @pytest.mark.parametrize("m", [1, 17, 64, 128])
 @pytest.mark.parametrize("n,k,fp8", [(128, 1792, False), (64, 2816, True), (320, 11008, False),
-                                     (64, 5632, True), (1024, 4864, False)])
+                                     (64, 5632, True), (1024, 4864, False),
+                                     (5120, 3072, False), (8192, 2816, True)])
 def test_uneven_splits(gpu_lib, tunables, m, n, k, fp8):
     """Where the divisors of the chunk count leave the chip empty, the last K
     split is shorter than the others: plain products, with and without a
