@@ -75,9 +75,11 @@ __device__ __forceinline__ u32x2 fp8_encode8(const u32x4& x, float scale, float 
 // head_dim % 8 == 0 and 16-byte aligned source rows, lanes take 16-byte
 // pieces of the rows, 256 pieces (16 rows of 128) per pass with every load
 // in flight at once; a page of at most 256 pieces is read once.
-__device__ __forceinline__ void fp8_write_page_head(uint8_t* page, uint32_t kvh, const uint16_t* src_base,
-                                    const int32_t* row_of, uint32_t bs, uint32_t kv_heads,
-                                    uint32_t head_dim, uint32_t row_bytes, uint32_t data_bytes) {
+__device__ __forceinline__ void fp8_write_page_head(uint8_t* page, uint32_t kvh,
+                                                    const uint16_t* src_base, const int32_t* row_of,
+                                                    uint32_t bs, uint32_t kv_heads,
+                                                    uint32_t head_dim, uint32_t row_bytes,
+                                                    uint32_t data_bytes) {
     const int lane = threadIdx.x & 63;
     float* sp = reinterpret_cast<float*>(page + data_bytes) + kvh;
     const float old = *sp;
@@ -180,7 +182,7 @@ __device__ __forceinline__ void fp8_write_page_head(uint8_t* page, uint32_t kvh,
                 }
             } else {
 #pragma unroll 1
-        for (uint32_t u = 0; u < bs; ++u) {
+                for (uint32_t u = 0; u < bs; ++u) {
                     if (row_of[u] >= 0) continue;
                     uint8_t* row = page + static_cast<uint64_t>(u) * row_bytes + kvh * head_dim;
 #pragma unroll 1
