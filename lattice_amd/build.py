@@ -6,7 +6,9 @@
 libkcmm.so: the C++ host runtime (pool_core.cpp, tiering.cpp, ffi.cpp; g++) plus the HIP
 kernels (kernels/*.hip; hipcc --offload-arch=gfx950), linked with hipcc.
 libkcmm_hostcheck.so: the same host runtime over a host-memory page backing
-(tests/hostcheck), so CPU tests exercise the product's bookkeeping code.
+(csrc/hostcheck), so CPU tests exercise the product's bookkeeping code.  Its
+sources are the package's own: a runtime that needs another device function
+changes its stand-in with it, whichever tests lie beside it.
 Objects go to lattice_amd/_build/; the libraries are written in-tree.
 """
 from __future__ import annotations
@@ -40,6 +42,7 @@ HIP_FLAGS = [
 CXX_FLAGS = ["-O2", "-fPIC", "-std=c++17", "-Wall", "-Wextra", "-Wno-unused-parameter"]
 
 HOST_SOURCES = ["pool_core.cpp", "tiering.cpp", "ffi.cpp", "tunables.cpp"]
+HOSTCHECK_SOURCES = [*HOST_SOURCES, "hostcheck/host_device.cpp"]
 HIP_SOURCES = ["kernels/backing.hip", "kernels/attn_decode.hip", "kernels/attn_prefill.hip",
                "kernels/kv_write.hip",
                "kernels/page_copy.hip", "kernels/gemm.hip", "kernels/gemm_tiled.hip",
@@ -86,8 +89,8 @@ def build_kcmm(jobs: int = 8) -> Path:
 
 def build_hostcheck() -> Path:
     """Host-only build of the pool runtime for the CPU test tier."""
-    (BUILD / "hostcheck").mkdir(parents=True, exist_ok=True)
-    srcs = [CSRC / s for s in HOST_SOURCES] + [HOSTCHECK_DIR / "host_device.cpp"]
+    HOSTCHECK_DIR.mkdir(parents=True, exist_ok=True)
+    srcs = [CSRC / s for s in HOSTCHECK_SOURCES]
     tmp = HOSTCHECK_LIB.with_suffix(".so.tmp")
     _run([CXX, *CXX_FLAGS, "-shared", "-o", str(tmp), *map(str, srcs), "-Wl,--no-undefined"])
     os.replace(tmp, HOSTCHECK_LIB)
@@ -95,8 +98,8 @@ def build_hostcheck() -> Path:
 
 
 def build_all(jobs: int = 8) -> None:
+    build_kcmm(jobs)      # the product first: it needs nothing of the check build
     build_hostcheck()
-    build_kcmm(jobs)
 
 
 def main() -> None:

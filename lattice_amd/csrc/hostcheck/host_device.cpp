@@ -16,8 +16,8 @@
 #include <string>
 #include <vector>
 
-#include "../../lattice_amd/csrc/device_api.hpp"
-#include "../../lattice_amd/csrc/vmm_backing.hpp"
+#include "../device_api.hpp"
+#include "../vmm_backing.hpp"
 
 namespace kcmm {
 namespace {
