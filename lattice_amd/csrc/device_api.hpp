@@ -51,9 +51,12 @@ void reload_tunables();
 // graph capture: run each shape once before capturing it.
 bool stream_workspace(uint64_t stream, int slot, size_t bytes, void** out, bool zero_fill,
                       std::string* err);
-// Whether stream_workspace can serve `bytes` now: the buffer is large enough
-// already, or the stream is not being captured (growth allocates).
-bool stream_workspace_ready(uint64_t stream, int slot, size_t bytes);
+// Whether a call that can also run without scratch may take `bytes` of it.
+// Not under a capture: the graph would keep the address of a buffer that a
+// later growth, or the thread's exit, frees, and two graphs replayed on two
+// streams would share it.  (`in_capture`: the call's other variant needs the
+// scratch too; under a capture it may then use a buffer that is large enough.)
+bool stream_scratch(uint64_t stream, int slot, size_t bytes, bool in_capture = false);
 // Buffers of exited threads are freed by the next workspace allocation;
 // this frees them now (device synchronize first).  Count of those pending.
 bool release_orphaned_workspaces(std::string* err);
@@ -181,7 +184,7 @@ struct GemmWideArgs {
     GemmWidePlan plan;
     uint64_t stream;
 };
-GemmWidePlan gemm_wide_plan(uint32_t m, uint32_t n, uint32_t k, bool swiglu);
+GemmWidePlan gemm_wide_plan(uint32_t m, uint32_t n, uint32_t k, bool swiglu, int max_splits = 8);
 bool gemm_wide(const GemmWideArgs& a, std::string* err);
 
 // How a plain product of this shape runs (under the current KCMM_GEMM_*

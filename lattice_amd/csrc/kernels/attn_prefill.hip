@@ -762,7 +762,7 @@ bool launch_mfma(const dev::AttnPrefillArgs& a, PrefillParams& p, hipStream_t s,
     // 25 / 22 us, 2000 68 / 26, 8000 237 / 46; 512 behind 2000 84 / 46; 1000
     // behind 1000 68 / 54; 4 sequences of up to 120 behind 2000 70 / 40.  More
     // parts than fill the CUs once lose (512 behind 2000: 4 parts 45 us, 8 57).
-    // A capture that may not allocate runs unsplit.
+    // A capture runs unsplit, and its graph holds no workspace.
     const long long busy = std::max<long long>((a.total_query_tokens + TWG - 1) / TWG, a.batch) *
                            p.kv_heads;
     const long long cap_tiles = ((static_cast<long long>(p.mbps) << p.bs_shift) + KT - 1) / KT;
@@ -770,7 +770,7 @@ bool launch_mfma(const dev::AttnPrefillArgs& a, PrefillParams& p, hipStream_t s,
         {256 / std::max(1LL, busy), cap_tiles / kSplitTiles, static_cast<long long>(kMaxSplits)}));
     const size_t cols = static_cast<size_t>(blocks) * std::max(splits, 1) * NW * NCB * 16;
     const size_t part_bytes = cols * (D + 2) * sizeof(float);
-    if (splits > 1 && !dev::stream_workspace_ready(a.stream, 5, part_bytes)) splits = 1;
+    if (splits > 1 && !dev::stream_scratch(a.stream, 5, part_bytes)) splits = 1;
     const dim3 grid(static_cast<unsigned>(blocks), splits > 1 ? splits : 1);
     auto run = [&](auto split) {
         hipLaunchKernelGGL((attn_prefill_mfma<DT, D, G, NW, NCB, KT, decltype(split)::value>), grid,

@@ -234,19 +234,18 @@ bool stream_workspace(uint64_t stream, int slot, size_t bytes, void** out, bool 
     return true;
 }
 
-bool stream_workspace_ready(uint64_t stream, int slot, size_t bytes) {
-    int dev = 0;
-    if (hipGetDevice(&dev) == hipSuccess) {
-        std::lock_guard<std::mutex> lk(ws_mutex());
-        const auto it = ws_table().find(std::make_tuple(dev, stream, slot, std::this_thread::get_id()));
-        if (it != ws_table().end() && it->second.bytes >= bytes) return true;
-    }
+bool stream_scratch(uint64_t stream, int slot, size_t bytes, bool in_capture) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(reinterpret_cast<hipStream_t>(stream), &cs) != hipSuccess) {
         (void)hipGetLastError();   // (the null stream while another one is captured)
         return false;
     }
-    return cs == hipStreamCaptureStatusNone;
+    if (cs == hipStreamCaptureStatusNone) return true;
+    int dev = 0;
+    if (!in_capture || hipGetDevice(&dev) != hipSuccess) return false;
+    std::lock_guard<std::mutex> lk(ws_mutex());
+    const auto it = ws_table().find(std::make_tuple(dev, stream, slot, std::this_thread::get_id()));
+    return it != ws_table().end() && it->second.bytes >= bytes;
 }
 
 bool release_orphaned_workspaces(std::string* err) {

@@ -581,17 +581,15 @@ int splits_for(int M, int N, int K, bool wf8, bool equal = false) {
     return s;
 }
 
-// splits_for a launch on `stream`.  Under a capture whose stream never ran
-// the shape, the partials of an uneven split cannot be allocated: equal
-// splits then, which for most such shapes need none.
+// splits_for a launch on `stream`.  A capture takes equal splits, which for
+// most of the unevenly split shapes need no partials: no graph then holds the
+// address of a buffer that only the uneven split asked for.
 int splits_on(uint64_t stream, const GemmParams& p) {
     const bool wf8 = p.wscale != nullptr;
     const int s = splits_for(p.M, p.N, p.K, wf8);
     const int e = splits_for(p.M, p.N, p.K, wf8, true);
-    if (s != e && !dev::stream_workspace_ready(
-                      stream, 1, static_cast<size_t>(s) * p.M * p.N * sizeof(float)))
-        return e;
-    return s;
+    const size_t bytes = static_cast<size_t>(s) * p.M * p.N * sizeof(float);
+    return s == e || dev::stream_scratch(stream, 1, bytes) ? s : e;
 }
 
 // Launch the streaming kernel with `splits` K splits; splits > 1 or

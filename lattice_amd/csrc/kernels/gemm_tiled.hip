@@ -387,10 +387,11 @@ double tiled_us(const TiledConfig& c, double M, double N, double K) {
 // least 8% below this kernel's (both models are off by 4-8%, so closer ones
 // stay here: over the same 180 products every choice but three is within 2%
 // of the faster kernel).  A forced tile (KCMM_GEMM_TILE 0..10) stays here.
-bool use_wide(const TiledConfig& c, uint32_t m, uint32_t n, uint32_t k, dev::GemmWidePlan* plan) {
+bool use_wide(const TiledConfig& c, uint32_t m, uint32_t n, uint32_t k, dev::GemmWidePlan* plan,
+              int max_splits = 8) {
     const int forced = dev::tunable_or(dev::Tun::kGemmTile, -1);
     if (forced >= 0 && forced < kCfgs) return false;
-    *plan = dev::gemm_wide_plan(m, n, k, false);
+    *plan = dev::gemm_wide_plan(m, n, k, false, max_splits);
     if (plan->splits == 0) return false;
     if (forced > 100) return true;
     // (tiles of configurations other than 0, 9, 10 are N % 128 != 0 shapes)
@@ -419,12 +420,13 @@ bool gemm_tiled(uint64_t x, uint64_t w, uint64_t wscale, uint64_t y, uint32_t m,
     const TiledConfig c = choose(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k));
     if (splits != nullptr) *splits = 1;
     GemmWidePlan wp;
-    const bool wide = wscale == 0 && use_wide(c, m, n, k, &wp);
-    // a shape that ran unsplit here before the wide kernel may be captured
-    // without a call before it: no new split then
+    bool wide = wscale == 0 && use_wide(c, m, n, k, &wp);
+    // A shape that this kernel runs unsplit can be captured without a call
+    // before it, and its graph outlives any workspace: the wide kernel takes it
+    // unsplit, or not at all, under a capture.
     if (wide && wp.splits > 1 && c.splits == 1 &&
-        !stream_workspace_ready(stream, 1, static_cast<size_t>(wp.splits) * m * n * sizeof(float)))
-        wp.splits = 1;
+        !stream_scratch(stream, 1, static_cast<size_t>(wp.splits) * m * n * sizeof(float)))
+        wide = use_wide(c, m, n, k, &wp, 1);
     const int ksplits = wide ? wp.splits : c.splits;
     float* partials = nullptr;
     if (ksplits > 1) {

@@ -425,7 +425,7 @@ namespace dev {
 // error is larger there.  KCMM_GEMM_SPLITS forces the split (0 splits in the
 // result: it cannot be had); KCMM_GEMM_TILE = 100 + fb0 the token tiles'
 // height, 100 + 10 fb1 + fb0 two heights, half of the weight tiles each.
-GemmWidePlan gemm_wide_plan(uint32_t m, uint32_t n, uint32_t k, bool swiglu) {
+GemmWidePlan gemm_wide_plan(uint32_t m, uint32_t n, uint32_t k, bool swiglu, int max_splits) {
     const int M = static_cast<int>(m), N = static_cast<int>(n), K = static_cast<int>(k);
     const int forced = std::max(0, tunable_or(Tun::kGemmTile, -1) - 100);
     const int forced_splits = swiglu ? 1 : tunable_or(Tun::kGemmSplits, 0);
@@ -439,7 +439,7 @@ GemmWidePlan gemm_wide_plan(uint32_t m, uint32_t n, uint32_t k, bool swiglu) {
     };
     for (int fb = 1; fb <= 4; ++fb) {
         if (forced ? fb != forced % 10 : fb > 1 && 64 * (fb - 1) >= M) continue;
-        for (int s = 1; s <= (swiglu ? 1 : 8); s *= 2) {
+        for (int s = 1; s <= (swiglu ? 1 : max_splits); s *= 2) {
             if (chunks % s || chunks / s < (s > 1 ? 4 : 2)) break;
             if (forced_splits > 0 && s != forced_splits) continue;
             GemmWidePlan c;

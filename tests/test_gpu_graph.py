@@ -13,11 +13,13 @@ Cases: embedding + a three-layer kcmm_decode_layers_on_stream call + logits
 (bf16 and fp8-e4m3 pools; the fp8 page writer's zero-restored counters are
 replayed too), standalone paged decode attention (bf16, fp8), and a
 split-K projection with its reduction kernel."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import oracle as O
-from lattice_amd.bindings import KV_BF16, KV_FP8, memcpy_dtoh
+from lattice_amd.bindings import KV_BF16, KV_FP8, hip, memcpy_dtoh
 from lattice_amd.workload import build_decode_case
 from tests.test_gpu_glue import _layer_weights, bf16_dev
 
@@ -139,3 +141,137 @@ def test_split_gemm_graph_replays(gpu_lib):
         gpu_lib.gemm_bf16_add(x.data_ptr(), w.data_ptr(), r.data_ptr(), y.data_ptr(), m, n, k, s)
 
     _check_replays(torch, run, lambda: [y])
+
+
+class _KernelNode(C.Structure):   # hipKernelNodeParams
+    _fields_ = [("block", C.c_uint32 * 3), ("extra", C.c_void_p), ("func", C.c_void_p),
+                ("grid", C.c_uint32 * 3), ("params", C.c_void_p), ("shared", C.c_uint32)]
+
+
+def _captured_grids(run):
+    """Grids of the kernels that run(stream) leaves in a captured graph."""
+    h = hip()
+    st = C.c_void_p()
+    graph = C.c_void_p()
+    n = C.c_size_t()
+    assert h.hipStreamCreateWithFlags(C.byref(st), C.c_uint(1)) == 0
+    try:
+        run(st.value)                                     # a warm stream
+        assert h.hipStreamSynchronize(st) == 0
+        assert h.hipStreamBeginCapture(st, C.c_int(1)) == 0
+        try:
+            run(st.value)
+        finally:
+            rc = h.hipStreamEndCapture(st, C.byref(graph))
+        assert rc == 0
+        assert h.hipGraphGetNodes(graph, None, C.byref(n)) == 0
+        nodes = (C.c_void_p * n.value)()
+        assert h.hipGraphGetNodes(graph, nodes, C.byref(n)) == 0
+        grids = []
+        for node in nodes:
+            kp = _KernelNode()
+            assert h.hipGraphKernelNodeGetParams(C.c_void_p(node), C.byref(kp)) == 0
+            grids.append(tuple(kp.grid))
+        assert h.hipGraphDestroy(graph) == 0
+        return grids
+    finally:
+        h.hipStreamDestroy(st)
+
+
+def _scratch_free_work(torch, lib, what):
+    """(run, run_more, output, close): a call that can run without scratch
+    but takes some when run eagerly, and one that makes the stream's buffer
+    of that slot grow."""
+    g = torch.Generator(device="cuda")
+    g.manual_seed(11)
+    if what == "prefill":
+        case = build_decode_case(lib, batch=2, num_q_heads=32, kv_heads=8, head_dim=128,
+                                 block_size=16, ctx_lens=[4000, 900], dtype=KV_BF16, seed=3)
+        q = torch.randn((300, 32, 128), generator=g, device="cuda").to(torch.bfloat16)
+        out = torch.empty_like(q)
+        dv = case.dev
+
+        def prefill(lens, mbps):
+            qsl = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32,
+                               device="cuda")
+            bt = dv["bt"][:, :mbps].contiguous()
+            sl = torch.clamp(dv["sl"], max=mbps * 16)
+
+            def run(s):
+                case.pool.paged_attn_prefill(
+                    layer_idx=0, query_ptr=q.data_ptr(), out_ptr=out.data_ptr(),
+                    block_tables_ptr=bt.data_ptr(), seq_lens_ptr=sl.data_ptr(),
+                    query_start_loc_ptr=qsl.data_ptr(), block_offsets_f16_ptr=dv["offs"].data_ptr(),
+                    batch=2, total_query_tokens=int(sum(lens)), num_q_heads=32, kv_heads=8,
+                    head_dim=128, block_size=16, max_blocks_per_seq=mbps,
+                    scale=1 / np.sqrt(128), stream_ptr=s)
+            return run
+
+        return prefill([30, 20], 70), prefill([200, 100], 250), out[:50], case.pool.destroy
+    m, n, k, fp8 = dict(uneven=(5, 320, 11008, False), uneven_fp8=(5, 320, 11008, True),
+                        wide=(777, 6144, 4096, False))[what]
+    assert lib.gemm_plan(m, n, k, fp8_weights=fp8)["splits"] > 1
+    # the larger call: four times the rows, or the down projection (four splits of 777 x 4096)
+    more = (777, 4096, 14336) if what == "wide" else (4 * m, n, k)
+    x = torch.randn((more[0], more[2]), generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn((more[1], more[2]), generator=g, device="cuda") * 0.02
+    w = w.to(torch.float8_e4m3fn).view(torch.uint8) if fp8 else w.to(torch.bfloat16)
+    scale = torch.full((n,), 0.5, device="cuda")
+    y = torch.empty((max(m * n, more[0] * more[1]),), device="cuda", dtype=torch.bfloat16)
+
+    def product(m, n, k):
+        def run(s):
+            if fp8:
+                lib.gemm_fp8w_bf16(x.data_ptr(), w.data_ptr(), scale.data_ptr(), y.data_ptr(), m, n,
+                                   k, s)
+            else:
+                lib.gemm_bf16(x.data_ptr(), w.data_ptr(), y.data_ptr(), m, n, k, s)
+        return run
+
+    return product(m, n, k), product(*more), y[:m * n], lambda: None
+
+
+@pytest.mark.parametrize("what", ["prefill", "uneven", "uneven_fp8", "wide"])
+def test_captures_hold_no_optional_scratch(gpu_lib, what):
+    """Calls that can run without scratch do so under every capture, on a warm
+    stream too: one kernel with the whole key range or K in each workgroup
+    (grid.y 1), so that the graph holds no address of a buffer which a later,
+    larger call on the stream frees.  The replays after such a call, and on
+    another stream, equal those of a graph captured on a cold stream."""
+    import torch
+    run, run_more, out, close = _scratch_free_work(torch, gpu_lib, what)
+    try:
+        grids = _captured_grids(run)
+        assert len(grids) == 1 and grids[0][1] == 1, grids
+        graphs = []
+        for warm in (False, True):
+            st = torch.cuda.Stream()
+            graph = torch.cuda.CUDAGraph()
+            if warm:
+                run(st.cuda_stream)
+            torch.cuda.synchronize()
+            with torch.cuda.graph(graph, stream=st):
+                run(st.cuda_stream)
+            graphs.append((graph, st))
+        run(torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        eager = out.clone()
+        run_more(graphs[1][1].cuda_stream)               # the slot grows
+        torch.cuda.synchronize()
+        seen = []
+        for _ in range(2):
+            for graph, _st in graphs:
+                out.fill_(float("nan"))
+                torch.cuda.synchronize()
+                graph.replay()
+                torch.cuda.synchronize()
+                seen.append(out.clone())
+                run_more(torch.cuda.current_stream().cuda_stream)
+                torch.cuda.synchronize()
+        assert all(torch.equal(s, seen[0]) for s in seen)
+        # another order of the same fp32 sums, rounded to bf16
+        d = (seen[0].double() - eager.double()).norm() / eager.double().norm()
+        print(f"captured / eager {what}: {float(d):.2e}", flush=True)
+        assert float(d) <= 1e-2
+    finally:
+        close()
