@@ -417,16 +417,24 @@ bool gemm_tiled(uint64_t x, uint64_t w, uint64_t wscale, uint64_t y, uint32_t m,
         *err = "tiled gemm needs m > 0, n % 64 == 0 and k % 64 == 0";
         return false;
     }
-    const TiledConfig c = choose(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k));
+    TiledConfig c = choose(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k));
     if (splits != nullptr) *splits = 1;
     GemmWidePlan wp;
     bool wide = wscale == 0 && use_wide(c, m, n, k, &wp);
-    // A shape that this kernel runs unsplit can be captured without a call
-    // before it, and its graph outlives any workspace: the wide kernel takes it
-    // unsplit, or not at all, under a capture.
-    if (wide && wp.splits > 1 && c.splits == 1 &&
-        !stream_scratch(stream, 1, static_cast<size_t>(wp.splits) * m * n * sizeof(float)))
-        wide = use_wide(c, m, n, k, &wp, 1);
+    // Without scratch for the plan's partials: this kernel's plan if it has
+    // (it often takes half of the wide one's), the wide kernel unsplit, or
+    // this one unsplit.  A shape that this kernel runs unsplit can be captured
+    // without a call before it, and its graph outlives any workspace: no
+    // scratch for it under a capture.
+    const bool may_capture = c.splits > 1;
+    auto scratch = [&](int s) {
+        return s == 1 || stream_scratch(stream, 1, static_cast<size_t>(s) * m * n * sizeof(float),
+                                        may_capture);
+    };
+    if (!scratch(wide ? wp.splits : c.splits)) {
+        if (!scratch(c.splits)) c.splits = 1;
+        wide = wscale == 0 && use_wide(c, m, n, k, &wp, 1);
+    }
     const int ksplits = wide ? wp.splits : c.splits;
     float* partials = nullptr;
     if (ksplits > 1) {

@@ -148,15 +148,17 @@ class _KernelNode(C.Structure):   # hipKernelNodeParams
                 ("grid", C.c_uint32 * 3), ("params", C.c_void_p), ("shared", C.c_uint32)]
 
 
-def _captured_grids(run):
-    """Grids of the kernels that run(stream) leaves in a captured graph."""
+def _captured_grids(run, warm=None):
+    """Grids of the kernels that run(stream) leaves in a graph captured on a
+    stream which ran warm(stream) before."""
     h = hip()
     st = C.c_void_p()
     graph = C.c_void_p()
     n = C.c_size_t()
     assert h.hipStreamCreateWithFlags(C.byref(st), C.c_uint(1)) == 0
     try:
-        run(st.value)                                     # a warm stream
+        if warm is not None:
+            warm(st.value)
         assert h.hipStreamSynchronize(st) == 0
         assert h.hipStreamBeginCapture(st, C.c_int(1)) == 0
         try:
@@ -241,7 +243,7 @@ def test_captures_hold_no_optional_scratch(gpu_lib, what):
     import torch
     run, run_more, out, close = _scratch_free_work(torch, gpu_lib, what)
     try:
-        grids = _captured_grids(run)
+        grids = _captured_grids(run, warm=run)
         assert len(grids) == 1 and grids[0][1] == 1, grids
         graphs = []
         for warm in (False, True):
@@ -275,3 +277,59 @@ def test_captures_hold_no_optional_scratch(gpu_lib, what):
         assert float(d) <= 1e-2
     finally:
         close()
+
+
+@pytest.mark.parametrize("m,n,k,slot,kernels", [
+    (777, 4096, 14336, 0, 1),    # both kernels split it (4 and 2 ways): unsplit on a cold stream
+    (777, 6144, 4096, 0, 1),     # only the wide kernel splits it
+    (300, 4096, 14336, 4, 2),    # the slot holds the tiled kernel's 4 splits, not the wide one's 8
+    (300, 4096, 14336, 3, 1)])   # nor those
+def test_wide_splits_under_capture(gpu_lib, tunables, m, n, k, slot, kernels):
+    """A product whose split partials do not fit the stream's workspace is
+    captured with fewer splits, or none, instead of allocating in the capture.
+    Its replays equal each other and the float64 product (bound: fp32 sums of
+    k products, 2^-24 each, and one rounding to bf16)."""
+    import torch
+    assert gpu_lib.gemm_plan(m, n, k)["splits"] > 1
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + n)
+    x = torch.randn((m, k), generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn((n, k), generator=g, device="cuda") * 0.02).to(torch.bfloat16)
+    y = torch.empty((m, n), device="cuda", dtype=torch.bfloat16)
+    small = torch.empty((m, n), device="cuda", dtype=torch.bfloat16)
+
+    def run(s):
+        gpu_lib.gemm_bf16(x.data_ptr(), w.data_ptr(), y.data_ptr(), m, n, k, s)
+
+    def warm(s):   # a slot of `slot` splits' partials (buffers get a quarter more than asked for)
+        rows = m * slot // 4 * 4 // 5
+        if slot == 0:
+            return
+        tunables.setenv("KCMM_GEMM_TILE", "9")
+        tunables.setenv("KCMM_GEMM_SPLITS", "4")
+        gpu_lib.gemm_bf16(x.data_ptr(), w.data_ptr(), small.data_ptr(), rows, n, k, s)
+        tunables.delenv("KCMM_GEMM_TILE")
+        tunables.delenv("KCMM_GEMM_SPLITS")
+
+    assert len(_captured_grids(run, warm)) == kernels
+    st = torch.cuda.Stream()
+    warm(st.cuda_stream)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=st):
+        run(st.cuda_stream)
+    seen = []
+    for _ in range(3):
+        y.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        seen.append(y.clone())
+        run(torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+    assert all(torch.equal(s, seen[0]) for s in seen)
+    ref = x.double() @ w.double().t().contiguous()
+    mag = x.double().abs() @ w.double().abs().t().contiguous()
+    tol = k * 2.0 ** -24 * mag + 2.0 ** -8 * ref.abs() * 1.01
+    for got in (seen[0], y):
+        assert float(((got.double() - ref).abs() / tol).max()) <= 1.0
