@@ -186,6 +186,7 @@ struct GemmWideArgs {
 };
 GemmWidePlan gemm_wide_plan(uint32_t m, uint32_t n, uint32_t k, bool swiglu, int max_splits = 8);
 bool gemm_wide(const GemmWideArgs& a, std::string* err);
+int gemm_wide_forced();   // the tiling that KCMM_GEMM_TILE forces, less 100; 0: none
 
 // How a plain product of this shape runs (under the current KCMM_GEMM_*
 // settings): kernel 0 = weight-stream, 1 = LDS-tiled; K splits; tiling (tiled

@@ -393,8 +393,9 @@ bool use_wide(const TiledConfig& c, uint32_t m, uint32_t n, uint32_t k, dev::Gem
     if (forced >= 0 && forced < kCfgs) return false;
     *plan = dev::gemm_wide_plan(m, n, k, false, max_splits);
     if (plan->splits == 0) return false;
-    if (forced > 100) return true;
-    // (tiles of configurations other than 0, 9, 10 are N % 128 != 0 shapes)
+    if (dev::gemm_wide_forced() != 0) return true;
+    // (choose() offers configurations 0, 9 and 10 only, the ones modelled; for
+    // N % 128 != 0 that is 10)
     return plan->us < 0.92 * tiled_us(c, m, n, k);
 }
 

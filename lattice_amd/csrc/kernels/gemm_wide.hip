@@ -416,6 +416,12 @@ double wide_us(const dev::GemmWidePlan& c, int M, int N, int K, bool swiglu) {
 
 namespace dev {
 
+// (fb0 is 1..4; any other value above 100 forces nothing)
+int gemm_wide_forced() {
+    const int f = tunable_or(Tun::kGemmTile, -1) - 100;
+    return f > 0 && f % 10 >= 1 && f % 10 <= 4 ? f : 0;
+}
+
 // The plan of least modelled time: token tiles of 64 .. 256 (a ragged last
 // tile only as high as it needs), K splits of at least 4 chunks for plain
 // products, and -- when whole rounds of tiles leave a partly filled last round
@@ -427,7 +433,7 @@ namespace dev {
 // height, 100 + 10 fb1 + fb0 two heights, half of the weight tiles each.
 GemmWidePlan gemm_wide_plan(uint32_t m, uint32_t n, uint32_t k, bool swiglu, int max_splits) {
     const int M = static_cast<int>(m), N = static_cast<int>(n), K = static_cast<int>(k);
-    const int forced = std::max(0, tunable_or(Tun::kGemmTile, -1) - 100);
+    const int forced = gemm_wide_forced();
     const int forced_splits = swiglu ? 1 : tunable_or(Tun::kGemmSplits, 0);
     const int bn = swiglu ? 128 : 256;
     const int tiles_n = (N + bn - 1) / bn, chunks = K / 64;

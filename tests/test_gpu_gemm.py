@@ -566,3 +566,27 @@ def test_uneven_splits_under_capture(gpu_lib, fp8):
     mag = x.cpu().double().abs() @ wd.abs().t()
     tol = 2 * k * 2.0 ** -24 * mag + 2 * 2.0 ** -8 * eager.cpu().abs() * 1.01
     assert float(((seen[0].double() - eager).abs().cpu() / tol).max()) <= 1.0
+
+
+@pytest.mark.parametrize("tile", ["100", "105", "110", "999"])
+def test_tilings_that_do_not_exist_force_nothing(gpu_lib, tunables, tile):
+    """KCMM_GEMM_TILE above 100 without a token-tile height of 1..4: plain and
+    SwiGLU products run as with the variable unset."""
+    import torch
+    m, n, k = 130, 320, 512
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3)
+    x = torch.randn((m, k), generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn((2 * n, k), generator=g, device="cuda") * 0.02).to(torch.bfloat16)
+    s = torch.cuda.current_stream().cuda_stream
+    seen = []
+    for value in (None, tile):
+        if value:
+            tunables.setenv("KCMM_GEMM_TILE", value)
+        act = torch.full((m, n), float("nan"), device="cuda", dtype=torch.bfloat16)
+        gpu_lib.gemm_bf16_swiglu(x.data_ptr(), w.data_ptr(), act.data_ptr(), m, n, k, s)
+        torch.cuda.synchronize()
+        seen.append((act, run(gpu_lib, x, w), gpu_lib.gemm_plan(m, 2 * n, k)))
+    assert torch.isfinite(seen[0][0].float()).all()
+    assert torch.equal(seen[0][0], seen[1][0]) and torch.equal(seen[0][1], seen[1][1])
+    assert seen[0][2] == seen[1][2]
