@@ -15,7 +15,7 @@
 //    workgroup read the same tokens' rows of neighbouring heads together:
 //    with HW = Hkv a workgroup reads whole token rows (all heads, 2 KiB
 //    contiguous at the Llama-3-8B shape) instead of one head's 256-byte
-//    pieces at a 2 KiB stride (HW by the batch's size, see stream_hw);
+//    pieces at a 2 KiB stride (see stream_hw);
 //  * one tile read serves all G = Hq/Hkv query heads of its kv head (GQA
 //    reuse: each K/V byte is read from HBM once);
 //  * every load instruction covers eight tokens x 128 contiguous bytes (whole
@@ -1145,22 +1145,21 @@ int env_int(dev::Tun t, int dflt, int lo, int hi) {
 int stream_waves(int dtype) {
     return env_int(dev::Tun::kAttnWaves, dtype == kDtFP8 ? 2048 : 1024, 1, 1 << 20);
 }
-// Waves per workgroup by the batch's size (head, tile entries of the list at
-// full tables; call times, 32/8 heads of 128 unless said):
-//  * fp8 pages: 8 above 4096 entries (a row of 1 KiB read together), else 1 --
-//    8-wave workgroups are then too few (one sequence of 1456 tokens 11.1 us
-//    with 1, 14.4 with 8; of 10000 19.8 / 20.8; 16 of 1000 .. 4000 28.9 / 27.7);
-//  * 16-bit pages: 4 above 16384 entries at head_dim 128 with whole groups of 8
-//    kv heads, one workgroup per CU (64 sequences of 512 .. 4096 tokens 99.8 us
-//    with 4, 102.4 with 1; two of 41000 and 50000 69.5 / 73.1; 128 of 500 ..
-//    3000 152 / 160, 16 kv heads; the decode step is as fast), else 1 (16 of
-//    1000 .. 4000 40.0 / 38.5; 64 of 300 .. 1000 40.6 / 39.7; head_dim 64: 64
-//    sequences 56.6 / 53.6).
-int stream_hw(int dtype, int head_dim, int kv_heads, long long entries) {
-    int hw = 1;
-    if (dtype == kDtFP8) hw = entries > 4096 ? 8 : 1;
-    else if (head_dim == 128 && kv_heads % 8 == 0 && entries > 16384) hw = 4;
-    return env_int(dev::Tun::kAttnHw, hw, 1, 8);
+// Waves per workgroup:
+//  * 16-bit pages: 1.  Four-wave workgroups make attention calls alone faster
+//    (64 sequences of 512 .. 4096 tokens: kernel 103 us against 105.5), but the
+//    call slower where it follows a layer's other kernels (116.5 against 111),
+//    and the 32-layer step that it is part of 7.325 ms against 7.235 (Llama-3-8B
+//    shape, three alternating runs each, spread 0.01).
+//  * fp8 pages: 8 (a row of 1 KiB read together) where the tables have room for
+//    more than 8192 (kv head, tile) entries, else 1 -- 8-wave workgroups are then
+//    too few, whatever the lengths are.  Call times with 1 / 8, 32/8 heads of
+//    128: one sequence of 1456 tokens 11.9 / 15.6 us, 10000 17.3 / 21.5, 30000
+//    27.8 / 28.2; 8 of 3000 .. 4000 22.3 / 23.2; 12 of 3000 .. 4000 26.9 / 26.8;
+//    2 of 30000 34.2 / 32.6; 32 of 10000 111 / 100.  The host does not know the
+//    lengths: wider tables take 8, the better one at their full length.
+int stream_hw(int dtype, long long entries) {
+    return env_int(dev::Tun::kAttnHw, dtype == kDtFP8 && entries > 8192 ? 8 : 1, 1, 8);
 }
 int stream_min_tiles() { return env_int(dev::Tun::kAttnMinTiles, 0, 1, 1 << 16); }
 int stream_depth() { return env_int(dev::Tun::kAttnDepth, 2, 2, 3); }
@@ -1176,7 +1175,7 @@ bool launch_stream(AttnParams& p, hipStream_t s, bool no_alloc, std::string* err
     }
     if (p.batch == 0) return true;
     const int depth = stream_depth();
-    int hw = std::min(stream_hw(DT, D, p.kv_heads, tmax), depth == 3 ? 4 : 8);
+    int hw = std::min(stream_hw(DT, tmax), depth == 3 ? 4 : 8);
     while (p.kv_heads % hw) --hw;
     p.hw = hw;
     p.min_tiles = stream_min_tiles();

@@ -400,10 +400,11 @@ def test_stream_kernel_timing(gpu_lib):
     (6, 2, 128, KV_BF16, [700, 129, 1], 1),             # 96 quads: threads past the last
     (14, 2, 128, KV_BF16, [161, 96], 1),                # 224 quads, 4..6 parts
     (32, 8, 128, KV_BF16, [150, 290] * 18, 1),          # 288 (b, g) pairs: 4-wave workgroups
-    (32, 8, 128, KV_FP8, [1456], None), (32, 8, 128, KV_FP8, [1000] * 17, None),   # HW 1 / 8
+    (32, 8, 128, KV_FP8, [1456], None), (32, 8, 128, KV_FP8, [1000] * 17, None),   # HW 1
+    (32, 8, 128, KV_FP8, [1000] * 33, None),                                       # HW 8
     (8, 2, 128, KV_BF16, [1024, 1024], None), (8, 2, 128, KV_BF16, [1024, 1056], None),   # slice 1 / 2
     (8, 2, 64, KV_BF16, [5120], None), (8, 2, 64, KV_BF16, [5121], None),                 # slice 2 / 4
-    (16, 16, 128, KV_F16, [1025] * 32, None)])          # 16896 entries: four waves per workgroup
+    (16, 16, 128, KV_F16, [1025] * 32, None)])          # 16896 entries on 1024 slices
 def test_merge_and_slice_rules(gpu_lib, tunables, hq, hkv, d, dtype, ctx, min_tiles):
     """The log-sum-exp merge over many parts, output widths and workgroup
     sizes, and both sides of each rule that picks slice length and waves per

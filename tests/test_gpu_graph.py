@@ -148,8 +148,8 @@ class _KernelNode(C.Structure):   # hipKernelNodeParams
                 ("grid", C.c_uint32 * 3), ("params", C.c_void_p), ("shared", C.c_uint32)]
 
 
-def _captured_grids(run, warm=None):
-    """Grids of the kernels that run(stream) leaves in a graph captured on a
+def _captured_kernels(run, warm=None):
+    """(grid, block) of the kernels that run(stream) leaves in a graph captured on a
     stream which ran warm(stream) before."""
     h = hip()
     st = C.c_void_p()
@@ -169,13 +169,13 @@ def _captured_grids(run, warm=None):
         assert h.hipGraphGetNodes(graph, None, C.byref(n)) == 0
         nodes = (C.c_void_p * n.value)()
         assert h.hipGraphGetNodes(graph, nodes, C.byref(n)) == 0
-        grids = []
+        kernels = []
         for node in nodes:
             kp = _KernelNode()
             assert h.hipGraphKernelNodeGetParams(C.c_void_p(node), C.byref(kp)) == 0
-            grids.append(tuple(kp.grid))
+            kernels.append((tuple(kp.grid), tuple(kp.block)))
         assert h.hipGraphDestroy(graph) == 0
-        return grids
+        return kernels
     finally:
         h.hipStreamDestroy(st)
 
@@ -243,8 +243,8 @@ def test_captures_hold_no_optional_scratch(gpu_lib, what):
     import torch
     run, run_more, out, close = _scratch_free_work(torch, gpu_lib, what)
     try:
-        grids = _captured_grids(run, warm=run)
-        assert len(grids) == 1 and grids[0][1] == 1, grids
+        kernels = _captured_kernels(run, warm=run)
+        assert len(kernels) == 1 and kernels[0][0][1] == 1, kernels
         graphs = []
         for warm in (False, True):
             st = torch.cuda.Stream()
@@ -311,7 +311,7 @@ def test_wide_splits_under_capture(gpu_lib, tunables, m, n, k, slot, kernels):
         tunables.delenv("KCMM_GEMM_TILE")
         tunables.delenv("KCMM_GEMM_SPLITS")
 
-    assert len(_captured_grids(run, warm)) == kernels
+    assert len(_captured_kernels(run, warm)) == kernels
     st = torch.cuda.Stream()
     warm(st.cuda_stream)
     torch.cuda.synchronize()
@@ -333,3 +333,39 @@ def test_wide_splits_under_capture(gpu_lib, tunables, m, n, k, slot, kernels):
     tol = k * 2.0 ** -24 * mag + 2.0 ** -8 * ref.abs() * 1.01
     for got in (seen[0], y):
         assert float(((got.double() - ref).abs() / tol).max()) <= 1.0
+
+
+@pytest.mark.parametrize("dtype,ctx,tokens,waves", [
+    (KV_BF16, [600] * 64, 4800, 1),      # 9728 (kv head, tile) entries, 76800 in the wide table
+    (KV_FP8, [1456], 32768, 1),          # 368 and 8192
+    (KV_FP8, [600] * 64, 4800, 8)])
+def test_decode_workgroups_in_wide_tables(gpu_lib, dtype, ctx, tokens, waves):
+    """A table wider than its sequences, as a server keeps it at its maximum
+    length, gets the workgroups of a narrow one and the same result."""
+    import torch
+    case = build_decode_case(gpu_lib, batch=len(ctx), num_q_heads=32, kv_heads=8, head_dim=128,
+                             block_size=16, ctx_lens=ctx, dtype=dtype, seed=len(ctx))
+    try:
+        dv = case.dev
+        wide = torch.nn.functional.pad(dv["bt"], (0, tokens // 16 - case.mbps)).contiguous()
+        seen = []
+        for bt in (dv["bt"], wide):
+            out = torch.full((len(ctx), 32, 128), float("nan"), dtype=torch.bfloat16, device="cuda")
+
+            def run(s):
+                case.pool.paged_attn_decode(layer_idx=0, query_ptr=dv["q"].data_ptr(),
+                                            out_ptr=out.data_ptr(), block_tables_ptr=bt.data_ptr(),
+                                            seq_lens_ptr=dv["sl"].data_ptr(),
+                                            block_offsets_f16_ptr=dv["offs"].data_ptr(),
+                                            batch=len(ctx), num_q_heads=32, kv_heads=8,
+                                            head_dim=128, block_size=16,
+                                            max_blocks_per_seq=bt.shape[1],
+                                            scale=1.0 / np.sqrt(128), stream_ptr=s)
+
+            assert _captured_kernels(run, warm=run)[0][1] == (64 * waves, 1, 1)
+            run(torch.cuda.current_stream().cuda_stream)
+            torch.cuda.synchronize()
+            seen.append(out)
+        assert torch.isfinite(seen[0].float()).all() and torch.equal(seen[0], seen[1])
+    finally:
+        case.pool.destroy()
