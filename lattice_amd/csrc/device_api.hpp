@@ -44,7 +44,7 @@ void reload_tunables();
 // attention segment table, 3: decode layer-step activations, 4: the final
 // norm's output, 5: prefill attention key splits, 6: tiering staging on
 // the null stream, 7: fp8 RoPE/append staging, 8: fp8 page-writer row
-// table).  `zero_fill` buffers start zeroed by a fill kernel, and their
+// table, 9: counts of the prefill key splits).  `zero_fill` buffers start zeroed by a fill kernel, and their
 // users leave them zeroed.  Keyed by host thread as well, so a thread that
 // grows a buffer never frees one another thread has been handed.  Growth
 // synchronizes the stream and calls hipMalloc, so it cannot happen under

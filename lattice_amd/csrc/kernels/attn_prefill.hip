@@ -48,17 +48,43 @@ struct PrefillParams {
     float scale_log2;
     float scale;
     // key splits (SPLIT): per (item, kv head) and split, the 256 columns'
-    // unnormalised outputs [column][D] and (max, denominator) pairs
+    // unnormalised outputs and (max, denominator) pairs; per (item, kv head)
+    // four counts (zero between calls)
     float* part_acc;
     float* part_ml;
+    int32_t* counts;
     int splits;
 };
 
-// Tiles per key split of a workgroup with nt tiles: equal parts, but no part
-// shorter than 8 tiles (a part costs its page-table chain, about 4 tiles).
-constexpr int kSplitTiles = 8;
+// Tiles per key split of an item with nt tiles: equal parts, an even number of
+// tiles (the loop runs two at a time), none shorter than 8, and no split below
+// 18.  A part costs the page-table chain and the combining about 7 us, as much
+// as 8 tiles (500 tokens without a prefix, 16 tiles in the longest item: 22.7
+// us unsplit, 23.3 in two parts; 64 behind 500, 18 tiles: 24.8 and 23.3).
+constexpr int kSplitTiles = 8, kSplitFrom = 18;
+constexpr int kMaxSplits = 16;
+// Looks (of about 1 us) that a workgroup takes for the other parts before it
+// goes.  Parts that run side by side end within few us; longer waits hold CUs
+// that parts of a second round need (32 looks, 384 workgroups: 65 us against 45).
+constexpr int kPolls = 8;
 __device__ __forceinline__ int split_tiles(int nt, int splits) {
-    return max(kSplitTiles, (nt + splits - 1) / splits);
+    if (nt < kSplitFrom) return nt;
+    return max(kSplitTiles, ((nt + splits - 1) / splits + 1) & ~1);
+}
+
+// Partial results pass between workgroups of any XCD through device-coherent
+// accesses, which need no cache write-back or invalidation around them.
+__device__ __forceinline__ void put_pair(float* p, float a, float b) {
+    const uint64_t v = __float_as_uint(a) | static_cast<uint64_t>(__float_as_uint(b)) << 32;
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t get_pair(const float* p) {
+    return __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float pair_lo(uint64_t v) { return __uint_as_float(static_cast<uint32_t>(v)); }
+__device__ __forceinline__ float pair_hi(uint64_t v) {
+    return __uint_as_float(static_cast<uint32_t>(v >> 32));
 }
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
@@ -183,11 +209,12 @@ __device__ __forceinline__ void find_item(int item, int batch, const int32_t* __
 }
 
 // Workgroups over (query-token block, kv head), kv head fastest: blockIdx.x
-// = item * Hkv + g, items in longest-first order (see below).  Workgroups are dealt to the 8 XCDs round-robin, so with
-// 8 kv heads every XCD serves one head and its L2 holds that head's pages
-// (shared prefixes included) for all sequences.
-// With SPLIT, blockIdx.y takes one part of the workgroup's keys; a workgroup
-// with more than one part leaves partial results for attn_prefill_merge.
+// = item * Hkv + g, items in longest-first order (find_item).  Workgroups are
+// dealt to the 8 XCDs round-robin, so with 8 kv heads every XCD serves one head
+// and its L2 holds that head's pages (shared prefixes included) for all
+// sequences.
+// With SPLIT, blockIdx.y takes one part of the item's keys; of an item with
+// more than one part, the workgroups that finish last combine them.
 template <int DT, int D, int G, int NW, int NCB, int KT, bool SPLIT>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2)))
 void attn_prefill_mfma(PrefillParams p, const uint8_t* __restrict__ kreg,
@@ -236,13 +263,13 @@ void attn_prefill_mfma(PrefillParams p, const uint8_t* __restrict__ kreg,
     const int nt_wg = (max(0, first_pos + min(tok0_wg + TWG, len)) + KT - 1) / KT;
     // this workgroup's tiles t_beg .. t_end (all of them without SPLIT)
     int t_beg = 0, t_end = nt_wg;
-    bool partial = false;
+    int parts = 1;
     if constexpr (SPLIT) {
         const int per = split_tiles(nt_wg, p.splits);
         t_beg = blockIdx.y * per;
         if (t_beg > 0 && t_beg >= nt_wg) return;   // uniform
         t_end = min(nt_wg, t_beg + per);
-        partial = nt_wg > per;
+        parts = max(1, (nt_wg + per - 1) / per);
     }
     const int tok0 = tok0_wg + wave * TPW;  // this wave's first query (chunk index)
     const bool wave_live = tok0 < len;
@@ -550,24 +577,129 @@ void attn_prefill_mfma(PrefillParams p, const uint8_t* __restrict__ kreg,
     }
 
     // ---- store the columns that are real queries ----
-    if (!wave_live) return;
     if constexpr (SPLIT) {
-        if (partial) {
-            const size_t unit = static_cast<size_t>(blockIdx.x) * p.splits + blockIdx.y;
+        if (parts > 1) {   // (uniform)
+            // each lane's values in its own order: [split][wave][column block][element pair][lane]
+            const size_t unit0 = static_cast<size_t>(blockIdx.x) * p.splits;
+            constexpr int LANE2 = 64 * 2;   // floats of one pair of every lane
+            auto acc_at = [&](int s, int w, int cb) {
+                return p.part_acc + (((unit0 + s) * NW + w) * NCB + cb) * (DB * 2 * LANE2) + lane * 2;
+            };
+            auto ml_at = [&](int s, int w, int cb) {
+                return p.part_ml + ((((unit0 + s) * NW + w) * NCB + cb) * 16 + ln) * 2;
+            };
+            if (wave_live) {
 #pragma unroll
-            for (int cb = 0; cb < NCB; ++cb) {
-                const size_t col = unit * (NW * NCB * 16) + (wave * NCB + cb) * 16 + ln;
-                if (lg == 0) {
-                    p.part_ml[2 * col] = m_run[cb];
-                    p.part_ml[2 * col + 1] = lsum[cb][0];
+                for (int cb = 0; cb < NCB; ++cb) {
+                    if (lg == 0) put_pair(ml_at(blockIdx.y, wave, cb), m_run[cb], lsum[cb][0]);
+                    float* o = acc_at(blockIdx.y, wave, cb);
+#pragma unroll
+                    for (int db = 0; db < DB; ++db) {
+                        put_pair(o + (2 * db) * LANE2, acc[cb][db][0], acc[cb][db][1]);
+                        put_pair(o + (2 * db + 1) * LANE2, acc[cb][db][2], acc[cb][db][3]);
+                    }
                 }
-                float* o = p.part_acc + col * D + 4 * lg;
-#pragma unroll
-                for (int db = 0; db < DB; ++db) *reinterpret_cast<f32x4*>(o + 16 * db) = acc[cb][db];
             }
+            // Every wave's stores are performed before the workgroup counts
+            // itself in.  A workgroup that then sees all parts in takes some of
+            // the waves' columns at a time until none is left; one that does not
+            // within kPolls looks goes.  The last one in always sees them all,
+            // so every column is combined, and no one waits for more than that.
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __shared__ int s_word;
+            int32_t* const count = p.counts + static_cast<size_t>(blockIdx.x) * 4;   // in, taken, out
+            auto add = [&](int i, int v) {
+                return __hip_atomic_fetch_add(count + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            };
+            __syncthreads();
+            if (tid == 0) {
+                int in = add(0, 1) + 1;
+                for (int i = 0; in < parts && i < kPolls; ++i) {
+                    __builtin_amdgcn_s_sleep(4);
+                    in = __hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                s_word = in == parts;
+            }
+            __syncthreads();
+            const int live = (min(len - tok0_wg, TWG) + TPW - 1) / TPW;   // waves with queries
+            int most = 1;                                                  // waves taken at a time
+            while (most * parts < live) most *= 2;                         // (at most NW / 2)
+            for (bool go = s_word != 0; go;) {
+                __syncthreads();   // s_word is read
+                if (tid == 0) s_word = add(1, most);
+                __syncthreads();
+                const int first = s_word;
+                go = first < live;
+                const int per_wave = NW / most;   // waves on one wave's columns
+                const int w0 = first + wave / per_wave;
+                if (!go || w0 >= live) continue;
+                const int units = NCB * DB / per_wave;   // 16-dim blocks for this wave, of one cb
+                const int u0 = (wave % per_wave) * units, cb = u0 / DB;
+                // weights 2^(max - overall max) of the parts over the denominator
+                uint64_t ml[kMaxSplits];
+                float w[kMaxSplits], top = -INFINITY, l = 0.0f;
+#pragma unroll
+                for (int s = 0; s < kMaxSplits; ++s)
+                    if (s < parts) ml[s] = get_pair(ml_at(s, w0, cb));
+#pragma unroll
+                for (int s = 0; s < kMaxSplits; ++s)
+                    if (s < parts) top = fmaxf(top, pair_lo(ml[s]));
+#pragma unroll
+                for (int s = 0; s < kMaxSplits; ++s) {
+                    if (s >= parts) continue;
+                    // a part without a visible key (max = -inf) has weight 0
+                    w[s] = pair_lo(ml[s]) == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(pair_lo(ml[s]) - top);
+                    l += w[s] * pair_hi(ml[s]);
+                }
+                const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+                const int t = tok0_wg + w0 * TPW + cb * TPB + ln / G;
+                uint16_t* o = reinterpret_cast<uint16_t*>(p.out) +
+                              ((static_cast<size_t>(q0) + t) * p.num_q_heads + g * G + ln % G) * D + 4 * lg;
+                constexpr int UB = 2;   // blocks in flight
+                for (int u = 0; u < units; u += UB) {
+                    uint64_t v[kMaxSplits][UB][2];
+                    f32x4 sum[UB];
+#pragma unroll
+                    for (int s = 0; s < kMaxSplits; ++s)
+                        if (s < parts) {
+#pragma unroll
+                            for (int e = 0; e < UB; ++e) {
+                                const float* a = acc_at(s, w0, cb) + 2 * (u0 % DB + min(u + e, units - 1)) * LANE2;
+                                v[s][e][0] = get_pair(a);
+                                v[s][e][1] = get_pair(a + LANE2);
+                            }
+                        }
+#pragma unroll
+                    for (int e = 0; e < UB; ++e) sum[e] = f32x4{0, 0, 0, 0};
+#pragma unroll
+                    for (int s = 0; s < kMaxSplits; ++s)
+                        if (s < parts) {
+#pragma unroll
+                            for (int e = 0; e < UB; ++e) {
+                                sum[e][0] += w[s] * pair_lo(v[s][e][0]);
+                                sum[e][1] += w[s] * pair_hi(v[s][e][0]);
+                                sum[e][2] += w[s] * pair_lo(v[s][e][1]);
+                                sum[e][3] += w[s] * pair_hi(v[s][e][1]);
+                            }
+                        }
+#pragma unroll
+                    for (int e = 0; e < UB; ++e) {
+                        if (u + e >= units || t >= len) continue;
+                        u32x2 r;
+                        r[0] = pack2<MDT>(sum[e][0] * inv, sum[e][1] * inv);
+                        r[1] = pack2<MDT>(sum[e][2] * inv, sum[e][3] * inv);
+                        *reinterpret_cast<u32x2*>(o + 16 * (u0 % DB + u + e)) = r;
+                    }
+                }
+            }
+            // the last one out leaves the counts at zero
+            if (tid == 0 && add(2, 1) == parts - 1)
+                for (int i = 0; i < 3; ++i)
+                    __hip_atomic_store(count + i, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             return;
         }
     }
+    if (!wave_live) return;
 #pragma unroll
     for (int cb = 0; cb < NCB; ++cb) {
         const float lt = lsum[cb][0];
@@ -585,68 +717,6 @@ void attn_prefill_mfma(PrefillParams p, const uint8_t* __restrict__ kreg,
                 *reinterpret_cast<u32x2*>(o + 16 * db) = w;
             }
         }
-    }
-}
-
-// Combines the key splits of (item, kv head) workgroup blockIdx.x for the 32
-// columns of its wave blockIdx.y: weights 2^(max - overall max) per column and
-// split in LDS, then every thread sums four dims of a column at a time.
-constexpr int kMaxSplits = 16;
-template <int DT, int D, int G, int NW, int NCB, int KT>
-__global__ __launch_bounds__(256) void attn_prefill_merge(PrefillParams p,
-                                                          const int32_t* __restrict__ sl,
-                                                          const int32_t* __restrict__ qsl) {
-    constexpr int MDT = DT == kDtFP8 ? kDtBF16 : DT;
-    constexpr int TPB = 16 / G, TPW = NCB * TPB, TWG = NW * TPW, COLS = NCB * 16;
-    __shared__ float s_w[kMaxSplits][COLS];
-    const int tid = threadIdx.x;
-    const int g = static_cast<int>(blockIdx.x) % p.kv_heads;
-    int b, blk;
-    find_item<TWG>(static_cast<int>(blockIdx.x) / p.kv_heads, p.batch, qsl, tid & 63, b, blk);
-    if (b < 0) return;
-    const int q0 = qsl[b], len = qsl[b + 1] - q0;
-    const int L = min(sl[b], p.mbps << p.bs_shift);
-    const int nt = (max(0, L - len + min((blk + 1) * TWG, len)) + KT - 1) / KT;
-    const int per = split_tiles(nt, p.splits);
-    const int tok0 = blk * TWG + static_cast<int>(blockIdx.y) * TPW;
-    if (nt <= per || tok0 >= len) return;   // (uniform: one part, or no query)
-    const int parts = (nt + per - 1) / per;
-    const size_t col0 = static_cast<size_t>(blockIdx.x) * p.splits * (NW * COLS) + blockIdx.y * COLS;
-    auto col_at = [&](int s, int c) { return col0 + static_cast<size_t>(s) * (NW * COLS) + c; };
-    if (tid < COLS) {
-        float top = -INFINITY, l = 0.0f;
-        for (int s = 0; s < parts; ++s) top = fmaxf(top, p.part_ml[2 * col_at(s, tid)]);
-        for (int s = 0; s < parts; ++s) {
-            const float m = p.part_ml[2 * col_at(s, tid)];
-            // a part without a visible key (m = -inf) has weight 0
-            const float w = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - top);
-            s_w[s][tid] = w;
-            l += w * p.part_ml[2 * col_at(s, tid) + 1];
-        }
-        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-        for (int s = 0; s < parts; ++s) s_w[s][tid] *= inv;
-    }
-    __syncthreads();
-    for (int i = tid; i < COLS * D / 4; i += 256) {
-        const int c = i / (D / 4), d = (i - c * (D / 4)) * 4;
-        const int t = tok0 + c / 16 * TPB + c % 16 / G;
-        if (t >= len) continue;
-        f32x4 o = f32x4{0, 0, 0, 0};
-        for (int s0 = 0; s0 < parts; s0 += 4) {
-            f32x4 v[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                v[e] = *reinterpret_cast<const f32x4*>(p.part_acc + col_at(min(s0 + e, parts - 1), c) * D + d);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (s0 + e < parts) o += s_w[s0 + e][c] * v[e];
-        }
-        u32x2 w;
-        w[0] = pack2<MDT>(o[0], o[1]);
-        w[1] = pack2<MDT>(o[2], o[3]);
-        *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(p.out) +
-                                  ((static_cast<size_t>(q0) + t) * p.num_q_heads + g * G + c % G) * D +
-                                  d) = w;
     }
 }
 
@@ -752,26 +822,31 @@ bool launch_mfma(const dev::AttnPrefillArgs& a, PrefillParams& p, hipStream_t s,
         *err = "prefill: too many query tokens";
         return false;
     }
-    // Too few token blocks for one workgroup per CU: split the keys.  The
-    // host knows the chunk's tokens and the tables' width, not the lengths:
-    // as many parts as fill the CUs once, each at least 8 tiles of a full
-    // table (the parts of a shorter sequence are longer ones, fewer:
-    // split_tiles).  A merge kernel follows, about 2 us where nothing was
-    // split after all (64 tokens without a prefix in a wide table 10.5 ->
-    // 12.3 us).  32/8 heads of 128, bf16, unsplit / split: 64 tokens behind 500
-    // 25 / 22 us, 2000 68 / 26, 8000 237 / 46; 512 behind 2000 84 / 46; 1000
-    // behind 1000 68 / 54; 4 sequences of up to 120 behind 2000 70 / 40.  More
-    // parts than fill the CUs once lose (512 behind 2000: 4 parts 45 us, 8 57).
+    // Too few items for one workgroup per CU: split the keys.  The host knows
+    // the chunk's tokens and the tables' width, not the lengths: it offers as
+    // many parts as fill the CUs once, and the workgroups take as many of them
+    // as their item has tiles for (split_tiles), none for a short one, in the
+    // one launch (a merge kernel after it cost short prompts in wide tables 2 us:
+    // 64 tokens without a prefix 10.1 -> 12.1 us, 200 14.1 -> 16.3).  32/8 heads of
+    // 128, bf16, unsplit / split: 64 tokens behind 500 24.8 / 23.3 us, 2000 67.9
+    // / 21.9, 8000 238 / 33.2; 512 behind 2000 80.8 / 40.3; 1000 behind 1000 65.8
+    // / 47.0; 4 sequences of up to 120 behind 2000 69.0 / 35.8; 64 and 200 without
+    // a prefix 10.1 and 14.1 / 10.1 and 14.3.  Tables 8 times as wide: the same.
     // A capture runs unsplit, and its graph holds no workspace.
-    const long long busy = std::max<long long>((a.total_query_tokens + TWG - 1) / TWG, a.batch) *
-                           p.kv_heads;
+    //
+    // items: the most that these tokens make (one per sequence, and one more
+    // per TWG further tokens)
+    const long long seqs = std::min(a.batch, a.total_query_tokens);
+    const long long busy = ((a.total_query_tokens - seqs) / TWG + seqs) * p.kv_heads;
     const long long cap_tiles = ((static_cast<long long>(p.mbps) << p.bs_shift) + KT - 1) / KT;
     int splits = static_cast<int>(std::min<long long>(
-        {256 / std::max(1LL, busy), cap_tiles / kSplitTiles, static_cast<long long>(kMaxSplits)}));
-    const size_t cols = static_cast<size_t>(blocks) * std::max(splits, 1) * NW * NCB * 16;
+        {256 / busy, cap_tiles < kSplitFrom ? 1 : (cap_tiles + kSplitTiles - 1) / kSplitTiles,
+         static_cast<long long>(kMaxSplits)}));
+    const size_t cols = static_cast<size_t>(busy) * std::max(splits, 1) * NW * NCB * 16;
     const size_t part_bytes = cols * (D + 2) * sizeof(float);
+    const size_t count_bytes = static_cast<size_t>(busy) * 4 * sizeof(int32_t);
     if (splits > 1 && !dev::stream_scratch(a.stream, 5, part_bytes)) splits = 1;
-    const dim3 grid(static_cast<unsigned>(blocks), splits > 1 ? splits : 1);
+    const dim3 grid(static_cast<unsigned>(splits > 1 ? busy : blocks), splits > 1 ? splits : 1);
     auto run = [&](auto split) {
         hipLaunchKernelGGL((attn_prefill_mfma<DT, D, G, NW, NCB, KT, decltype(split)::value>), grid,
                            dim3(NW * 64), 0, s, p, reinterpret_cast<const uint8_t*>(a.k_base),
@@ -782,18 +857,15 @@ bool launch_mfma(const dev::AttnPrefillArgs& a, PrefillParams& p, hipStream_t s,
                            reinterpret_cast<const uint64_t*>(a.offsets_f16));
     };
     if (splits > 1) {
-        void* ws = nullptr;
-        if (!dev::stream_workspace(a.stream, 5, part_bytes, &ws, false, err))
+        void *ws = nullptr, *counts = nullptr;
+        if (!dev::stream_workspace(a.stream, 5, part_bytes, &ws, false, err) ||
+            !dev::stream_workspace(a.stream, 9, count_bytes, &counts, true, err))
             return false;
         p.splits = splits;
         p.part_ml = static_cast<float*>(ws);
         p.part_acc = p.part_ml + 2 * cols;
+        p.counts = static_cast<int32_t*>(counts);
         run(std::true_type{});
-        KCMM_HIP_CHECK(hipGetLastError(), err);
-        hipLaunchKernelGGL((attn_prefill_merge<DT, D, G, NW, NCB, KT>),
-                           dim3(static_cast<unsigned>(blocks), NW), dim3(256), 0, s, p,
-                           reinterpret_cast<const int32_t*>(a.seq_lens),
-                           reinterpret_cast<const int32_t*>(a.query_start_loc));
     } else {
         run(std::false_type{});
     }

@@ -330,3 +330,49 @@ def test_key_splits_under_capture(gpu_lib):
         assert rel_err(got, ref) <= TOL[KV_BF16]
     finally:
         case.pool.destroy()
+
+
+@pytest.mark.parametrize("dtype,hq,hkv,d", [(KV_BF16, 32, 8, 128), (KV_FP8, 16, 4, 128),
+                                            (KV_F16, 8, 8, 64)])
+@pytest.mark.parametrize("widen", [1, 8])
+def test_key_splits_repeat_on_two_streams(gpu_lib, dtype, hq, hkv, d, widen):
+    """Split items are combined by whichever workgroups end last, in a fixed
+    order: calls on two streams at once give the same bits every time, equal
+    to the oracle's result, also in tables 8 times as wide as the sequences
+    (more parts offered) and with unsplit items beside the split ones."""
+    import torch
+    ctx, lens = [2500, 577, 576, 60], [70, 9, 33, 60]   # 79, 19, 18 and 2 tiles
+    case = build_decode_case(gpu_lib, batch=4, num_q_heads=hq, kv_heads=hkv, head_dim=d,
+                             block_size=16, ctx_lens=ctx, dtype=dtype, seed=21)
+    try:
+        got, ref = run_prefill(case, lens, hq, seed=7)
+        assert np.isfinite(got).all() and rel_err(got, ref) <= TOL[dtype]
+        bt = torch.nn.functional.pad(case.dev["bt"], (0, case.mbps * (widen - 1))).contiguous()
+        io = torch.float16 if dtype == KV_F16 else torch.bfloat16
+        rows = sum(lens)
+        q = encode16(io_dtype(dtype),
+                     np.random.default_rng(7).standard_normal((rows, hq, d)).astype(np.float32))
+        qt = torch.from_numpy(q.view(np.int16)).view(io).cuda()
+        qsl = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32, device="cuda")
+        dv = case.dev
+        streams = [torch.cuda.Stream() for _ in range(2)]
+        outs = [[torch.full((rows, hq, d), float("nan"), dtype=io, device="cuda") for _ in range(12)]
+                for _ in streams]
+        torch.cuda.synchronize()
+        for i in range(12):
+            for st, out in zip(streams, outs):
+                case.pool.paged_attn_prefill(
+                    layer_idx=0, query_ptr=qt.data_ptr(), out_ptr=out[i].data_ptr(),
+                    block_tables_ptr=bt.data_ptr(), seq_lens_ptr=dv["sl"].data_ptr(),
+                    query_start_loc_ptr=qsl.data_ptr(), block_offsets_f16_ptr=dv["offs"].data_ptr(),
+                    batch=4, total_query_tokens=rows, num_q_heads=hq, kv_heads=hkv, head_dim=d,
+                    block_size=16, max_blocks_per_seq=case.mbps * widen, scale=1 / math.sqrt(d),
+                    stream_ptr=st.cuda_stream)
+        torch.cuda.synchronize()
+        first = outs[0][0]
+        assert torch.isfinite(first.float()).all()
+        assert all(torch.equal(o, first) for out in outs for o in out)
+        assert rel_err(first.float().cpu().numpy().astype(np.float64).reshape(got.shape),
+                       ref) <= TOL[dtype]
+    finally:
+        case.pool.destroy()
