@@ -184,8 +184,6 @@ __global__ __launch_bounds__(256) void kv_slots_fp8_collect(SlotArgs a, uint32_t
 }
 
 // grid (ceil(batch / R)); 64 * waves threads; dynamic LDS R * block_size * 4.
-// (The resolve step is written without nested branches: the compiler dropped
-// the id of rows with an active flag from an if / else-if chain here.)
 __global__ __launch_bounds__(64 * kFp8MaxWaves) void kv_slots_fp8_write(SlotArgs a,
                                                                          uint32_t batch, uint32_t R,
                                                                          int32_t* lead,
@@ -201,13 +199,11 @@ __global__ __launch_bounds__(64 * kFp8MaxWaves) void kv_slots_fp8_write(SlotArgs
         // this workgroup's rows, one per lane: status, then the distinct pages
         const int64_t slot = t < R && r0 + t < batch ? a.slots[r0 + t] : -1;
         const int64_t b = block_of(a, slot < 0 ? 0 : slot);
-        const bool past = b >= static_cast<int64_t>(a.offsets_len);
-        uint32_t active = 1;
-        if (a.valid != nullptr) active = a.valid[slot < 0 || past ? 0 : b];
-        if (a.status != nullptr && slot >= 0 && (past || active == 0))
-            atomicCAS(a.status, 0, past ? 1 : 2);
-        const int32_t id =   // (offsets_len <= 2^28)
-            slot < 0 || past || active == 0 ? -1 : static_cast<int32_t>(b);
+        const bool row = slot >= 0, past = b >= static_cast<int64_t>(a.offsets_len);
+        bool active = row && !past;
+        if (active && a.valid != nullptr) active = a.valid[b] != 0;
+        if (a.status != nullptr && row && !active) atomicCAS(a.status, 0, past ? 1 : 2);
+        const int32_t id = active ? static_cast<int32_t>(b) : -1;   // (offsets_len <= 2^28)
         bool first = id >= 0;
         for (uint32_t j = 0; j + 1 < R; ++j) {
             const int32_t other = __shfl(id, j);
