@@ -99,11 +99,39 @@ __device__ __forceinline__ float bf16_round_f32(float f) {
     return bf16_bits_to_f32(f32_to_bf16_bits(f));
 }
 
+// The same by the hardware conversion: the bits of f32_to_bf16_bits for every
+// float but NaN (whose sign and payload it keeps).
+__device__ __forceinline__ float bf16_round_hw(float f) {
+    return static_cast<float>(static_cast<__bf16>(f));
+}
+
+// Eight values as bf16, the bits of f32_to_bf16_bits: hardware conversions
+// (the integer form of 128 values per lane cost the wide GEMM's store 3% of a
+// 2048-token gate/up product), and the integer form where a value is NaN.
+__device__ __forceinline__ u32x4 pack_bf16x8(const float (&v)[8]) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    u32x4 o;
+    bool nan = false;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const bf16x2 p = {static_cast<__bf16>(v[2 * i]), static_cast<__bf16>(v[2 * i + 1])};
+        o[i] = __builtin_bit_cast(uint32_t, p);
+        nan |= __builtin_isunordered(v[2 * i], v[2 * i + 1]);
+    }
+    if (__builtin_expect(__any(nan), 0)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            o[i] = f32_to_bf16_bits(v[2 * i]) | (f32_to_bf16_bits(v[2 * i + 1]) << 16);
+    }
+    return o;
+}
+
 // Decoder-layer element arithmetic shared by the standalone glue kernels and
 // the GEMM epilogues that fuse them, so both give identical bits.
 //  * RoPE of one rotate-half pair (x1 = element i, x2 = element i + D/2):
 //    x1' = x1 c - x2 s, x2' = x2 c + x1 s, with c, s of pos * inv_freq[i];
-//  * SwiGLU: bf16(bf16(silu(g)) * u), the roundings of a bf16 model.
+//  * SwiGLU: bf16(bf16(silu(g)) * u), the roundings of a bf16 model
+//    (swiglu_product leaves the last one to the store).
 __device__ __forceinline__ void rope_cos_sin(int pos, float inv_freq, float* c, float* s) {
     const float ang = static_cast<float>(pos) * inv_freq;
     *c = cosf(ang);
@@ -115,9 +143,12 @@ __device__ __forceinline__ float rope_first(float x1, float x2, float c, float s
 __device__ __forceinline__ float rope_second(float x1, float x2, float c, float s) {
     return __builtin_fmaf(x2, c, x1 * s);
 }
+template <typename Round>
+__device__ __forceinline__ float swiglu_product(float g, float u, Round round) {
+    return round(g / (1.0f + __expf(-g))) * u;
+}
 __device__ __forceinline__ float swiglu_bf16(float g, float u) {
-    const float sg = bf16_round_f32(g / (1.0f + __expf(-g)));
-    return bf16_round_f32(sg * u);
+    return bf16_round_f32(swiglu_product(g, u, [](float x) { return bf16_round_f32(x); }));
 }
 
 }  // namespace kcmm

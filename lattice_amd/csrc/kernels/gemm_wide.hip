@@ -42,7 +42,6 @@ namespace kcmm {
 namespace {
 
 typedef __attribute__((address_space(3))) void* lds_ptr;
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 // 16 bytes per lane from global memory straight into LDS at lds + 16 * lane
 // (lds is wave-uniform).
@@ -73,14 +72,6 @@ __device__ __forceinline__ void phase_barrier() {
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("" ::: "memory");
-}
-
-__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
-    const bf16x2 v = {static_cast<__bf16>(lo), static_cast<__bf16>(hi)};
-    return __builtin_bit_cast(uint32_t, v);
-}
-__device__ __forceinline__ float round_bf16(float x) {
-    return static_cast<float>(static_cast<__bf16>(x));
 }
 
 struct WideParams {
@@ -263,20 +254,15 @@ __device__ __forceinline__ void wide_tile(const WideParams& p, uint8_t* lds, int
             if constexpr (EPI == kWideSwiglu) {
                 const int n = n0 + wn * 32 + 8 * lg;
                 if (n >= p.N) continue;
-                u32x4 o;
+                float v[8];
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    float v[4];
+                for (int i = 0; i < 2; ++i)
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const float g = round_bf16(acc[0][i][bh][j][r]);
-                        const float u = round_bf16(acc[1][i][bh][j][r]);
-                        v[r] = round_bf16(g / (1.0f + __expf(-g))) * u;
-                    }
-                    o[2 * i] = pack_bf16(v[0], v[1]);
-                    o[2 * i + 1] = pack_bf16(v[2], v[3]);
-                }
-                *reinterpret_cast<u32x4*>(p.Y + static_cast<size_t>(m) * p.N + n) = o;
+                    for (int r = 0; r < 4; ++r)
+                        v[4 * i + r] = swiglu_product(bf16_round_hw(acc[0][i][bh][j][r]),
+                                                      bf16_round_hw(acc[1][i][bh][j][r]),
+                                                      [](float x) { return bf16_round_hw(x); });
+                *reinterpret_cast<u32x4*>(p.Y + static_cast<size_t>(m) * p.N + n) = pack_bf16x8(v);
             } else {
 #pragma unroll
                 for (int ah = 0; ah < 2; ++ah) {
@@ -299,14 +285,11 @@ __device__ __forceinline__ void wide_tile(const WideParams& p, uint8_t* lds, int
                         const u32x4 rr = *reinterpret_cast<const u32x4*>(p.R + at);
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
-                            v[2 * e] = round_bf16(v[2 * e]) + __uint_as_float(rr[e] << 16);
-                            v[2 * e + 1] = round_bf16(v[2 * e + 1]) + __uint_as_float(rr[e] & 0xffff0000u);
+                            v[2 * e] = bf16_round_hw(v[2 * e]) + __uint_as_float(rr[e] << 16);
+                            v[2 * e + 1] = bf16_round_hw(v[2 * e + 1]) + __uint_as_float(rr[e] & 0xffff0000u);
                         }
                     }
-                    u32x4 o;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) o[e] = pack_bf16(v[2 * e], v[2 * e + 1]);
-                    *reinterpret_cast<u32x4*>(p.Y + at) = o;
+                    *reinterpret_cast<u32x4*>(p.Y + at) = pack_bf16x8(v);
                 }
             }
         }

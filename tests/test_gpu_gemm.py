@@ -590,3 +590,47 @@ def test_tilings_that_do_not_exist_force_nothing(gpu_lib, tunables, tile):
     assert torch.isfinite(seen[0][0].float()).all()
     assert torch.equal(seen[0][0], seen[1][0]) and torch.equal(seen[0][1], seen[1][1])
     assert seen[0][2] == seen[1][2]
+
+
+@pytest.mark.parametrize("m,n,k", [(256, 320, 256), (1, 98304, 4096)])
+def test_wide_kernel_special_values(gpu_lib, tunables, m, n, k):
+    """NaN of any sign and payload, infinities and signed zeros in the
+    residual, the tokens and the weights: the wide kernel's bits are the
+    weight-stream kernel's (every NaN as 0x7fc0), in the residual and the
+    SwiGLU stores."""
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    special = torch.tensor([0x7fc0, 0xffc1 - 65536, 0x7f81, 0xff93 - 65536, 0x7f80, 0xff80 - 65536,
+                            0x8000 - 65536, 0x0001], dtype=torch.int16, device="cuda")
+
+    def normal(shape, scale=1.0):
+        return (torch.randn(shape, generator=g, device="cuda") * scale).to(torch.bfloat16)
+
+    def sprinkle(t, every):
+        flat = t.view(torch.int16).view(-1)
+        at = torch.arange(3, flat.numel(), every, device="cuda")
+        flat[at] = special[torch.arange(at.numel(), device="cuda") % 8]
+        return t
+
+    s = torch.cuda.current_stream().cuda_stream
+    x, w, r = normal((m, k)), normal((n, k), 0.02), sprinkle(normal((m, n)), 37)
+    if m > 1:
+        sprinkle(x[m // 2:], 8 * k + 5)   # some tokens and some weight rows
+        sprinkle(w[n // 2:], 16 * k + 3)
+        tunables.setenv("KCMM_GEMM_TILE", "104")
+        tunables.setenv("KCMM_GEMM_SPLITS", "1")
+    seen = []
+    for tiled in ("0", "1"):
+        tunables.setenv("KCMM_GEMM_TILED", tiled)
+        y = r.clone()
+        gpu_lib.gemm_bf16_add(x.data_ptr(), w.data_ptr(), y.data_ptr(), y.data_ptr(), m, n, k, s)
+        act = torch.zeros((m, n // 2), dtype=torch.bfloat16, device="cuda")
+        gpu_lib.gemm_bf16_swiglu(x.data_ptr(), w.data_ptr(), act.data_ptr(), m, n // 2, k, s)
+        torch.cuda.synchronize()
+        seen.append((y.view(torch.int16), act.view(torch.int16)))
+    (y0, a0), (y1, a1) = seen
+    print(f"special values {m}x{n}x{k}: {int((y0 != y1).sum())} and {int((a0 != a1).sum())} differ",
+          flush=True)
+    assert bool(y0.view(torch.bfloat16).isnan().any()) and bool((y0 == 0x7fc0).any())
+    assert torch.equal(y0, y1) and torch.equal(a0, a1)
