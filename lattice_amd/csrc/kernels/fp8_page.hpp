@@ -31,12 +31,17 @@ __device__ __forceinline__ uint32_t f32_to_fp8e4m3(float x) {
     return sign | code;
 }
 
-// x / scale clamped to the e4m3 range, for 2^-100 <= scale <= 2^100, r = 1 /
+// x / scale clamped to the e4m3 range, for scales in the range below, r = 1 /
 // scale and x not NaN: x * r with one residual step is the correctly rounded
 // quotient wherever it matters to four significant bits (Markstein's division;
-// checked against x / scale for every bf16 x and 32639 scales).  The hardware
-// conversion of it gives the bits of f32_to_fp8e4m3(x / scale) (the two agree
-// on every float but NaN, whose sign the hardware does not keep).
+// tests/test_fp8_quotient.py sweeps it against x / scale).  Its callers pass
+// any bf16 value up to 448 * scale, or a stored code's value times an older,
+// smaller scale -- 24 significant bits, so the residual of a quotient of 2^-11
+// and more has bits down to 2^-57 * scale, which the lower bound keeps above
+// the smallest float (at 2^-100 a few codes fell to the neighbour of a tie).
+// The hardware conversion gives the bits of f32_to_fp8e4m3 (the two agree on
+// every float but NaN, whose sign the hardware does not keep).
+constexpr float kFp8QuotientMin = 0x1p-80f, kFp8QuotientMax = 0x1p100f;
 __device__ __forceinline__ float fp8_quotient(float x, float scale, float r) {
     const float q = x * r;
     return __builtin_amdgcn_fmed3f(copysignf(fmaf(fmaf(-q, scale, x), r, q), x), -448.0f, 448.0f);
@@ -144,8 +149,8 @@ __device__ __forceinline__ void fp8_write_page_head(uint8_t* page, uint32_t kvh,
         scale = old;
         if (amax > 448.0f * old) {
             scale = amax / 448.0f;
-            if ((head_dim & 15) == 0 && (row_bytes & 15) == 0 && scale >= 0x1p-100f &&
-                scale <= 0x1p100f) {
+            if ((head_dim & 15) == 0 && (row_bytes & 15) == 0 && scale >= kFp8QuotientMin &&
+                scale <= kFp8QuotientMax) {
                 // 16-byte pieces of all unwritten slots at once: one memory
                 // round trip for the page instead of one per slot
                 const uint32_t pieces = head_dim / 16;
@@ -194,7 +199,7 @@ __device__ __forceinline__ void fp8_write_page_head(uint8_t* page, uint32_t kvh,
             }
         }
     }
-    if (vec && !__any(nan) && scale >= 0x1p-100f && scale <= 0x1p100f) {
+    if (vec && !__any(nan) && scale >= kFp8QuotientMin && scale <= kFp8QuotientMax) {
         const float r = 1.0f / scale;
         uint8_t* base = page + kvh * head_dim;
 #pragma unroll 1
