@@ -833,7 +833,9 @@ bool gemm_bf16_add_rmsnorm(uint64_t x, uint64_t w, uint64_t hidden, uint64_t nor
                            std::string* err) {
     float* part = nullptr;
     int splits = 1;
-    if (m > 128 && dev::tunable_or(dev::Tun::kGemmTiled, 1) != 0) {
+    // x may lie in hidden: its rows are then read before any is written
+    const bool apart = x + 2ull * m * k <= hidden || hidden + 2ull * m * n <= x;
+    if (m > 128 && apart && dev::tunable_or(dev::Tun::kGemmTiled, 1) != 0) {
         // many tokens: as gemm_bf16 with the residual (an unsplit product
         // adds it in its own store), its split sum left to the RMSNorm kernel
         if (!shape_ok(m, n, k, err) ||

@@ -155,3 +155,26 @@ def test_add_rmsnorm_matches_unfused(gpu_lib, tunables, m, n, k):
     torch.cuda.synchronize()
     assert np.array_equal(_bits(h), _bits(h_ref))
     assert np.array_equal(_bits(y), _bits(y_ref))
+
+
+@pytest.mark.parametrize("m", [100, 200, 2048])
+def test_add_rmsnorm_of_the_hidden_rows_themselves(gpu_lib, tunables, m):
+    """x may be the hidden rows (n == k): every product reads them as they
+    were before the call, at all token counts."""
+    import torch
+    n = 4096
+    w = _randn_bf16(torch, (n, n), 0.02, 22)
+    nw = _randn_bf16(torch, (n,), 1.0, 24)
+    h0 = _randn_bf16(torch, (m, n), 1.0, 23)
+    sp = torch.cuda.current_stream().cuda_stream
+    seen = []   # x apart on the weight-stream kernel, then x = hidden: the same kernel and bits
+    for tiled in ("0", "1"):
+        tunables.setenv("KCMM_GEMM_TILED", tiled)
+        h, y = h0.clone(), torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+        x = h0.clone() if tiled == "0" else h
+        gpu_lib.gemm_bf16_add_rmsnorm(x.data_ptr(), w.data_ptr(), h.data_ptr(), nw.data_ptr(),
+                                      y.data_ptr(), m, n, n, 1e-5, sp)
+        torch.cuda.synchronize()
+        seen.append((h, y))
+    assert np.array_equal(_bits(seen[0][0]), _bits(seen[1][0]))
+    assert np.array_equal(_bits(seen[0][1]), _bits(seen[1][1]))
