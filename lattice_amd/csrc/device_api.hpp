@@ -51,12 +51,15 @@ void reload_tunables();
 // graph capture: run each shape once before capturing it.
 bool stream_workspace(uint64_t stream, int slot, size_t bytes, void** out, bool zero_fill,
                       std::string* err);
-// Whether a call that can also run without scratch may take `bytes` of it.
-// Not under a capture: the graph would keep the address of a buffer that a
-// later growth, or the thread's exit, frees, and two graphs replayed on two
-// streams would share it.  (`in_capture`: the call's other variant needs the
-// scratch too; under a capture it may then use a buffer that is large enough.)
-bool stream_scratch(uint64_t stream, int slot, size_t bytes, bool in_capture = false);
+// For a call that can also run without scratch: whether stream_workspace now
+// hands out `bytes` (the buffer is grown here if need be).  Not where memory is
+// short, and not under a capture: the graph would keep the address of a buffer
+// that a later growth, or the thread's exit, frees, and two graphs replayed on
+// two streams would share it.  (`in_capture`: the call's other variant needs
+// the scratch too; under a capture it may then use a buffer that is large
+// enough.)  Growing does not disturb a capture on another thread.
+bool stream_scratch(uint64_t stream, int slot, size_t bytes, bool in_capture = false,
+                    bool zero_fill = false);
 // Buffers of exited threads are freed by the next workspace allocation;
 // this frees them now (device synchronize first).  Count of those pending.
 bool release_orphaned_workspaces(std::string* err);

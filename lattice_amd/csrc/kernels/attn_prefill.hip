@@ -845,7 +845,9 @@ bool launch_mfma(const dev::AttnPrefillArgs& a, PrefillParams& p, hipStream_t s,
     const size_t cols = static_cast<size_t>(busy) * std::max(splits, 1) * NW * NCB * 16;
     const size_t part_bytes = cols * (D + 2) * sizeof(float);
     const size_t count_bytes = static_cast<size_t>(busy) * 4 * sizeof(int32_t);
-    if (splits > 1 && !dev::stream_scratch(a.stream, 5, part_bytes)) splits = 1;
+    if (splits > 1 && !(dev::stream_scratch(a.stream, 5, part_bytes) &&
+                        dev::stream_scratch(a.stream, 9, count_bytes, false, true)))
+        splits = 1;
     const dim3 grid(static_cast<unsigned>(splits > 1 ? busy : blocks), splits > 1 ? splits : 1);
     auto run = [&](auto split) {
         hipLaunchKernelGGL((attn_prefill_mfma<DT, D, G, NW, NCB, KT, decltype(split)::value>), grid,

@@ -203,15 +203,17 @@ bool free_orphans_locked(std::string* err) {
 
 }  // namespace
 
-bool stream_workspace(uint64_t stream, int slot, size_t bytes, void** out, bool zero_fill,
-                      std::string* err) {
+namespace {
+// `orphans`: free those of exited threads first (which synchronizes the device).
+bool workspace(uint64_t stream, int slot, size_t bytes, void** out, bool zero_fill, bool orphans,
+               std::string* err) {
     (void)&t_ws_owner;   // registers this thread's owner (its destructor runs at thread exit)
     int dev = 0;
     KCMM_HIP_CHECK(hipGetDevice(&dev), err);
     std::lock_guard<std::mutex> lk(ws_mutex());
     Ws& w = ws_table()[std::make_tuple(dev, stream, slot, std::this_thread::get_id())];
     if (w.bytes < bytes) {
-        if (!free_orphans_locked(err)) return false;
+        if (orphans && !free_orphans_locked(err)) return false;
         if (w.ptr) {
             KCMM_HIP_CHECK(hipStreamSynchronize(reinterpret_cast<hipStream_t>(stream)), err);
             KCMM_HIP_CHECK(hipFree(w.ptr), err);
@@ -233,19 +235,38 @@ bool stream_workspace(uint64_t stream, int slot, size_t bytes, void** out, bool 
     *out = w.ptr;
     return true;
 }
+}  // namespace
 
-bool stream_scratch(uint64_t stream, int slot, size_t bytes, bool in_capture) {
+bool stream_workspace(uint64_t stream, int slot, size_t bytes, void** out, bool zero_fill,
+                      std::string* err) {
+    return workspace(stream, slot, bytes, out, zero_fill, true, err);
+}
+
+bool stream_scratch(uint64_t stream, int slot, size_t bytes, bool in_capture, bool zero_fill) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(reinterpret_cast<hipStream_t>(stream), &cs) != hipSuccess) {
         (void)hipGetLastError();   // (the null stream while another one is captured)
         return false;
     }
-    if (cs == hipStreamCaptureStatusNone) return true;
+    const bool capturing = cs != hipStreamCaptureStatusNone;
+    if (capturing && !in_capture) return false;
     int dev = 0;
-    if (!in_capture || hipGetDevice(&dev) != hipSuccess) return false;
-    std::lock_guard<std::mutex> lk(ws_mutex());
-    const auto it = ws_table().find(std::make_tuple(dev, stream, slot, std::this_thread::get_id()));
-    return it != ws_table().end() && it->second.bytes >= bytes;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    {
+        std::lock_guard<std::mutex> lk(ws_mutex());
+        const auto it = ws_table().find(std::make_tuple(dev, stream, slot, std::this_thread::get_id()));
+        if (it != ws_table().end() && it->second.bytes >= bytes) return true;
+    }
+    if (capturing) return false;
+    // an allocation, or a device synchronization for the orphans, may break a
+    // capture that another thread has begun
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    void* p = nullptr;
+    std::string why;
+    const bool ok = workspace(stream, slot, bytes, &p, zero_fill, false, &why);
+    if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return ok;
 }
 
 bool release_orphaned_workspaces(std::string* err) {

@@ -369,3 +369,50 @@ def test_decode_workgroups_in_wide_tables(gpu_lib, dtype, ctx, tokens, waves):
         assert torch.isfinite(seen[0].float()).all() and torch.equal(seen[0], seen[1])
     finally:
         case.pool.destroy()
+
+
+@pytest.mark.parametrize("what", ["prefill", "uneven", "wide"])
+def test_first_call_beside_another_threads_capture(gpu_lib, what):
+    """A thread's first calls on its stream (its scratch grows twice), while another thread captures a
+    graph (in the mode that forbids allocations on all threads): the scratch
+    that it would take is no reason to fail or to break that capture."""
+    import threading
+    import torch
+    run, run_more, out, close = _scratch_free_work(torch, gpu_lib, what)
+    try:
+        x = torch.zeros(64, device="cuda")
+        (x + 1.0).sum()                                   # torch's kernels are loaded
+        st, gs = torch.cuda.Stream(), torch.cuda.Stream()
+        run(torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        want = out.clone()
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        failed = []
+        run_more(torch.cuda.current_stream().cuda_stream)   # (every kernel is loaded)
+        torch.cuda.synchronize()
+
+        def first_call():
+            try:
+                for call in (run, run_more, run):
+                    call(st.cuda_stream)
+            except Exception as e:                        # noqa: BLE001 (re-raised below)
+                failed.append(e)
+
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=gs, capture_error_mode="global"):
+            x.add_(1.0)
+            t = threading.Thread(target=first_call)
+            t.start()
+            t.join()
+            x.add_(1.0)
+        assert not failed, failed
+        torch.cuda.synchronize()
+        for _ in range(3):
+            graph.replay()
+        torch.cuda.synchronize()
+        assert float(x[0]) == 6.0
+        d = (out.double() - want.double()).norm() / want.double().norm()
+        assert float(d) <= 1e-2                           # (maybe in another order of the sums)
+    finally:
+        close()
