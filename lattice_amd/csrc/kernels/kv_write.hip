@@ -155,20 +155,29 @@ __device__ __forceinline__ int64_t block_of(const SlotArgs& a, int64_t slot) {
 // order) and dropping a page that an earlier row names.  The waves then take
 // the (page, kv head, K|V) triples of the pages left.
 //
-// R = 1 up to 512 rows (a decode step's appends: every row has its own page),
-// else 16 (a prompt's rows fill a page each): 4507 prompt rows, 16 slots per
-// page, took 381 us with one workgroup per row, a serial walk over the rows of
-// a page and a separate pass that counted them (9 us); 21 us so, most of it
-// the walk over the slot ids and the chain of loads behind it.  A single row's
-// append in a decode step 16 -> 7 us.
+// R gives every CU one workgroup of up to 16 waves: a prompt's rows fill a page
+// each and want R near the page's rows, a decode step's have a page each and
+// want as many waves as the chip holds, and the host cannot tell them apart.
+// One workgroup per row, a serial walk over a page's rows and a pass that
+// counted them (9 us) before / R = 16 with 8 waves above 512 rows / so, us, 8 kv
+// heads, 16-slot pages: 600 prompt rows 57 / 15.9 / 9.6, 2400 290 / 13.1 / 11.2,
+// 4500 359 / 21.1 / 18.3, 8100 648 / 27.0 / 24.7; one row per page, 600 rows 27.5
+// / 79 / 16.8, 2000 66 / 84 / 37, 8000 237 / 162 / 128 (2 kv heads 58 / 82 / 44).
+// The pages are found through a hash table: comparing each slot id with up to
+// 32 of them took most of the time of 8000 rows (2 kv heads 86 us).
 //
 // A call of more than kFp8ScanRows rows would spend its time walking the
 // slot ids (every workgroup walks all): `lead` / `cnt` (int32 per block id,
 // zero between calls) then collect, per page, batch - (first row) and the
 // number of rows, and a workgroup walks from its own rows on until it has
-// them all.
+// them all; R = 12 with 4 waves there (9000 rows with a page each, 8 / 2 kv
+// heads: 146 / 48 us, with 16 and 8 183 / 70; 12000 prompt rows 39 and 37).
 constexpr uint32_t kFp8ScanRows = 8192;
-constexpr uint32_t kFp8RowsPerGroup = 16;
+constexpr uint32_t kFp8RowsPerGroup = 32;
+constexpr uint32_t kFp8Slots = 256;   // of the hash table that finds a workgroup's pages by block id
+__device__ __forceinline__ uint32_t fp8_hash(int32_t id) {
+    return (static_cast<uint32_t>(id) * 0x9E3779B1u) >> 24;
+}
 
 __global__ __launch_bounds__(256) void kv_slots_fp8_collect(SlotArgs a, uint32_t batch,
                                                             int32_t* lead, int32_t* cnt) {
@@ -192,6 +201,7 @@ __global__ __launch_bounds__(64 * kFp8MaxWaves) void kv_slots_fp8_write(SlotArgs
     __shared__ int32_t s_id[kFp8RowsPerGroup];           // the list: block ids
     __shared__ int32_t s_left[kFp8RowsPerGroup];         // collected: rows not found yet
     __shared__ int32_t s_dead[kFp8RowsPerGroup];         // an earlier row leads the page
+    __shared__ int32_t s_key[kFp8Slots], s_page[kFp8Slots];   // block id (-1: free) -> place in the list
     __shared__ int32_t s_pages;
     const uint32_t r0 = blockIdx.x * R, t = threadIdx.x;
     const uint32_t bs = a.block_size;
@@ -214,12 +224,19 @@ __global__ __launch_bounds__(64 * kFp8MaxWaves) void kv_slots_fp8_write(SlotArgs
             first = __atomic_load_n(lead + id, __ATOMIC_RELAXED) == static_cast<int32_t>(batch - r0 - t);
             if (first) rows = __atomic_load_n(cnt + id, __ATOMIC_RELAXED);
         }
+        for (uint32_t i = t; R > 1 && i < kFp8Slots; i += 64) s_key[i] = -1;
+        __builtin_amdgcn_wave_barrier();
         const uint64_t m = __ballot(first);
         if (first) {
             const int at = __popcll(m & ((1ull << t) - 1));
             s_id[at] = id;
             s_left[at] = rows;
             s_dead[at] = 0;
+            if (R > 1) {
+                uint32_t h = fp8_hash(id);   // (at most kFp8RowsPerGroup of them: a free one is near)
+                while (atomicCAS(s_key + h, -1, id) != -1) h = (h + 1) % kFp8Slots;
+                s_page[h] = at;
+            }
         }
         if (t == 0) s_pages = __popcll(m);
     }
@@ -243,16 +260,23 @@ __global__ __launch_bounds__(64 * kFp8MaxWaves) void kv_slots_fp8_write(SlotArgs
             if (slot[i] < 0) continue;
             const uint32_t rr = base + t + i * nt;
             const int64_t id = block_of(a, slot[i]);
-            for (int j = 0; j < pages; ++j) {
-                if (__builtin_amdgcn_readfirstlane(s_id[j]) != id) continue;
-                // (a page dropped here may still be entered by others: its
-                // table is not used)
-                if (rr < r0) s_dead[j] = 1;
-                atomicMax(row_of + j * bs + static_cast<uint32_t>(slot[i] - id * bs),
-                          static_cast<int32_t>(rr));
-                if (lead != nullptr) atomicSub(s_left + j, 1);
-                break;
+            if (id >= static_cast<int64_t>(a.offsets_len)) continue;
+            int j = 0;
+            if (R == 1) {
+                if (id != s_id[0]) continue;
+            } else {
+                uint32_t h = fp8_hash(static_cast<int32_t>(id));
+                int32_t key = s_key[h];
+                while (key != id && key != -1) key = s_key[h = (h + 1) % kFp8Slots];
+                if (key == -1) continue;
+                j = s_page[h];
             }
+            // (a page dropped here may still be entered by others: its table
+            // is not used)
+            if (rr < r0) s_dead[j] = 1;
+            atomicMax(row_of + j * bs + static_cast<uint32_t>(slot[i] - id * bs),
+                      static_cast<int32_t>(rr));
+            if (lead != nullptr) atomicSub(s_left + j, 1);
         }
         if (lead != nullptr) {
             __syncthreads();
@@ -421,11 +445,13 @@ bool kv_write_device_slots(const KvDeviceSlotsArgs& a, std::string* err) {
                                sa, a.batch, lead, cnt);
             KCMM_HIP_CHECK(hipGetLastError(), err);
         }
-        const uint32_t R =
-            a.batch <= 512 ? 1
-                           : std::max(1u, std::min(kFp8RowsPerGroup, kFp8MaxBlockSize / a.block_size));
-        // (8 waves: two workgroups fit a CU, so a prompt's are one round)
-        const uint32_t waves = R > 1 ? 8u : std::min<uint32_t>(2 * a.kv_heads, kFp8MaxWaves);
+        // (the slot tables of R pages take the LDS of one page of kFp8MaxBlockSize)
+        // Up to 512 rows of at most 4 kv heads the chip holds a workgroup per row.
+        const bool single = a.batch <= 512 && a.kv_heads <= 4;
+        const uint32_t R = std::max(1u, std::min({lead != nullptr ? 12u : single ? 1u : (a.batch + 255) / 256,
+                                                  kFp8RowsPerGroup, kFp8MaxBlockSize / a.block_size}));
+        const uint32_t most = lead != nullptr ? 4u : (a.batch + R - 1) / R > 256 ? 8u : kFp8MaxWaves;
+        const uint32_t waves = std::min(2 * a.kv_heads * R, most);
         hipLaunchKernelGGL(kv_slots_fp8_write, dim3((a.batch + R - 1) / R), dim3(64 * waves),
                            static_cast<size_t>(R) * a.block_size * 4, s, sa, a.batch, R, lead, cnt);
     } else {

@@ -334,7 +334,7 @@ def test_fp8_device_slots_status_and_repeat_calls(gpu_lib):
                                              (520, (2, 20, 512), 1)],
                          ids=["r600", "r513-d72", "r700-bs64", "r9001-collected", "r520-d20-bs512"])
 def test_fp8_prompt_rows_bytes(gpu_lib, rows, geom, first):
-    """Calls of more than 512 rows (16 rows per workgroup), of more than 8192
+    """Calls of more than 512 rows (several rows per workgroup), of more than 8192
     (rows counted per page first), head_dim not a multiple of 8 and
     misaligned sources (element-wise path), two calls on the same pages (the
     second raises scales, so unwritten slots are re-encoded), a few repeated
@@ -392,6 +392,64 @@ def test_fp8_prompt_rows_bytes(gpu_lib, rows, geom, first):
             assert int(st.item()) in want, (call, int(st.item()))
             O.kv_write_device_slots(KV_FP8, ok, ov, bits[0], bits[1], slots, offs, valid, bs, hk, d,
                                     g_row, data_bytes)
+            gk, gv = region_bytes(pool)
+            assert np.array_equal(gk, ok), f"K after call {call}"
+            assert np.array_equal(gv, ov), f"V after call {call}"
+    finally:
+        pool.destroy()
+
+
+@pytest.mark.parametrize("rows,hk,bs", [(257, 5, 8), (257, 2, 8), (513, 1, 8), (1100, 1, 16),
+                                        (4097, 2, 8), (8192, 1, 8), (8193, 1, 8), (1500, 1, 256)])
+def test_fp8_rows_of_many_pages_bytes(gpu_lib, rows, hk, bs):
+    """Calls whose rows mostly have a page each (a decode step of many
+    sequences): up to 32 pages per workgroup, found by block id, and 12 where
+    the rows are counted first; shuffled, with some pages named by several
+    rows far apart, slots written twice, padding, an id past the table, huge
+    slot values and an inactive id; a second call raises the scales.  Every
+    byte as the oracle's."""
+    import torch
+    rng = np.random.default_rng(rows + hk)
+    d = 64
+    pool = gpu_lib.create_pool(make_config(num_layers=1, kv_heads=hk, head_dim=d, max_batch=rows,
+                                           max_seq_len=bs, block_size=bs), KV_FP8)
+    try:
+        ids = []
+        while len(ids) < rows:
+            ids += pool.alloc_blocks(min(4096, rows - len(ids)))
+        ids = rng.permutation(np.asarray(ids, dtype=np.int64))
+        zero_regions(pool)
+        nb = pool.stats()["superblock_count"] * SB
+        ok, ov = np.zeros(nb, np.uint8), np.zeros(nb, np.uint8)
+        offs = np.asarray(pool.all_block_offsets_f16(), np.uint64)
+        offs_t = torch.from_numpy(offs.view(np.int64)).cuda()
+        valid = np.ones(len(offs), np.uint8)
+        valid[ids[rows // 2]] = 0
+        valid_t = torch.from_numpy(valid).cuda()
+        for call in range(2):
+            slots = ids * bs + rng.integers(bs, size=rows)
+            for _ in range(20):                       # pages and slots of other rows
+                i, j = rng.integers(rows, size=2)
+                slots[i] = slots[j] // bs * bs + rng.integers(bs)
+                i, j = rng.integers(rows, size=2)
+                slots[i] = slots[j]
+            slots[rng.integers(rows, size=6)] = [-1, -1, len(offs) * bs, (1 << 32) * bs + 3,
+                                                 (1 << 62) + 5, -7]
+            bits = O.encode(O.BF16, (rng.standard_normal((2, rows, hk * d)) * 4.0 ** call)
+                            .astype(np.float32))
+            k, v = (torch.from_numpy(b.view(np.int16)).cuda() for b in bits)
+            sl = torch.from_numpy(slots).cuda()
+            st = torch.zeros(1, dtype=torch.int32, device="cuda")
+            stream = torch.cuda.current_stream()
+            pool.append_kv_device_slots_on_stream(
+                layer_idx=0, slot_mapping_ptr=sl.data_ptr(), block_offsets_f16_ptr=offs_t.data_ptr(),
+                valid_blocks_ptr=valid_t.data_ptr(), block_offsets_f16_len=len(offs), batch=rows,
+                k_src_ptr=k.data_ptr(), v_src_ptr=v.data_ptr(), status_ptr=st.data_ptr(),
+                stream_ptr=stream.cuda_stream)
+            stream.synchronize()
+            assert int(st.item()) in (1, 2)
+            O.kv_write_device_slots(KV_FP8, ok, ov, bits[0], bits[1], slots, offs, valid, bs, hk, d,
+                                    hk * d, hk * d * bs)
             gk, gv = region_bytes(pool)
             assert np.array_equal(gk, ok), f"K after call {call}"
             assert np.array_equal(gv, ov), f"V after call {call}"
