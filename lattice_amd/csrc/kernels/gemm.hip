@@ -517,51 +517,76 @@ __global__ __launch_bounds__(256) void gemm_split_swiglu(const float* __restrict
 // K splits: the smallest divisor of K/kch giving at least `target` workgroups
 // (KCMM_GEMM_WGS, default 256: fewer, longer splits measured faster than
 // 512-1024 at the Llama-3-8B decode shapes) with each split at least two
-// chunks long; at most 16.  A split that gives 7/8 of the target is taken
-// too: one round with a few idle CUs beats a second round (one token, bf16,
-// more -> fewer splits: 5120 x 3072 at 4 -> 3 10.9 -> 9.7 us, 7680 x 2560 at
-// 5 -> 2 13.9 -> 10.6, 5120 x 13824 at 6 -> 3 25.2 -> 25.6; 64 tokens 17.1 ->
-// 13.1, 20.0 -> 14.8, 38.4 -> 34.2).  Not unsplit: 15360 x 5120 40.6 us
-// unsplit, 27.4 at 2.  Where the divisors leave more than a quarter of the
-// target empty (K / kch prime, or twice a prime), the last split may be
-// shorter than the others: the smallest count that is enough with no split
-// empty (one token, bf16, equal -> uneven splits: 4096 x 11008 at 1 -> 4
-// splits 79 -> 19.6 us, 1024 x 2816 at 1 -> 6 22.3 -> 7.6, 3584 x 18944 at
-// 2 -> 4 38.7 -> 25.2; 64 tokens 99 -> 25.3, 27.6 -> 9.0, 58 -> 35).
-int choose_splits(int N, int K, int kch, int mgroups, bool equal) {
+// chunks long; at most 16.  Where that divisor goes past the target and the
+// one before it gives 7/8 of it, the one before: one round with a few idle
+// CUs beats a second round (one token, bf16, more -> fewer splits: 5120 x 3072
+// at 4 -> 3 10.9 -> 9.7 us, 7680 x 2560 at 5 -> 2 13.9 -> 10.6, 5120 x 13824 at
+// 6 -> 3 25.2 -> 25.6; 64 tokens 17.1 -> 13.1, 20.0 -> 14.8, 38.4 -> 34.2); not
+// the unsplit one (15360 x 5120 40.6 us unsplit, 27.4 at 2), and not below a
+// divisor that meets the target (2048 x 14336, 65 tokens: 21.7 us at 8, 23.3 at
+// 7).  Where the divisors leave more than a quarter of the target empty (K /
+// kch prime, or twice a prime), the last split may be shorter than the others:
+// as many as fit one round, if the longest split with the cost of the split sum
+// (that of about 512 elements) is a fifth shorter than the divisor's (one token,
+// bf16, equal -> uneven splits: 4096 x 11008 at 1 -> 4 splits 79 -> 19.6 us,
+// 1024 x 2816 at 1 -> 6 22.3 -> 7.6, 3584 x 18944 at 2 -> 4 38.7 -> 25.2; 64 tokens
+// 99 -> 25.3, 27.6 -> 9.0, 58 -> 35; not 11008 x 11008, 55.5 unsplit and 61 at 2,
+// nor 9024 x 768 with fp8 weights, 5.4 and 7.1).
+int choose_splits(int N, int K, int kch, int mgroups, int* equal) {
     const int chunks = K / kch;
     const int forced = dev::tunable_or(dev::Tun::kGemmSplits, 0);
-    if (forced >= 1 && forced <= 16 && chunks % forced == 0) return forced;
+    if (forced >= 1 && forced <= 16 && chunks % forced == 0) return *equal = forced;
     const int target = dev::tunable_or(dev::Tun::kGemmWgs, 256);
     const int tiles = (N / 64) * mgroups;
-    auto enough = [&](int s) { return tiles * s >= target || (s > 1 && 8 * tiles * s >= 7 * target); };
-    int best = 1;
+    int best = 1, before = 1;
     for (int s = 1; s <= std::min(chunks, 16); ++s) {
         if (chunks % s) continue;
         if (chunks / s < 2 && s > 1) break;
+        before = best;
         best = s;
-        if (enough(s)) break;
+        if (tiles * s >= target) break;
     }
-    if (equal || 4 * tiles * best >= 3 * target) return best;
-    for (int s = best + 1; s <= 16; ++s) {
+    if (before > 1 && tiles * best > target && 8 * tiles * before >= 7 * target) best = before;
+    *equal = best;
+    if (4 * tiles * best >= 3 * target) return best;
+    auto cost = [&](int s) { return (chunks + s - 1) / s + (s > 1 ? std::max(1, 512 / kch) : 0); };
+    int uneven = best;
+    for (int s = best + 1; s <= 16 && tiles * s <= target; ++s) {
         const int per = (chunks + s - 1) / s;
         if (per < 2) break;
-        if ((s - 1) * per >= chunks) continue;
-        best = s;
-        if (enough(s)) break;
+        if ((s - 1) * per < chunks && cost(s) < cost(uneven)) uneven = s;
     }
-    return best;
+    return 5 * cost(uneven) < 4 * cost(best) ? uneven : best;
 }
 
-// Tile shape by M: token blocks per pass (the activation chunk, M x KCH
-// bf16, is 32 KiB).
-// fp8 weights need at least 128-element chunks (one 128-byte weight line);
-// up to 16 tokens they take 512-element ones, as many weight bytes in flight
-// as bf16's 256 (M = 1: 28672 x 4096 26.4 -> 23.6 us, 4096 x 14336 15.7 -> 14.2;
-// bf16 at 512: 43 -> 47; fp8 at 64 tokens was slower with them).
+// Chunk length and K splits of a product: chunks by M (the activation chunk,
+// M x kch bf16, is 32 KiB).  fp8 weights need at least 128-element chunks (one
+// 128-byte weight line); up to 16 tokens they take 512-element ones, as many
+// weight bytes in flight as bf16's 256 (one token: 28672 x 4096 25.4 -> 23.1 us,
+// 4096 x 14336 15.9 -> 14.2; bf16 at 512: 43 -> 47; fp8 at 64 tokens was slower
+// with them).  Not where they leave fewer K splits (2048 x 2048 at 4 splits of
+// 256 6.5 us, at 2 of 512 7.2) or few chunks (128256 x 512 15.0 -> 19.8), and
+// not for split products of more than one round of workgroups, which fit a CU
+// twice with the shorter ones (11008 x 14336 at 2 splits 33.6 -> 35.0).
+struct StreamPlan {
+    int kch, splits;
+    int equal;   // the splits without uneven ones
+};
+StreamPlan stream_plan(int M, int N, int K, bool wf8) {
+    StreamPlan p{M <= 64 ? 256 : M <= 128 || wf8 ? 128 : 64, 1, 1};
+    const int rows = M <= 16 ? 16 : M <= 32 ? 32 : M <= 64 ? 64 : M <= 128 ? 128 : 256;
+    p.splits = choose_splits(N, K, p.kch, (M + rows - 1) / rows, &p.equal);
+    if (M <= 16 && wf8 && K % 512 == 0 && K >= 4096 &&
+        (p.splits == 1 || N / 64 * p.splits <= 256)) {
+        StreamPlan q{512, 1, 1};
+        q.splits = choose_splits(N, K, 512, 1, &q.equal);
+        if (q.splits == p.splits) return q;
+    }
+    return p;
+}
 template <typename F>
-bool by_m(int M, int K, F&& f, bool wf8 = false) {
-    if (M <= 16 && wf8 && K % 512 == 0)
+bool by_m(int M, const StreamPlan& p, F&& f, bool wf8) {
+    if (M <= 16 && p.kch == 512)
         return f(std::integral_constant<int, 1>{}, std::integral_constant<int, 512>{});
     if (M <= 16) return f(std::integral_constant<int, 1>{}, std::integral_constant<int, 256>{});
     if (M <= 32) return f(std::integral_constant<int, 2>{}, std::integral_constant<int, 256>{});
@@ -571,33 +596,24 @@ bool by_m(int M, int K, F&& f, bool wf8 = false) {
     return f(std::integral_constant<int, 16>{}, std::integral_constant<int, 64>{});
 }
 
-int splits_for(int M, int N, int K, bool wf8, bool equal = false) {
-    int s = 1;
-    by_m(M, K, [&](auto mb, auto kch) {
-        const int mgroups = (M + 16 * mb.value - 1) / (16 * mb.value);
-        s = choose_splits(N, K, kch.value, mgroups, equal);
-        return true;
-    }, wf8);
-    return s;
-}
-
-// splits_for a launch on `stream`.  A capture takes equal splits, which for
+// The plan for a launch on `stream`.  A capture takes equal splits, which for
 // most of the unevenly split shapes need no partials: no graph then holds the
 // address of a buffer that only the uneven split asked for.
-int splits_on(uint64_t stream, const GemmParams& p) {
-    const bool wf8 = p.wscale != nullptr;
-    const int s = splits_for(p.M, p.N, p.K, wf8);
-    const int e = splits_for(p.M, p.N, p.K, wf8, true);
-    const size_t bytes = static_cast<size_t>(s) * p.M * p.N * sizeof(float);
-    return s == e || dev::stream_scratch(stream, 1, bytes) ? s : e;
+StreamPlan plan_on(uint64_t stream, const GemmParams& p) {
+    StreamPlan plan = stream_plan(p.M, p.N, p.K, p.wscale != nullptr);
+    if (plan.splits != plan.equal &&
+        !dev::stream_scratch(stream, 1, static_cast<size_t>(plan.splits) * p.M * p.N * sizeof(float)))
+        plan.splits = plan.equal;
+    return plan;
 }
 
-// Launch the streaming kernel with `splits` K splits; splits > 1 or
+// Launch the streaming kernel with the plan's K splits; splits > 1 or
 // want_partials writes fp32 partials [splits][M][N] to the stream's workspace
 // (returned in *part) instead of running the epilogue.
 template <int EPI, bool WF8 = false>
-bool launch_stream(GemmParams p, int splits, bool want_partials, float** part, uint64_t stream,
-                   std::string* err) {
+bool launch_stream(GemmParams p, const StreamPlan& plan, bool want_partials, float** part,
+                   uint64_t stream, std::string* err) {
+    const int splits = plan.splits;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     p.part = nullptr;
     if (splits > 1 || want_partials) {
@@ -608,7 +624,7 @@ bool launch_stream(GemmParams p, int splits, bool want_partials, float** part, u
         p.part = static_cast<float*>(ws);
     }
     if (part) *part = p.part;
-    return by_m(p.M, p.K, [&](auto mb, auto kch) {
+    return by_m(p.M, plan, [&](auto mb, auto kch) {
         constexpr int MB = decltype(mb)::value, KCH = decltype(kch)::value;
         p.klen = (p.K / KCH + splits - 1) / splits * KCH;
         if constexpr (!WF8 && KCH > 256) {
@@ -677,11 +693,11 @@ bool launch_stream(GemmParams p, int splits, bool want_partials, float** part, u
 
 // launch_stream on bf16 weights, or on fp8-e4m3 weights when p.wscale is set
 template <int EPI>
-bool launch_weights(const GemmParams& p, int splits, bool want_partials, float** part,
+bool launch_weights(const GemmParams& p, const StreamPlan& plan, bool want_partials, float** part,
                     uint64_t stream, std::string* err) {
     if (p.wscale != nullptr)
-        return launch_stream<EPI, true>(p, splits, want_partials, part, stream, err);
-    return launch_stream<EPI>(p, splits, want_partials, part, stream, err);
+        return launch_stream<EPI, true>(p, plan, want_partials, part, stream, err);
+    return launch_stream<EPI>(p, plan, want_partials, part, stream, err);
 }
 
 bool shape_ok(uint32_t m, uint32_t n, uint32_t k, std::string* err) {
@@ -761,9 +777,10 @@ bool gemm_bf16(uint64_t x, uint64_t w, uint64_t y, uint32_t m, uint32_t n, uint3
     GemmParams p = base_params(x, w, m, n, k);
     p.Y = reinterpret_cast<uint16_t*>(y);
     p.R = reinterpret_cast<const uint16_t*>(residual);
-    const int splits = splits_on(stream, p);
+    const StreamPlan plan = plan_on(stream, p);
+    const int splits = plan.splits;
     float* part = nullptr;
-    if (!launch_stream<kEpiPlain>(p, splits, false, &part, stream, err)) return false;
+    if (!launch_stream<kEpiPlain>(p, plan, false, &part, stream, err)) return false;
     if (splits > 1) {
         const int MN = p.M * p.N;
         hipLaunchKernelGGL(gemm_split_reduce, dim3((MN / 4 + 255) / 256), dim3(256), 0,
@@ -786,8 +803,8 @@ bool gemm_plan(uint32_t m, uint32_t n, uint32_t k, bool fp8_weights, GemmPlan* p
         plan->tile = 100 + long_weights_fb(m);
     } else {
         plan->kernel = 0;
-        plan->splits = splits_for(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k),
-                                  fp8_weights);
+        plan->splits = stream_plan(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k),
+                                   fp8_weights).splits;
         plan->tile = -1;
     }
     plan->partial_bytes = plan->splits > 1
@@ -811,9 +828,10 @@ bool gemm_fp8w_bf16(uint64_t x, uint64_t w8, uint64_t wscale, uint64_t y, uint32
     p.Y = reinterpret_cast<uint16_t*>(y);
     p.R = reinterpret_cast<const uint16_t*>(residual);
     p.wscale = reinterpret_cast<const float*>(wscale);
-    const int splits = splits_on(stream, p);
+    const StreamPlan plan = plan_on(stream, p);
+    const int splits = plan.splits;
     float* part = nullptr;
-    if (!launch_stream<kEpiPlain, true>(p, splits, false, &part, stream, err)) return false;
+    if (!launch_stream<kEpiPlain, true>(p, plan, false, &part, stream, err)) return false;
     if (splits > 1) return gemm_split_reduce_launch(part, p.Y, p.R, p.M * p.N, splits, stream, err);
     return true;
 }
@@ -824,8 +842,9 @@ bool gemm_bf16_partials(uint64_t x, uint64_t w, uint32_t m, uint32_t n, uint32_t
     if (!shape_ok(m, n, k, err)) return false;
     GemmParams p = base_params(x, w, m, n, k);
     p.wscale = reinterpret_cast<const float*>(wscale);
-    *splits = splits_on(stream, p);
-    return launch_weights<kEpiPlain>(p, *splits, true, part, stream, err);
+    const StreamPlan plan = plan_on(stream, p);
+    *splits = plan.splits;
+    return launch_weights<kEpiPlain>(p, plan, true, part, stream, err);
 }
 
 bool gemm_bf16_add_rmsnorm(uint64_t x, uint64_t w, uint64_t hidden, uint64_t norm_w, uint64_t y,
@@ -875,9 +894,10 @@ bool gemm_bf16_swiglu(uint64_t x, uint64_t w_gate_up, uint64_t act, uint32_t m, 
     GemmParams p = base_params(x, w_gate_up, m, 2 * inter, k);
     p.Y = reinterpret_cast<uint16_t*>(act);
     p.wscale = reinterpret_cast<const float*>(wscale);
-    const int splits = splits_on(stream, p);
+    const StreamPlan plan = plan_on(stream, p);
+    const int splits = plan.splits;
     float* part = nullptr;
-    if (!launch_weights<kEpiSwiglu>(p, splits, false, &part, stream, err)) return false;
+    if (!launch_weights<kEpiSwiglu>(p, plan, false, &part, stream, err)) return false;
     if (splits > 1) {
         const int n = p.M * static_cast<int>(inter);
         hipLaunchKernelGGL(gemm_split_swiglu, dim3((n / 4 + 255) / 256), dim3(256), 0,
@@ -923,9 +943,10 @@ bool gemm_bf16_rope_append(uint64_t x, uint64_t w_qkv, uint32_t m, uint32_t k,
     p.mbps = static_cast<int>(a.mbps);
     p.row_bytes = static_cast<int>(a.row_bytes);
     p.wscale = reinterpret_cast<const float*>(wscale);
-    const int splits = splits_on(a.stream, p);
+    const StreamPlan plan = plan_on(a.stream, p);
+    const int splits = plan.splits;
     float* part = nullptr;
-    if (!launch_weights<kEpiRope>(p, splits, false, &part, a.stream, err)) return false;
+    if (!launch_weights<kEpiRope>(p, plan, false, &part, a.stream, err)) return false;
     if (splits > 1) return rope_append_from_partials(a, part, splits, err);
     return true;
 }

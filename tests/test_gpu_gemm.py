@@ -634,3 +634,35 @@ def test_wide_kernel_special_values(gpu_lib, tunables, m, n, k):
           flush=True)
     assert bool(y0.view(torch.bfloat16).isnan().any()) and bool((y0 == 0x7fc0).any())
     assert torch.equal(y0, y1) and torch.equal(a0, a1)
+
+
+@pytest.mark.parametrize("m,n,k,fp8,splits", [
+    (1, 4096, 11008, False, 4),      # 43 chunks, 64 tiles: uneven splits in one round
+    (1, 11008, 11008, False, 1),     # 172 tiles: a second round would eat the gain
+    (17, 9024, 768, True, 1),        # 3 chunks: the split sum costs more than it gains
+    (32, 4416, 768, False, 1),
+    (65, 384, 5120, True, 10),       # 14 uneven splits of 3 chunks against 10 of 4
+    (65, 2048, 14336, False, 8),     # 8 splits meet the target: not the 7 below it
+    (1, 5120, 3072, False, 3),       # 4 would go past it
+    (2, 2048, 2048, True, 4)])       # 512-element chunks would leave 2
+def test_split_rules(gpu_lib, m, n, k, fp8, splits):
+    """Both sides of the rules that choose K splits, and a product with each
+    against float64."""
+    import torch
+    assert gpu_lib.gemm_plan(m, n, k, fp8_weights=fp8)["splits"] == splits
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + n + k)
+    x = torch.randn((m, k), generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn((n, k), generator=g, device="cuda") * 0.02
+    w = w.to(torch.float8_e4m3fn) if fp8 else w.to(torch.bfloat16)
+    one = torch.ones(n, device="cuda")
+    y = torch.full((m, n), float("nan"), device="cuda", dtype=torch.bfloat16)
+    s = torch.cuda.current_stream().cuda_stream
+    if fp8:
+        gpu_lib.gemm_fp8w_bf16(x.data_ptr(), w.data_ptr(), one.data_ptr(), y.data_ptr(), m, n, k, s)
+    else:
+        gpu_lib.gemm_bf16(x.data_ptr(), w.data_ptr(), y.data_ptr(), m, n, k, s)
+    ref = x.double() @ w.double().t().contiguous()
+    mag = x.double().abs() @ w.double().abs().t().contiguous()
+    tol = k * 2.0 ** -24 * mag + 2.0 ** -8 * ref.abs() * 1.01
+    assert float(((y.double() - ref).abs() / tol).max()) <= 1.0
