@@ -352,10 +352,11 @@ int kcmm_gemm_bf16_add_on_stream(uint64_t x_ptr, uint64_t w_ptr, uint64_t residu
 /** The O projection with its residual add and the post-attention RMSNorm
  *  (ref llama_transformer.rs:356-362: o GEMM, add.cu, rms_norm.cu):
  *  hidden = bf16(hidden + bf16(x * w^T)) in place ([m][n]), then normed =
- *  rmsnorm(hidden) with weight norm_w.  Bit-identical to
- *  kcmm_gemm_bf16_add_on_stream followed by kcmm_rmsnorm_bf16_on_stream; the
- *  split-K partial sums are finished inside the RMSNorm kernel.  n % 64 ==
- *  0, k % 256 == 0. */
+ *  rmsnorm(hidden) with weight norm_w.  Up to 128 tokens bit-identical to
+ *  kcmm_gemm_bf16_add_on_stream followed by kcmm_rmsnorm_bf16_on_stream
+ *  (above, some shapes run on another kernel, whose sums are in another
+ *  order); the split-K partial sums are finished inside the RMSNorm kernel.
+ *  n % 64 == 0, k % 256 == 0. */
 int kcmm_gemm_bf16_add_rmsnorm_on_stream(uint64_t x_ptr, uint64_t w_ptr, uint64_t hidden_ptr,
                                          uint64_t norm_w_ptr, uint64_t normed_ptr, uint32_t m,
                                          uint32_t n, uint32_t k, float eps,

@@ -169,6 +169,7 @@ bool gemm_tiled(uint64_t x, uint64_t w, uint64_t wscale, uint64_t y, uint32_t m,
 // Its K splits and tiling (0..10 of the tiled kernel; 100 + token tile
 // height / 64 on the wide kernel).
 void gemm_tiled_plan(uint32_t m, uint32_t n, uint32_t k, bool fp8_weights, int* splits, int* tile);
+double gemm_tiled_us(uint32_t m, uint32_t n, uint32_t k);   // its modelled time, bf16 weights
 
 // The product for prompt-sized m on 256-row tiles of 8 waves
 // (kernels/gemm_wide.hip), bf16 weights.  swiglu: w = [gate; up] with n rows
@@ -254,9 +255,9 @@ bool gemm_bf16_partials(uint64_t x, uint64_t w, uint32_t m, uint32_t n, uint32_t
                         uint64_t stream, float** part, int* splits, std::string* err,
                         uint64_t wscale = 0);
 
-// hidden = bf16(hidden + bf16(X W^T)) in place, y = rmsnorm(hidden): the bits
-// of gemm_bf16 with the residual followed by rmsnorm_bf16, the split partials
-// (if the plan has any) summed in the RMSNorm kernel.
+// hidden = bf16(hidden + bf16(X W^T)) in place, y = rmsnorm(hidden): up to 128
+// tokens the bits of gemm_bf16 with the residual followed by rmsnorm_bf16, the
+// split partials (if the plan has any) summed in the RMSNorm kernel.
 bool gemm_bf16_add_rmsnorm(uint64_t x, uint64_t w, uint64_t hidden, uint64_t norm_w, uint64_t y,
                            uint32_t m, uint32_t n, uint32_t k, float eps, uint64_t stream,
                            std::string* err);

@@ -22,6 +22,7 @@
 // members of a pair (RoPE i and i + D/2; gate j and up I + j) land in the
 // same wave, 32 lanes apart.
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <type_traits>
 
@@ -517,7 +518,9 @@ __global__ __launch_bounds__(256) void gemm_split_swiglu(const float* __restrict
 // K splits: the smallest divisor of K/kch giving at least `target` workgroups
 // (KCMM_GEMM_WGS, default 256: fewer, longer splits measured faster than
 // 512-1024 at the Llama-3-8B decode shapes) with each split at least two
-// chunks long; at most 16.  Where that divisor goes past the target and the
+// chunks long; at most 16.  Up to 128 tokens (not `many`, whose workgroups of 4
+// waves fit a CU twice: I 1984, K 14848, 296 tokens of SwiGLU at 4 -> 2 splits 93
+// -> 132): where that divisor goes past the target and the
 // one before it gives 7/8 of it, the one before: one round with a few idle
 // CUs beats a second round (one token, bf16, more -> fewer splits: 5120 x 3072
 // at 4 -> 3 10.9 -> 9.7 us, 7680 x 2560 at 5 -> 2 13.9 -> 10.6, 5120 x 13824 at
@@ -532,7 +535,7 @@ __global__ __launch_bounds__(256) void gemm_split_swiglu(const float* __restrict
 // 1024 x 2816 at 1 -> 6 22.3 -> 7.6, 3584 x 18944 at 2 -> 4 38.7 -> 25.2; 64 tokens
 // 99 -> 25.3, 27.6 -> 9.0, 58 -> 35; not 11008 x 11008, 55.5 unsplit and 61 at 2,
 // nor 9024 x 768 with fp8 weights, 5.4 and 7.1).
-int choose_splits(int N, int K, int kch, int mgroups, int* equal) {
+int choose_splits(int N, int K, int kch, int mgroups, bool many, int* equal) {
     const int chunks = K / kch;
     const int forced = dev::tunable_or(dev::Tun::kGemmSplits, 0);
     if (forced >= 1 && forced <= 16 && chunks % forced == 0) return *equal = forced;
@@ -546,9 +549,9 @@ int choose_splits(int N, int K, int kch, int mgroups, int* equal) {
         best = s;
         if (tiles * s >= target) break;
     }
-    if (before > 1 && tiles * best > target && 8 * tiles * before >= 7 * target) best = before;
+    if (!many && before > 1 && tiles * best > target && 8 * tiles * before >= 7 * target) best = before;
     *equal = best;
-    if (4 * tiles * best >= 3 * target) return best;
+    if (many || 4 * tiles * best >= 3 * target) return best;
     auto cost = [&](int s) { return (chunks + s - 1) / s + (s > 1 ? std::max(1, 512 / kch) : 0); };
     int uneven = best;
     for (int s = best + 1; s <= 16 && tiles * s <= target; ++s) {
@@ -575,11 +578,11 @@ struct StreamPlan {
 StreamPlan stream_plan(int M, int N, int K, bool wf8) {
     StreamPlan p{M <= 64 ? 256 : M <= 128 || wf8 ? 128 : 64, 1, 1};
     const int rows = M <= 16 ? 16 : M <= 32 ? 32 : M <= 64 ? 64 : M <= 128 ? 128 : 256;
-    p.splits = choose_splits(N, K, p.kch, (M + rows - 1) / rows, &p.equal);
+    p.splits = choose_splits(N, K, p.kch, (M + rows - 1) / rows, M > 128, &p.equal);
     if (M <= 16 && wf8 && K % 512 == 0 && K >= 4096 &&
         (p.splits == 1 || N / 64 * p.splits <= 256)) {
         StreamPlan q{512, 1, 1};
-        q.splits = choose_splits(N, K, 512, 1, &q.equal);
+        q.splits = choose_splits(N, K, 512, 1, false, &q.equal);
         if (q.splits == p.splits) return q;
     }
     return p;
@@ -711,6 +714,49 @@ bool shape_ok(uint32_t m, uint32_t n, uint32_t k, std::string* err) {
         return false;
     }
     return true;
+}
+
+// Modelled time in us of this kernel above 128 tokens: a launch or two, the
+// chunks of the longest split in every round of workgroups, the partials, the
+// weights.  Fitted to timings of 756 SwiGLU products (I 32 .. 2816, K 256 ..
+// 14336, M 129 .. 4096): within 18% for nine in ten.
+double stream_us(const GemmParams& p, const StreamPlan& s) {
+    const double part = s.splits > 1 ? 4.0 * s.splits * p.M * p.N : 0.0;
+    const double wgs = p.N / 64.0 * ((p.M + 255) / 256) * s.splits;
+    return 7.1 + std::max(1.0, wgs / 256) * ((p.K / s.kch + s.splits - 1) / s.splits) * 0.92 +
+           0.2 * std::ceil(wgs / 256) + 0.46e-6 * part + 0.019e-6 * 2.0 * p.N * p.K;
+}
+
+// Whether a SwiGLU product above 128 tokens runs the wide kernel: when its
+// modelled time is a tenth below this kernel's (a quarter where the weights do
+// not fit the Infinity Cache: both models hold for weights in it).  Over the
+// 756 products the choice is the faster kernel, or within 9% of it.  Wide /
+// stream, us: I 32, K 14336, M 129 133 / 23; I 512, K 4096, M 512 43 / 20; I 1024,
+// K 4096, M 1024 46 / 52; I 6272, K 12800, M 131 160 / 137; I 14336, K 4096, M
+// 2048 357 / 690.  A capture without scratch for the partials takes the wide
+// kernel.
+bool swiglu_wide(uint64_t stream, const GemmParams& p, uint32_t inter) {
+    if (dev::gemm_wide_forced() != 0) return true;
+    const StreamPlan s = stream_plan(p.M, p.N, p.K, false);
+    const double margin = 2.0 * p.N * p.K > 256e6 ? 0.75 : 0.9;
+    return dev::gemm_wide_plan(p.M, inter, p.K, true).us < margin * stream_us(p, s) ||
+           (s.splits > 1 &&
+            !dev::stream_scratch(stream, 1, static_cast<size_t>(s.splits) * p.M * p.N * sizeof(float), true));
+}
+
+// Whether a product above 128 tokens whose partials the RMSNorm kernel sums
+// runs on this kernel: a few 64 x 64 tiles of short rows (161 x 128 x 768 9.0 us,
+// 10.2 on the many-token kernels and RMSNorm after them), or a modelled time a
+// tenth below the many-token kernels' (923 x 704 x 6400 38 / 49, 386 x 2176 x 4864
+// 39 / 41; most shapes are the other way, 2117 x 512 x 512 20 / 11).  A capture
+// without scratch for the partials takes the many-token kernels.
+bool rmsnorm_partials(uint64_t stream, const GemmParams& p) {
+    if (p.M <= 128 || dev::tunable_or(dev::Tun::kGemmTiled, 1) == 0) return true;
+    if (dev::tunable_or(dev::Tun::kGemmTile, -1) >= 0) return false;
+    const StreamPlan s = stream_plan(p.M, p.N, p.K, false);
+    const bool few = (p.M + 63) / 64 * (p.N / 64) <= 20 && p.K <= 768;
+    return (few || stream_us(p, s) < 0.9 * dev::gemm_tiled_us(p.M, p.N, p.K)) &&
+           dev::stream_scratch(stream, 1, static_cast<size_t>(s.splits) * p.M * p.N * sizeof(float), true);
 }
 
 // Decode-sized products over a long weight matrix (an lm_head) run the wide
@@ -854,11 +900,11 @@ bool gemm_bf16_add_rmsnorm(uint64_t x, uint64_t w, uint64_t hidden, uint64_t nor
     int splits = 1;
     // x may lie in hidden: its rows are then read before any is written
     const bool apart = x + 2ull * m * k <= hidden || hidden + 2ull * m * n <= x;
-    if (m > 128 && apart && dev::tunable_or(dev::Tun::kGemmTiled, 1) != 0) {
+    if (!shape_ok(m, n, k, err)) return false;
+    if (apart && !rmsnorm_partials(stream, base_params(x, w, m, n, k))) {
         // many tokens: as gemm_bf16 with the residual (an unsplit product
         // adds it in its own store), its split sum left to the RMSNorm kernel
-        if (!shape_ok(m, n, k, err) ||
-            !gemm_tiled(x, w, 0, hidden, m, n, k, stream, hidden, err, &part, &splits))
+        if (!gemm_tiled(x, w, 0, hidden, m, n, k, stream, hidden, err, &part, &splits))
             return false;
         if (part == nullptr) return rmsnorm_bf16(hidden, norm_w, y, m, n, eps, stream, err);
     } else if (!gemm_bf16_partials(x, w, m, n, k, stream, &part, &splits, err)) {
@@ -874,11 +920,13 @@ bool gemm_bf16_swiglu(uint64_t x, uint64_t w_gate_up, uint64_t act, uint32_t m, 
         return false;
     }
     if (!shape_ok(m, 2 * inter, k, err)) return false;
+    GemmParams p = base_params(x, w_gate_up, m, 2 * inter, k);
+    p.wscale = reinterpret_cast<const float*>(wscale);
     // many tokens, bf16 weights: the wide kernel, whose weight tiles hold gate
-    // and up rows (KCMM_GEMM_TILED=0 keeps the weight-stream kernel).  Faster
-    // at every measured size: 1.1-1.5x at M = 129..256, 2x from M = 320 on
-    // (gate/up of a 2048-token chunk at the Llama-3-8B shape 719 -> 370 us).
-    if (wscale == 0 && m > 128 && dev::tunable_or(dev::Tun::kGemmTiled, 1) != 0) {
+    // and up rows, or the weight-stream kernel, which can split K, for few
+    // tiles of long rows (KCMM_GEMM_TILED=0 keeps the weight-stream kernel)
+    if (wscale == 0 && m > 128 && dev::tunable_or(dev::Tun::kGemmTiled, 1) != 0 &&
+        swiglu_wide(stream, p, inter)) {
         GemmWideArgs a{};
         a.x = x;
         a.w = w_gate_up;
@@ -891,9 +939,7 @@ bool gemm_bf16_swiglu(uint64_t x, uint64_t w_gate_up, uint64_t act, uint32_t m, 
         a.stream = stream;
         return gemm_wide(a, err);
     }
-    GemmParams p = base_params(x, w_gate_up, m, 2 * inter, k);
     p.Y = reinterpret_cast<uint16_t*>(act);
-    p.wscale = reinterpret_cast<const float*>(wscale);
     const StreamPlan plan = plan_on(stream, p);
     const int splits = plan.splits;
     float* part = nullptr;

@@ -411,6 +411,15 @@ void gemm_tiled_plan(uint32_t m, uint32_t n, uint32_t k, bool fp8_weights, int* 
     *tile = wide ? 100 + wp.fb0 : c.id;
 }
 
+double gemm_tiled_us(uint32_t m, uint32_t n, uint32_t k) {
+    const TiledConfig c = choose(static_cast<int>(m), static_cast<int>(n), static_cast<int>(k));
+    GemmWidePlan wp;
+    if (use_wide(c, m, n, k, &wp)) return wp.us;
+    // (64-row tiles take 1.35 times their model where N % 128 != 0 and where
+    // they fill one to two rounds, which the choices above do not depend on)
+    return tiled_us(c, m, n, k) * (c.bn == 64 ? 1.35 : 1.0);
+}
+
 bool gemm_tiled(uint64_t x, uint64_t w, uint64_t wscale, uint64_t y, uint32_t m, uint32_t n,
                 uint32_t k, uint64_t stream, uint64_t residual, std::string* err, float** part,
                 int* splits) {

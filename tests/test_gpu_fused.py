@@ -178,3 +178,39 @@ def test_add_rmsnorm_of_the_hidden_rows_themselves(gpu_lib, tunables, m):
         seen.append((h, y))
     assert np.array_equal(_bits(seen[0][0]), _bits(seen[1][0]))
     assert np.array_equal(_bits(seen[0][1]), _bits(seen[1][1]))
+
+
+@pytest.mark.parametrize("m,n,k,stream", [(161, 128, 768, True), (923, 704, 6400, True),
+                                          (386, 2176, 4864, True), (556, 1024, 768, False)])
+def test_add_rmsnorm_kernel_choice(gpu_lib, tunables, m, n, k, stream):
+    """Above 128 tokens the product runs on the weight-stream kernel where
+    that is the faster one (then with the bits of KCMM_GEMM_TILED=0) and on
+    the many-token kernels elsewhere (the bits of the unfused calls)."""
+    import torch
+    x = _randn_bf16(torch, (m, k), 1.0, 31)
+    w = _randn_bf16(torch, (n, k), 0.02, 32)
+    h0 = _randn_bf16(torch, (m, n), 1.0, 33)
+    nw = (1.0 + 0.1 * _randn_bf16(torch, (n,), 1.0, 34).float()).to(torch.bfloat16)
+    sp = torch.cuda.current_stream().cuda_stream
+
+    def fused():
+        h, y = h0.clone(), torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+        gpu_lib.gemm_bf16_add_rmsnorm(x.data_ptr(), w.data_ptr(), h.data_ptr(), nw.data_ptr(),
+                                      y.data_ptr(), m, n, k, 1e-5, sp)
+        torch.cuda.synchronize()
+        return _bits(h), _bits(y)
+
+    def unfused():
+        h, y = h0.clone(), torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+        gpu_lib.gemm_bf16_add(x.data_ptr(), w.data_ptr(), h.data_ptr(), h.data_ptr(), m, n, k, sp)
+        gpu_lib.rmsnorm_bf16(h.data_ptr(), nw.data_ptr(), y.data_ptr(), m, n, 1e-5, sp)
+        torch.cuda.synchronize()
+        return _bits(h), _bits(y)
+
+    got = fused()
+    if stream:
+        tunables.setenv("KCMM_GEMM_TILED", "0")
+    want = unfused()
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+    ref = O.decode(O.BF16, _bits(h0)).astype(np.float64) + O.gemm_bf16_f64(_bits(x), _bits(w))
+    assert np.abs(O.decode(O.BF16, got[0]) - ref).max() <= 1e-2 * np.abs(ref).max()

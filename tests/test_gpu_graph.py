@@ -13,7 +13,9 @@ Cases: embedding + a three-layer kcmm_decode_layers_on_stream call + logits
 (bf16 and fp8-e4m3 pools; the fp8 page writer's zero-restored counters are
 replayed too), standalone paged decode attention (bf16, fp8), and a
 split-K projection with its reduction kernel."""
+import concurrent.futures
 import ctypes as C
+import functools
 
 import numpy as np
 import pytest
@@ -143,6 +145,16 @@ def test_split_gemm_graph_replays(gpu_lib):
     _check_replays(torch, run, lambda: [y])
 
 
+def in_new_thread(test):
+    """Runs a test in a thread of its own: workspaces belong to (stream, host
+    thread), so every stream is a cold one there, whichever tests ran before."""
+    @functools.wraps(test)
+    def run(*args, **kw):
+        with concurrent.futures.ThreadPoolExecutor(1) as ex:
+            return ex.submit(test, *args, **kw).result()
+    return run
+
+
 class _KernelNode(C.Structure):   # hipKernelNodeParams
     _fields_ = [("block", C.c_uint32 * 3), ("extra", C.c_void_p), ("func", C.c_void_p),
                 ("grid", C.c_uint32 * 3), ("params", C.c_void_p), ("shared", C.c_uint32)]
@@ -234,6 +246,7 @@ def _scratch_free_work(torch, lib, what):
 
 
 @pytest.mark.parametrize("what", ["prefill", "uneven", "uneven_fp8", "wide"])
+@in_new_thread
 def test_captures_hold_no_optional_scratch(gpu_lib, what):
     """Calls that can run without scratch do so under every capture, on a warm
     stream too: one kernel with the whole key range or K in each workgroup
@@ -284,6 +297,7 @@ def test_captures_hold_no_optional_scratch(gpu_lib, what):
     (777, 6144, 4096, 0, 1),     # only the wide kernel splits it
     (300, 4096, 14336, 4, 2),    # the slot holds the tiled kernel's 4 splits, not the wide one's 8
     (300, 4096, 14336, 3, 1)])   # nor those
+@in_new_thread
 def test_wide_splits_under_capture(gpu_lib, tunables, m, n, k, slot, kernels):
     """A product whose split partials do not fit the stream's workspace is
     captured with fewer splits, or none, instead of allocating in the capture.
@@ -416,3 +430,49 @@ def test_first_call_beside_another_threads_capture(gpu_lib, what):
         assert float(d) <= 1e-2                           # (maybe in another order of the sums)
     finally:
         close()
+
+
+@pytest.mark.parametrize("m,inter,k,wide", [(200, 64, 14336, False), (300, 512, 4096, False),
+                                            (129, 2816, 8192, False), (777, 2816, 1024, True),
+                                            (4096, 1024, 4096, True), (150, 14336, 4096, True)])
+@in_new_thread
+def test_swiglu_kernel_choice(gpu_lib, tunables, m, inter, k, wide):
+    """Gate/up products above 128 tokens: few tiles of long rows take the
+    weight-stream kernel with K splits (two kernels on a warm stream, the wide
+    one under a capture without scratch), others the wide kernel; both against
+    float64 (bound: the bf16 roundings of gate, up, silu and the product, and
+    fp32 sums of k terms, through silu's slope of at most 1.1)."""
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + inter)
+    x = torch.randn((m, k), generator=g, device="cuda").to(torch.bfloat16)
+    w = (torch.randn((2 * inter, k), generator=g, device="cuda") / k ** 0.5).to(torch.bfloat16)
+    act = torch.full((m, inter), float("nan"), device="cuda", dtype=torch.bfloat16)
+
+    def run(s):
+        gpu_lib.gemm_bf16_swiglu(x.data_ptr(), w.data_ptr(), act.data_ptr(), m, inter, k, s)
+
+    assert len(_captured_kernels(run)) == 1
+    assert len(_captured_kernels(run, warm=run)) == (1 if wide else 2)
+    gu = x.double() @ w.double().t().contiguous()
+    mag = x.double().abs() @ w.double().abs().t().contiguous() * (k * 2.0 ** -24)
+    gate, up = gu[:, :inter], gu[:, inter:]
+    silu = torch.nn.functional.silu(gate)
+    dg, du = (2.0 ** -8 * v.abs() + mag[:, i * inter:(i + 1) * inter] for i, v in enumerate((gate, up)))
+    bound = ((1.1 * dg + 2.0 ** -8 * silu.abs()) * (up.abs() + du) + silu.abs() * du +
+             2.0 ** -8 * (silu * up).abs()) * 1.05 + 1e-30
+    for graph in (False, True):
+        act.fill_(float("nan"))
+        if graph:
+            st = torch.cuda.Stream()
+            cg = torch.cuda.CUDAGraph()
+            torch.cuda.synchronize()
+            with torch.cuda.graph(cg, stream=st):
+                run(st.cuda_stream)
+            cg.replay()
+        else:
+            run(torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        worst = float(((act.double() - silu * up).abs() / bound).max())
+        print(f"swiglu {m}x{inter}x{k} graph={graph} worst {worst:.3f} of the bound", flush=True)
+        assert worst <= 1.0
