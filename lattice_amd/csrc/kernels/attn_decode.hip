@@ -752,8 +752,9 @@ void attn_decode_stream(AttnParams p, const int32_t* __restrict__ bt,
     }
 }
 
-// Log-sum-exp merge, one 4-wave workgroup per (b, kv head g) that spans several
-// slices of the streaming kernel (and per 1024 outputs): part k of the np
+// Log-sum-exp merge, one workgroup of 4 or 16 waves (launch_merge) per (b, kv
+// head g) that spans several slices of the streaming kernel (and per NT or more
+// outputs; NT / S quads of them): part k of the np
 // parts from slice wa on sits at the (b, g) unit k for k < kSegPieces and in
 // slot 0 of the wave for g of slice wa+k after that (wave rows (wa + k) * HW +
 // g % HW).  Threads split the outputs four at a time and the parts S ways (the

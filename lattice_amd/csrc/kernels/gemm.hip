@@ -102,6 +102,7 @@ struct GemmParams {
     float* part;         // non-null: write fp32 partials [split][M][N], no epilogue
     const float* wscale; // fp8 weights: fp32 scale per weight row [N] (row n of W times wscale[n])
     int M, N, K, klen;
+    int klast;           // length of the last K split (klen, or shorter)
     // rope_append
     uint16_t* q_out;     // [M][Hq][D]
     uint8_t* k_base;
@@ -284,7 +285,7 @@ void gemm_bf16_stream(GemmParams p) {
     const int K = p.K;
     const int m_base = blockIdx.z * MROWS;
     const int kbeg = blockIdx.y * p.klen;
-    const int nchunks = min(p.klen, K - kbeg) / KCH;   // the last split may be shorter
+    const int nchunks = (blockIdx.y + 1 == gridDim.y ? p.klast : p.klen) / KCH;
     const uint32_t rowb = static_cast<uint32_t>(K) * (WF8 ? 1 : 2);   // weight row bytes
 
     // the first CW waves stream weight rows; the rest (CW < NW) only stage
@@ -630,6 +631,7 @@ bool launch_stream(GemmParams p, const StreamPlan& plan, bool want_partials, flo
     return by_m(p.M, plan, [&](auto mb, auto kch) {
         constexpr int MB = decltype(mb)::value, KCH = decltype(kch)::value;
         p.klen = (p.K / KCH + splits - 1) / splits * KCH;
+        p.klast = p.K - (splits - 1) * p.klen;
         if constexpr (!WF8 && KCH > 256) {
             *err = "512-element chunks are for fp8 weights";
             return false;
