@@ -29,7 +29,7 @@
 // Measured (MI355X): 8192^3 776 us = 1.42 PFLOP/s (2.18 without the loads,
 // 1.35 in four phases of 16 MFMAs, 1.36 with the loads issued between the
 // MFMAs; the 128 x 256 tile 1.06); gate/up + SwiGLU of 2048 tokens at the
-// Llama-3-8B shape 719 us on the weight-stream kernel, 356 here (1.35
+// Llama-3-8B shape 690 us on the weight-stream kernel, 357 here (1.35
 // PFLOP/s); down + residual of 777 tokens 130 -> 100 us.
 #include <algorithm>
 #include <string>
@@ -409,7 +409,7 @@ int gemm_wide_forced() {
 // tile only as high as it needs), K splits of at least 4 chunks for plain
 // products, and -- when whole rounds of tiles leave a partly filled last round
 // -- lower token tiles for the weight tiles of that round (gate/up of 2048
-// tokens, 3.5 rounds of 256-token tiles: 369 -> 356 us with the last half
+// tokens, 3.5 rounds of 256-token tiles: 369 -> 357 us with the last half
 // round on 128-token tiles).  A split counts 5% more than its model, whose
 // error is larger there.  KCMM_GEMM_SPLITS forces the split (0 splits in the
 // result: it cannot be had); KCMM_GEMM_TILE = 100 + fb0 the token tiles'
