@@ -910,11 +910,12 @@ void launch_merge_nt(AttnParams& p, hipStream_t s) {
         hipLaunchKernelGGL((attn_decode_merge<DT, D, NT / 256, NT>), grid(256), block, 0, s, p, p.seg_info);
 }
 
-// Few (b, g) pairs have many parts each: 16-wave workgroups while one per CU
-// holds them all, else 4-wave ones.
+// Few (b, g) pairs have many parts each: 16-wave workgroups up to 64 pairs
+// (more waves than parts beyond: 19 sequences of 8 heads of 64 27.2 us with 16,
+// 26.0 with 4), then 4-wave ones.
 template <int DT, int D>
 void launch_merge(AttnParams& p, hipStream_t s) {
-    if (p.batch * p.kv_heads <= 256) launch_merge_nt<DT, D, 1024>(p, s);
+    if (p.batch * p.kv_heads <= 64) launch_merge_nt<DT, D, 1024>(p, s);
     else launch_merge_nt<DT, D, 256>(p, s);
 }
 
