@@ -1152,7 +1152,11 @@ int stream_waves(int dtype) {
 //    (64 sequences of 512 .. 4096 tokens: kernel 103 us against 105.5), but the
 //    call slower where it follows a layer's other kernels (116.5 against 111),
 //    and the 32-layer step that it is part of 7.325 ms against 7.235 (Llama-3-8B
-//    shape, three alternating runs each, spread 0.01).
+//    shape, three alternating runs each, spread 0.01).  A few long sequences
+//    would gain in the layer too (two of 24000 .. 50000 tokens 166.7 -> 161.6 us
+//    a layer, four of 20000 .. 30000 185.2 -> 178.5), but the host cannot tell
+//    them from short ones in wide tables, which lose (one of 1456 tokens 11.5
+//    us, 14.2 with four).
 //  * fp8 pages: 8 (a row of 1 KiB read together) where the tables have room for
 //    more than 8192 (kv head, tile) entries, else 1 -- 8-wave workgroups are then
 //    too few, whatever the lengths are.  Call times with 1 / 8, 32/8 heads of
